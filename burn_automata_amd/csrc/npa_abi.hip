@@ -397,9 +397,9 @@ npa_status npa_context_set_host_io(npa_context* ctx, int host_io) {
 }
 
 namespace {
-// Width of the feature-major rows a step's workspace holds: none when the fused second pass + MLP
+// Width of the feature rows a step's workspace holds: none when the fused second pass + MLP
 // kernel runs the step (its feature rows never leave LDS).
-uint32_t feature_rows_for(const npa::StepParams& p) { return npa::fused_update_applies(p) ? 0u : p.FP; }
+uint32_t feature_rows_for(const npa::StepParams& p) { return npa::fused_update_applies(p) ? 0u : p.F; }
 }  // namespace
 
 npa_status npa_context_set_mlp_engine(npa_context* ctx, int engine) {

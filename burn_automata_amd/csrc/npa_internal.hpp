@@ -271,7 +271,7 @@ __device__ __forceinline__ void hold_loaded(uint64_t i, float4 p, const float4 (
     for (int q = 0; q < NQ; ++q) o4[q] = v[q];
 }
 
-// Padded feature row used between the perception and MLP kernels:
+// Padded feature row of the fused update kernel:
 // [state SS][blur SS][grad SS*d][density-grad d?, position d?, zero padded to a multiple of 4].
 __host__ __device__ inline uint32_t padded_features(uint32_t SS, uint32_t d, uint32_t rest) {
     return 2 * SS + SS * d + (rest == 0 ? 0u : rest <= 4 ? 4u : 8u);
@@ -345,17 +345,20 @@ hipError_t launch_second_pass_2d(const StepParams& p, Workspace& ws, const StepI
                                  hipStream_t stream, Profiler* prof);
 hipError_t launch_second_pass_3d(const StepParams& p, Workspace& ws, const StepIO& io, int mode, int blocks,
                                  hipStream_t stream, Profiler* prof);
-// Padded weights, two layouts one after the other in one buffer: the MLP kernel's w1t [FP][HP]
-// (features at their padded positions), b1p [HP], w2t [H][OP] (transposed), b2p [OP]; then, at
-// float offset valu_weight_floats(p), the fused update kernel's (fused_weight_floats(p)).
-// Zeros everywhere else.
+// Padded weights in the layout of the kernel that serves the step: the fused update kernel's
+// (fused_weight_floats(p)) or the MLP kernel's (mlp_weight_floats(p)).
 size_t padded_weight_floats(const StepParams& p);
-size_t valu_weight_floats(const StepParams& p);
 size_t fused_weight_floats(const StepParams& p);
+size_t mlp_weight_floats(const StepParams& p);
 hipError_t launch_pad_weights(const StepParams& p, const float* w1, const float* b1, const float* w2,
                               const float* b2, float* wpad, hipStream_t stream);
 hipError_t launch_pad_weights_fused(const StepParams& p, const float* w1, const float* b1, const float* w2,
                                     const float* b2, float* wf, hipStream_t stream);
+hipError_t launch_mlp_weights(const StepParams& p, const float* w1, const float* b1, const float* w2,
+                              const float* b2, float* wp, hipStream_t stream);
+// The update MLP + masked Euler step over the compact feature rows in ws.features (npa_mlp.hip).
+hipError_t launch_mlp_euler(const StepParams& p, Workspace& ws, const StepIO& io, hipStream_t stream,
+                            Profiler* prof);
 // The fused second pass + update MLP + Euler step (npa_update.hip) for 16-wide sorted rows,
 // H <= 128, either MLP engine; wfused = the fused layout of the padded weights.
 bool fused_update_applies(const StepParams& p);

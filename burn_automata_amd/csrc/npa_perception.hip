@@ -903,7 +903,7 @@ __device__ __forceinline__ uint64_t residue_mask(uint32_t q) {
 // list) use the target itself with zero weights; the self pair's gradient terms and those of
 // coincident particles are zero as well. Zero terms leave every sum unchanged: each sum starts
 // at +0.0 and so never holds -0.0.
-// MODE 0: padded feature rows, feature-major (features[k * T + s]) for the MLP kernel.
+// MODE 0: feature rows [compact row][F] for the MLP kernel.
 // MODE 1: the perceive_with_options outputs in original particle order.
 // FL >= 0 fixes the option flags at compile time (bit 0 state gradient, bit 1 density gradient,
 // bit 2 moment correction); FL < 0 reads them from P.
@@ -1289,53 +1289,20 @@ __global__ __launch_bounds__(64) void k_perceive(StepParams P, const float4* __r
             pp[1] = p4.y;
             pp[2] = p4.z;
         }
-        if constexpr (MODE == 0) {
-            // padded layout [si SM][blur SM][grad SM*D][rest], feature-major; rest holds the
-            // density gradient and/or position (runtime count) followed by zeros.
-            const uint32_t T = P.T;
-            float* f = sfeatures + row;
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) f[(uint64_t)(c0 + c) * T] = si[c];
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) f[(uint64_t)(SM + c0 + c) * T] = blur[c];
-#pragma unroll
-            for (int k = 0; k < CPL * D; ++k) f[(uint64_t)(2 * SM + c0 * D + k) * T] = want_sg ? grad[k] : 0.0f;
-            if (q == 0) {
-                float rest[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) rest[k] = 0.0f;
-                int nr = 0;
-                if (want_dg) {
-#pragma unroll
-                    for (int a = 0; a < D; ++a) rest[a] = dg[a];
-                    nr = D;
-                }
-                if (P.position_features) {
-#pragma unroll
-                    for (int a = 0; a < D; ++a) {
-                        if (nr == D) rest[D + a] = pp[a];
-                        else rest[a] = pp[a];
-                    }
-                }
-                constexpr uint32_t base_rest = 2 * SM + SM * D;
-#pragma unroll
-                for (int r = 0; r < 8; ++r)
-                    if (base_rest + r < P.FP) f[(uint64_t)(base_rest + r) * T] = rest[r];
-            }
-        } else {
+        {
             const uint32_t S = P.S;
-            float* f = io.features + (uint64_t)i * P.F;
+            float* f = MODE == 0 ? sfeatures + (uint64_t)row * P.F : io.features + (uint64_t)i * P.F;
 #pragma unroll
             for (int c = 0; c < CPL; ++c)
                 if (c0 + c < S) {
                     f[c0 + c] = si[c];
                     f[S + c0 + c] = blur[c];
-                    if (io.blurred) io.blurred[(uint64_t)i * S + c0 + c] = blur[c];
+                    if (MODE == 1 && io.blurred) io.blurred[(uint64_t)i * S + c0 + c] = blur[c];
                     if (want_sg) {
 #pragma unroll
                         for (int a = 0; a < D; ++a) {
                             f[2 * S + (c0 + c) * D + a] = grad[c * D + a];
-                            if (io.state_gradient)
+                            if (MODE == 1 && io.state_gradient)
                                 io.state_gradient[((uint64_t)i * S + c0 + c) * D + a] = grad[c * D + a];
                         }
                     }
@@ -1346,7 +1313,7 @@ __global__ __launch_bounds__(64) void k_perceive(StepParams P, const float4* __r
 #pragma unroll
                     for (int a = 0; a < D; ++a) {
                         f[off + a] = dg[a];
-                        if (io.density_gradient) io.density_gradient[(uint64_t)i * D + a] = dg[a];
+                        if (MODE == 1 && io.density_gradient) io.density_gradient[(uint64_t)i * D + a] = dg[a];
                     }
                     off += D;
                 }
@@ -1360,340 +1327,6 @@ __global__ __launch_bounds__(64) void k_perceive(StepParams P, const float4* __r
 }
 
 #if NPA_PART_MAIN
-// Pads the model weights into the MLP kernel's layout, zeros everywhere else:
-//   w1t [FP][HP]  w1 transposed, features at their padded positions, HP = H rounded up to 128
-//   b1p [HP]
-//   w2t [H][OP]   w2 transposed, OP = D + SS rounded up to a multiple of 4
-//   b2p [OP]
-__global__ __launch_bounds__(256) void k_pad_weights(StepParams P, int D, const float* __restrict__ w1,
-                                                     const float* __restrict__ b1, const float* __restrict__ w2,
-                                                     const float* __restrict__ b2, float* __restrict__ wpad) {
-    const uint32_t S = P.S, SS = P.SS, F = P.F, H = P.H, FP = P.FP;
-    const uint32_t HP = (H + 127) / 128 * 128;
-    const uint32_t O = D + S, OP = (D + SS + 3) / 4 * 4;
-    const uint64_t n1 = (uint64_t)FP * HP, n2 = (uint64_t)H * OP;
-    const uint64_t total = n1 + HP + n2 + OP;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < total; k += (uint64_t)gridDim.x * blockDim.x) {
-        float v = 0.0f;
-        if (k < n1) {
-            const uint32_t q = (uint32_t)(k / HP), h = (uint32_t)(k - (uint64_t)q * HP);
-            // padded feature position q -> real feature index
-            int64_t fi = -1;
-            if (q < SS) fi = q < S ? (int64_t)q : -1;
-            else if (q < 2 * SS) fi = q - SS < S ? (int64_t)(S + q - SS) : -1;
-            else if (q < 2 * SS + SS * D) {  // gradient features exist only with the state gradient
-                const uint32_t g = q - 2 * SS;
-                fi = P.state_grad && g < S * D ? (int64_t)(2 * S + g) : -1;
-            } else {
-                const uint32_t r = q - (2 * SS + SS * D);
-                const uint32_t first = 2 * S + (P.state_grad ? S * D : 0);
-                fi = first + r < F ? (int64_t)(first + r) : -1;
-            }
-            if (fi >= 0 && h < H) v = w1[(uint64_t)h * F + fi];
-        } else if (k < n1 + HP) {
-            const uint32_t h = (uint32_t)(k - n1);
-            if (h < H) v = b1[h];
-        } else if (k < n1 + HP + n2) {
-            const uint64_t t = k - n1 - HP;
-            const uint32_t h = (uint32_t)(t / OP), o = (uint32_t)(t - (uint64_t)h * OP);
-            if (o < O) v = w2[(uint64_t)o * H + h];
-        } else {
-            const uint32_t o = (uint32_t)(k - n1 - HP - n2);
-            if (o < O) v = b2[o];
-        }
-        wpad[k] = v;
-    }
-}
-
-#endif  // NPA_PART_MAIN
-
-// Update MLP + motion scaling + 3D gates + masked Euler for 64 sorted slots per 4-wave block.
-// forward_update_from_features model.rs:900-940, forward_from_features_with_eps model.rs:867-898,
-// gates model.rs:806-837, euler_step step.rs:4-55.
-//   phase 1: lane = row; wave w computes hidden units [32w + 128p, 32w + 128p + 32) with the
-//            weights of feature k as wave-uniform scalar loads; each hidden sum starts from its
-//            bias and adds features k = 0..FM-1 in order (padded positions carry zero weights).
-//   phase 2: lane = row; wave w owns outputs [OPW*w, OPW*w + OPW); each output sum starts from its
-//            bias and adds hidden units h = 0..H-1 in order, reading them from LDS.
-//   phase 3: wave 0 applies motion scaling, gates, mask and the Euler step for its 64 rows.
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-// Phases 1 and 2 on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: A 16x4, B 4x16, D 16x16;
-// lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16]).
-// Wave w serves rows 16w..16w+15 of the block's 64. Each accumulator starts from its bias; the
-// matrix cores add the products in their own order, so the result differs from the reference's
-// sequential sum in the last bits.
-template <int FM, int OP>
-__device__ __forceinline__ void mlp_mfma(const StepParams& P, const float* __restrict__ sfeatures, uint32_t row0,
-                                         uint32_t nrows, uint32_t wave, uint32_t lane, const float* __restrict__ wpad,
-                                         float* hid, float* ul) {
-    const uint32_t H = P.H, T = P.T;
-    const uint32_t HP = (H + 127) / 128 * 128;
-    const float* w1t = wpad;
-    const float* b1p = w1t + (uint64_t)FM * HP;
-    const float* w2t = b1p + HP;
-    const float* b2p = w2t + (uint64_t)H * OP;
-    const uint32_t li = lane % 16, lk = lane / 16;
-    const uint32_t rl = 16 * wave + li;          // block-local row this lane feeds as A
-    const bool rvalid = row0 + rl < nrows;
-    // layer 1: hidden = relu(b1 + F W1^T), 16 rows x HP hidden per wave, 16 columns per tile
-    for (uint32_t hb = 0; hb < HP; hb += 128) {
-        v4f acc[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float bias = b1p[hb + 16 * t + li];
-            acc[t] = v4f{bias, bias, bias, bias};
-        }
-#pragma unroll 4
-        for (int k0 = 0; k0 < FM; k0 += 4) {
-            const uint32_t k = (uint32_t)k0 + lk;
-            const float a = rvalid ? sfeatures[(uint64_t)k * T + row0 + rl] : 0.0f;
-            const float* wk = w1t + (uint64_t)k * HP + hb + li;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, wk[16 * t], acc[t], 0, 0, 0);
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                hid[(hb + 16 * t + li) * 64 + 16 * wave + 4 * lk + r] = fmaxf(acc[t][r], 0.0f);
-    }
-    __syncthreads();
-    // layer 2: u = b2 + hidden W2^T, 16 rows x OP outputs per wave
-    constexpr int OT = (OP + 15) / 16;
-    v4f acc2[OT];
-#pragma unroll
-    for (int t = 0; t < OT; ++t) {
-        const uint32_t col = 16 * t + li;
-        const float bias = col < (uint32_t)OP ? b2p[col] : 0.0f;
-        acc2[t] = v4f{bias, bias, bias, bias};
-    }
-    for (uint32_t k0 = 0; k0 < HP; k0 += 4) {
-        const uint32_t k = k0 + lk;
-        const float a = hid[k * 64 + rl];
-#pragma unroll
-        for (int t = 0; t < OT; ++t) {
-            const uint32_t col = 16 * t + li;
-            const float b = (k < H && col < (uint32_t)OP) ? w2t[(uint64_t)k * OP + col] : 0.0f;
-            acc2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc2[t], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < OT; ++t) {
-        const uint32_t col = 16 * t + li;
-        if (col < (uint32_t)OP)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ul[(16 * wave + 4 * lk + r) * (OP + 1) + col] = acc2[t][r];
-    }
-}
-
-template <int D, int SM, int FM, int ENG>
-__global__ __launch_bounds__(256) void k_mlp_euler(StepParams P, const float* __restrict__ sfeatures,
-                                                   const float* __restrict__ sstate,
-                                                   const uint32_t* __restrict__ perm,
-                                                   const uint32_t* __restrict__ act_rows,
-                                                   const uint32_t* __restrict__ row_count,
-                                                   const float* __restrict__ wpad, StepIO io) {
-    constexpr int OP = (D + SM + 3) / 4 * 4;
-    constexpr int OPW = OP / 4;
-    extern __shared__ float lds[];
-    const uint32_t H = P.H, T = P.T;
-    const uint32_t HP = (H + 127) / 128 * 128;
-    // LDS: hid [HP][64] (for HP = 128 the four waves' w1t slices [4][FM][32] share its region
-    // before it is written); ul [64][OP + 1]; the VALU path's w2t copy [H][OP]
-    float* hid = lds;
-    const bool stage_w1 = HP == 128;  // one pass covers every hidden unit
-    float* ul = lds + (stage_w1 && 4 * FM * 32 > HP * 64 ? (size_t)4 * FM * 32 : (size_t)HP * 64);
-    const float* w1t = wpad;
-    const float* b1p = w1t + (uint64_t)FM * HP;
-    const float* w2t = b1p + HP;
-    const float* b2p = w2t + (uint64_t)H * OP;
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t row0 = blockIdx.x * 64;
-    const uint32_t nrows = *row_count;
-    if (row0 >= nrows) return;  // whole block
-    const uint32_t row = row0 + lane;
-    const bool valid = row < nrows;
-    const uint32_t s = act_rows[valid ? row : row0];  // sorted slot of this row's particle
-
-    if constexpr (ENG == 1) {
-        mlp_mfma<FM, OP>(P, sfeatures, row0, nrows, wave, lane, wpad, hid, ul);
-    } else {
-    float f[FM];
-#pragma unroll
-    for (int k = 0; k < FM; ++k) f[k] = valid ? sfeatures[(uint64_t)k * T + row] : 0.0f;
-
-    // phase 1: hidden units. With one pass (HP = 128) each wave stages its 32-unit slice of w1t in
-    // LDS (the region hid takes afterwards) and reads it back with broadcast loads, so no weight
-    // load waits on L2; wider layers read w1t from memory.
-    float* w2s = ul + 64 * (OP + 1);  // [H][OP]
-    if (stage_w1) {
-        float* w1s = lds + (size_t)wave * FM * 32;  // [FM][32] of this wave
-        const uint32_t hb = wave * 32;
-        for (uint32_t v = lane; v < (uint32_t)FM * 8; v += 64) {  // float4 v = (k, 4 units)
-            const uint32_t k = v / 8, j4 = v % 8;
-            reinterpret_cast<float4*>(w1s)[v] =
-                *reinterpret_cast<const float4*>(w1t + (uint64_t)k * HP + hb + 4 * j4);
-        }
-        __syncthreads();
-        float acc[32];
-#pragma unroll
-        for (int j = 0; j < 32; ++j) acc[j] = b1p[hb + j];
-#pragma unroll
-        for (int k = 0; k < FM; ++k) {
-            const float* wk = w1s + k * 32;
-            const float fk = f[k];
-#pragma unroll
-            for (int j = 0; j < 32; ++j) acc[j] += wk[j] * fk;
-        }
-        __syncthreads();  // every wave has read its slice before hid overwrites the region
-#pragma unroll
-        for (int j = 0; j < 32; ++j) hid[(hb + j) * 64 + lane] = fmaxf(acc[j], 0.0f);
-    } else {
-        for (uint32_t hb = wave * 32; hb < HP; hb += 128) {
-            float acc[32];
-#pragma unroll
-            for (int j = 0; j < 32; ++j) acc[j] = b1p[hb + j];
-#pragma unroll
-            for (int k = 0; k < FM; ++k) {
-                const float* wk = w1t + (uint64_t)k * HP + hb;
-                const float fk = f[k];
-#pragma unroll
-                for (int j = 0; j < 32; ++j) acc[j] += wk[j] * fk;
-            }
-#pragma unroll
-            for (int j = 0; j < 32; ++j) hid[(hb + j) * 64 + lane] = fmaxf(acc[j], 0.0f);
-        }
-    }
-    for (uint32_t v = threadIdx.x; v < H * OP / 4; v += blockDim.x)  // OP is a multiple of 4
-        reinterpret_cast<float4*>(w2s)[v] = reinterpret_cast<const float4*>(w2t)[v];
-    __syncthreads();
-
-    // phase 2: outputs
-    {
-        const uint32_t ob = wave * OPW;
-        float u[OPW];
-#pragma unroll
-        for (int o = 0; o < OPW; ++o) u[o] = b2p[ob + o];
-        for (uint32_t h = 0; h < H; ++h) {
-            const float hv = hid[h * 64 + lane];
-            const float* wr = w2s + h * OP + ob;
-#pragma unroll
-            for (int o = 0; o < OPW; ++o) u[o] += wr[o] * hv;
-        }
-#pragma unroll
-        for (int o = 0; o < OPW; ++o) ul[lane * (OP + 1) + ob + o] = u[o];
-    }
-    }  // ENG
-    __syncthreads();
-    if (wave != 0 || !valid) return;
-
-    // phase 3: motion scaling, gates, mask, Euler
-    const uint32_t S = P.S;
-    float u[D + SM];
-#pragma unroll
-    for (int o = 0; o < D + SM; ++o) u[o] = ul[lane * (OP + 1) + o];
-    const uint32_t b = s / P.N;
-    const uint32_t li = perm[s];
-    const uint32_t i = b * P.N + li;
-    float norm = 0.0f;
-#pragma unroll
-    for (int a = 0; a < D; ++a) norm += u[a] * u[a];
-    norm = sqrtf(norm);
-    float dx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int a = 0; a < D; ++a) dx[a] = P.alpha * u[a] * P.motion_eps / (1.0f + norm);
-    const float4 pos4 = io.pos[i];
-    const float porig[4] = {pos4.x, pos4.y, pos4.z, pos4.w};
-    float si[SM];
-    {
-        const float4* own = reinterpret_cast<const float4*>(sstate + (uint64_t)s * SM);
-#pragma unroll
-        for (int q = 0; q < SM / 4; ++q) {
-            const float4 v = own[q];
-            si[4 * q] = v.x;
-            si[4 * q + 1] = v.y;
-            si[4 * q + 2] = v.z;
-            si[4 * q + 3] = v.w;
-        }
-    }
-    float sg = 1.0f;
-    if (P.gates3d) {
-        const float liveness = si[3 < SM ? 3 : 0];
-        const float sd = si[7 < SM ? 7 : 0];
-        sg = clampf_((4.0f - liveness) * 2.0f, 0.0f, 1.0f);
-        float mg;
-        if (porig[3] >= 0.5f) {
-            mg = 0.0f;
-        } else {
-            const float dgate = clampf_((fabsf(sd) - 0.01f) / 0.02f, 0.0f, 1.0f);
-            mg = sg * dgate;
-        }
-#pragma unroll
-        for (int a = 0; a < D; ++a) dx[a] *= mg;
-    }
-    const float m = io.mask ? io.mask[i] : hash_mask(li, b, P.N, P.update_prob, P.step_index, P.base_seed);
-    float pn[4] = {porig[0], porig[1], porig[2], porig[3]};
-    constexpr int MEM = D == 3 ? 4 : 2;
-#pragma unroll
-    for (int a = 0; a < MEM; ++a) pn[a] += P.dt * dx[a] * m;
-    if (P.g.boundary == 0) {
-#pragma unroll
-        for (int a = 0; a < D; ++a) pn[a] = wrap_axis(pn[a], a, P.g);
-    }
-    io.out_pos[i] = make_float4(pn[0], pn[1], pn[2], pn[3]);
-    float nxt[SM];
-#pragma unroll
-    for (int c = 0; c < SM; ++c) {
-        float dsc = u[D + c];
-        if (P.gates3d) dsc *= sg;
-        float next = si[c] + P.dt * dsc * m;
-        if (clamped_channel(D, S, (uint32_t)c)) next = clampf_(next, -8.0f, 24.0f);
-        nxt[c] = next;
-    }
-    float* os = io.out_states + (uint64_t)i * S;
-    if (S == SM) {  // 16-byte aligned rows (checked on the host)
-        float4* o4 = reinterpret_cast<float4*>(os);
-#pragma unroll
-        for (int q = 0; q < SM / 4; ++q) o4[q] = make_float4(nxt[4 * q], nxt[4 * q + 1], nxt[4 * q + 2], nxt[4 * q + 3]);
-    } else {
-#pragma unroll
-        for (int c = 0; c < SM; ++c)
-            if ((uint32_t)c < S) os[c] = nxt[c];
-    }
-}
-
-#if NPA_PART_MAIN
-// forward_from_features_with_eps (model.rs:867-940) for explicit feature rows.
-__global__ __launch_bounds__(256) void k_mlp_forward(StepParams P, const float* __restrict__ features,
-                                                     uint32_t rows, const float* __restrict__ w1,
-                                                     const float* __restrict__ b1,
-                                                     const float* __restrict__ w2,
-                                                     const float* __restrict__ b2, float* __restrict__ dx,
-                                                     float* __restrict__ ds, int dim) {
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    const uint32_t F = P.F, H = P.H, S = P.S, O = dim + S;
-    const float* f = features + (uint64_t)r * F;
-    float u[3 + 32];
-    for (uint32_t o = 0; o < O; ++o) u[o] = b2[o];
-    for (uint32_t h = 0; h < H; ++h) {
-        float sum = b1[h];
-        const float* wr = w1 + (uint64_t)h * F;
-        for (uint32_t k = 0; k < F; ++k) sum += wr[k] * f[k];
-        const float hv = fmaxf(sum, 0.0f);
-        for (uint32_t o = 0; o < O; ++o) u[o] += w2[(uint64_t)o * H + h] * hv;
-    }
-    float norm = 0.0f;
-    for (int a = 0; a < dim; ++a) norm += u[a] * u[a];
-    norm = sqrtf(norm);
-    float* px = dx + 4 * (uint64_t)r;
-    px[0] = px[1] = px[2] = px[3] = 0.0f;
-    for (int a = 0; a < dim; ++a) px[a] = P.alpha * u[a] * P.motion_eps / (1.0f + norm);
-    for (uint32_t c = 0; c < S; ++c) ds[(uint64_t)r * S + c] = u[dim + c];
-}
-
 // euler_step  crates/burn_automata_kernels/src/reference/step.rs:4-55
 __global__ __launch_bounds__(256) void k_euler(GridParams g, const float4* __restrict__ pos,
                                                const float* __restrict__ states,
@@ -1892,78 +1525,21 @@ static hipError_t launch_perceive_d(const StepParams& p, Workspace& ws, const St
 }
 
 #if NPA_PART_MAIN
-size_t valu_weight_floats(const StepParams& p) {
-    const uint32_t D = (uint32_t)p.g.dim;
-    const size_t HP = (p.H + 127) / 128 * 128;
-    const size_t OP = (D + p.SS + 3) / 4 * 4;
-    return ((size_t)p.FP * HP + HP + (size_t)p.H * OP + OP + 3) / 4 * 4;  // the fused layout stays 16-byte aligned
-}
-
-size_t padded_weight_floats(const StepParams& p) { return valu_weight_floats(p) + fused_weight_floats(p); }
-
 bool fused_update_applies(const StepParams& p) {
     return p.SS == 16 && p.H <= 128 && (uint64_t)p.T * 64 < (1ull << 32);
 }
 
+size_t padded_weight_floats(const StepParams& p) {
+    return fused_update_applies(p) ? fused_weight_floats(p) : mlp_weight_floats(p);
+}
+
 hipError_t launch_pad_weights(const StepParams& p, const float* w1, const float* b1, const float* w2,
                               const float* b2, float* wpad, hipStream_t stream) {
-    const size_t n = valu_weight_floats(p);
-    const uint32_t blocks = (uint32_t)std::min<size_t>((n + 255) / 256, 1024);
-    hipLaunchKernelGGL(k_pad_weights, dim3(blocks), dim3(256), 0, stream, p, p.g.dim, w1, b1, w2, b2, wpad);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_pad_weights_fused(p, w1, b1, w2, b2, wpad + n, stream);
+    return fused_update_applies(p) ? launch_pad_weights_fused(p, w1, b1, w2, b2, wpad, stream)
+                                   : launch_mlp_weights(p, w1, b1, w2, b2, wpad, stream);
 }
 
 #endif  // NPA_PART_MAIN
-
-template <int D, int SM, int FM, int ENG>
-static hipError_t launch_mlp_e(const StepParams& p, Workspace& ws, const StepIO& io, hipStream_t stream,
-                               Profiler* prof) {
-    constexpr int OP = (D + SM + 3) / 4 * 4;
-    const size_t HP = (p.H + 127) / 128 * 128;
-    // hid [HP][64] (the VALU path first holds the four waves' w1t slices there), ul [64][OP+1],
-    // then the VALU path's w2t copy [H][OP]
-    const size_t hid_end = HP == 128 ? std::max<size_t>(HP * 64, 4 * (size_t)FM * 32) : HP * 64;
-    const size_t lds = (hid_end + 64 * (OP + 1) + (ENG == 0 ? (size_t)p.H * OP : 0)) * 4;
-    if (lds > 65536) {
-        static LdsLimitFlags limit;
-        const hipError_t e = raise_lds_limit((const void*)k_mlp_euler<D, SM, FM, ENG>, limit);
-        if (e != hipSuccess) return e;
-    }
-    const uint32_t blocks = (p.T + 63) / 64;
-    return launch_timed(prof, NPA_KERNEL_MLP, k_mlp_euler<D, SM, FM, ENG>, dim3(blocks), dim3(256), (uint32_t)lds,
-                        stream, p, ws.features.as<float>(), ws.sstate.as<float>(), ws.perm.as<uint32_t>(),
-                        ws.act_rows.as<uint32_t>(), ws.wl_count.as<uint32_t>() + 1, ws.wpad.as<float>(), io);
-}
-
-template <int D, int SM, int FM>
-static hipError_t launch_mlp_t(const StepParams& p, Workspace& ws, const StepIO& io, hipStream_t stream,
-                               Profiler* prof) {
-    if (p.mlp_engine != NPA_MLP_VALU) return launch_mlp_e<D, SM, FM, 1>(p, ws, io, stream, prof);
-    return launch_mlp_e<D, SM, FM, 0>(p, ws, io, stream, prof);
-}
-
-template <int D, int SM>
-static hipError_t launch_mlp_sm(const StepParams& p, Workspace& ws, const StepIO& io, hipStream_t stream,
-                                Profiler* prof) {
-    constexpr int base = 2 * SM + SM * D;
-    if (p.FP == (uint32_t)base) return launch_mlp_t<D, SM, base>(p, ws, io, stream, prof);
-    if (p.FP == (uint32_t)base + 4) return launch_mlp_t<D, SM, base + 4>(p, ws, io, stream, prof);
-    return launch_mlp_t<D, SM, base + 8>(p, ws, io, stream, prof);
-}
-
-template <int D>
-static hipError_t launch_mlp_d(const StepParams& p, Workspace& ws, const StepIO& io, hipStream_t stream,
-                               Profiler* prof) {
-    switch (p.SS) {
-        case 4: return launch_mlp_sm<D, 4>(p, ws, io, stream, prof);
-        case 8: return launch_mlp_sm<D, 8>(p, ws, io, stream, prof);
-        case 16: return launch_mlp_sm<D, 16>(p, ws, io, stream, prof);
-        case 24: return launch_mlp_sm<D, 24>(p, ws, io, stream, prof);
-        default: return launch_mlp_sm<D, 32>(p, ws, io, stream, prof);
-    }
-}
 
 // Second pass, then (mode 0) the update MLP, for one dimension; the rollout step's usual shape
 // (16-wide rows, H <= 128) runs both in the fused kernel, with either MLP engine.
@@ -1971,14 +1547,14 @@ template <int D>
 static hipError_t launch_second_pass(const StepParams& p, Workspace& ws, const StepIO& io, int mode, int blocks,
                                      hipStream_t stream, Profiler* prof) {
     if (mode == 0 && fused_update_applies(p)) {
-        const float* wfused = ws.wpad.as<float>() + valu_weight_floats(p);
+        const float* wfused = ws.wpad.as<float>();
         return D == 2 ? launch_update_fused_2d(p, ws, io, wfused, stream, prof)
                       : launch_update_fused_3d(p, ws, io, wfused, stream, prof);
     }
     const hipError_t e = mode == 0 ? launch_perceive_d<D, 0>(p, ws, io, blocks, stream, prof)
                                    : launch_perceive_d<D, 1>(p, ws, io, blocks, stream, prof);
     if (e != hipSuccess || mode != 0) return e;
-    return launch_mlp_d<D>(p, ws, io, stream, prof);
+    return launch_mlp_euler(p, ws, io, stream, prof);
 }
 
 #if NPA_PART_DIM2
@@ -2001,14 +1577,6 @@ hipError_t launch_update(const StepParams& p_in, Workspace& ws, const StepIO& io
     const int blocks = grid_blocks * 4;  // one wave per block
     return p.g.dim == 2 ? launch_second_pass_2d(p, ws, io, mode, blocks, stream, prof)
                         : launch_second_pass_3d(p, ws, io, mode, blocks, stream, prof);
-}
-
-hipError_t launch_mlp_forward(const StepParams& p, const float* features, uint32_t rows, const StepIO& io,
-                              float* dx, float* ds, hipStream_t stream) {
-    if (rows == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((rows + 255) / 256), dim3(256), 0, stream, p, features, rows,
-                       io.w1, io.b1, io.w2, io.b2, dx, ds, p.g.dim);
-    return hipGetLastError();
 }
 
 hipError_t launch_euler(const StepParams& p, const float4* pos, const float* states, const float4* dx,

@@ -1,0 +1,54 @@
+"""The update MLP on explicit rows and the two-kernel step, bit for bit against the oracle at the edges
+of its tiles: 16 rows per block, 64 hidden units per wave, chunks of 128 or 256 units, output groups of
+16, feature counts that are not a multiple of four."""
+import numpy as np
+import pytest
+
+from burn_automata_amd import synthetic as syn
+from burn_automata_amd.config import Boundary, HashGridConfig, HashGridMode, NpaConfig
+from burn_automata_amd.model import NpaModel
+from helpers import to_np
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _weights(m, seed):
+    rng = np.random.default_rng(seed)
+    F, H, Od = m.perception_dims(), m.hidden_dims, m.update_dims()
+    w = {"w1": rng.normal(size=H * F), "b1": rng.normal(size=H), "w2": rng.normal(size=Od * H), "b2": rng.normal(size=Od)}
+    return {k: (0.3 * v).astype(f32) for k, v in w.items()}
+
+
+@pytest.mark.parametrize("rows,d,S,H,dgrad", [
+    (1, 2, 16, 128, True), (15, 2, 16, 128, False), (16, 3, 24, 256, True), (17, 2, 1, 1, False), (33, 3, 32, 300, True),
+    (31, 2, 13, 64, True), (40, 3, 29, 65, False), (5, 2, 4, 129, True), (64, 2, 32, 513, True), (18, 3, 5, 63, False)])
+def test_mlp_forward_bit_exact(ctx, rows, d, S, H, dgrad):
+    m = NpaConfig(spatial_dims=d, state_dims=S, hidden_dims=H, density_grad=dgrad)
+    w = _weights(m, rows)
+    rng = np.random.default_rng(rows + H)
+    feats = rng.normal(size=(rows, m.perception_dims())).astype(f32)
+    feats.reshape(-1)[::7] *= f32(1e-30)   # denormal products
+    feats.reshape(-1)[::11] = f32(-0.0)
+    feats.reshape(-1)[::13] *= f32(1e6)
+    want_dx, want_ds = O.forward_from_features_with_eps(m, w, feats, 0.1)
+    dx, ds = NpaModel(m, w).forward_from_features_with_eps(feats, 0.1, ctx=ctx)
+    np.testing.assert_array_equal(to_np(dx), np.asarray(want_dx).reshape(rows, 4))
+    np.testing.assert_array_equal(to_np(ds), np.asarray(want_ds).reshape(rows, S))
+
+
+@pytest.mark.parametrize("d,S,H,n,periodic", [(2, 16, 256, 333, False), (2, 8, 129, 65, True), (3, 24, 256, 500, False),
+                                              (3, 32, 300, 47, False), (2, 5, 1, 15, False)])
+def test_two_kernel_step_bit_exact(ctx, d, S, H, n, periodic):
+    m = NpaConfig(spatial_dims=d, state_dims=S, hidden_dims=H, density_grad=d == 2)
+    g = HashGridConfig(d, Boundary.Periodic, HashGridMode.Grid, (10, 10, 10)[:d] + (1,) * (3 - d), 0.2, 32) if periodic \
+        else HashGridConfig(d, Boundary.Clamped, HashGridMode.Particle, (16, 16, 16), 0.1, 32)
+    w = _weights(m, n)
+    pos = syn.uniform_disk(n, 3, 0.8) if d == 2 else syn.uniform_ball(n, 3, 0.4)
+    st = syn.normal_states(n, S, 3)
+    mask = (np.random.default_rng(1).random(n) < 0.6).astype(f32)
+    want = O.step(m, w, pos, st, 1, n, g, 1.0, mask)
+    got = NpaModel(m, w).step(pos, st, 1, n, g, 1.0, update_mask=mask, ctx=ctx)
+    np.testing.assert_array_equal(to_np(got.next_positions), want.next_positions)
+    np.testing.assert_array_equal(to_np(got.next_states), want.next_states)
