@@ -81,7 +81,10 @@ __device__ __forceinline__ float f4(const float4& v, int k) { return k == 0 ? v.
 //
 // Bound: the ordered adds, one wave instruction per 64 of them, on up to 1,024 SIMDs: 16 rows x 64
 // units x F features take 64 F cycles. 16 rows per block (rather than a row per lane, 64 rows) keep
-// small systems on every CU: 4,096 rows are 256 blocks.
+// small systems on every CU: 4,096 rows are 256 blocks. Measured: forward_from_features of 32,008 rows,
+// F = 66, H = 128, O = 18: 1,304 us with a thread per row reading features and weights at a stride ->
+// 34.5 us; the step's MLP for 4,096 rows, F = 123, H = 256, O = 27: 67.5 us with 64 rows per block and
+// v_mul + v_add -> 21.3 us.
 //
 // The hidden units are taken in chunks of 64 per wave, so LDS does not grow with H.
 //
@@ -179,13 +182,19 @@ __device__ __forceinline__ void mlp_rows(uint32_t F, uint32_t H, uint32_t O, con
                 const uint32_t full = F / 4, rest = F % 4;
                 if constexpr (RAW) {
                     float* wt = tile + wave * 64 * kTileS;
-                    float next[16];  // instruction i: units 4 i + lane / 16, feature lane % 16 of the tile
-                    auto fetch = [&](uint32_t k0) {
+                    // load i: units 4 i + lane / 16, feature lane % 16 of the tile; units past H repeat the last
+                    // one (their sums are never read), features past F the last feature (never added)
+                    float next[16];
+                    const float* src[16];
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const uint32_t u = u0 + 4 * i + lk, k = k0 + li;
-                            next[i] = u < H && k < F ? raw.w1[(uint64_t)u * F + k] : 0.0f;
-                        }
+                    for (int i = 0; i < 16; ++i) {
+                        const uint32_t u = u0 + 4 * i + lk;
+                        src[i] = raw.w1 + (uint64_t)(u < H ? u : H - 1) * F;
+                    }
+                    auto fetch = [&](uint32_t k0) {
+                        const uint32_t k = k0 + li < F ? k0 + li : F - 1;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) next[i] = src[i][k];
                     };
                     fetch(0);
                     for (uint32_t k0 = 0; k0 < F; k0 += kTileK) {
@@ -193,26 +202,44 @@ __device__ __forceinline__ void mlp_rows(uint32_t F, uint32_t H, uint32_t O, con
 #pragma unroll
                         for (int i = 0; i < 16; ++i) wt[(4 * i + lk) * kTileS + li] = next[i];
                         mlp_wave_sync();
-                        if (k0 + kTileK < F) fetch(k0 + kTileK);
+                        fetch(k0 + kTileK);
                         const float4* b4 = reinterpret_cast<const float4*>(wt + lane * kTileS);
+                        const uint32_t left = full - k0 / 4;  // whole groups of four left
+                        if (left >= kTileK / 4) {
 #pragma unroll
-                        for (uint32_t g = 0; g < kTileK / 4; ++g) {
-                            const uint32_t k = k0 / 4 + g;
-                            if (k < full) add_products<4>(acc, a4[k], b4[g], zero16);
-                            else if (k == full && rest) add_rest(acc, a4[k], b4[g], zero16, rest);
+                            for (uint32_t g = 0; g < kTileK / 4; ++g) add_products<4>(acc, a4[k0 / 4 + g], b4[g], zero16);
+                        } else {
+                            for (uint32_t g = 0; g < left; ++g) add_products<4>(acc, a4[k0 / 4 + g], b4[g], zero16);
+                            add_rest(acc, a4[full], b4[left], zero16, rest);
                         }
                     }
                 } else {
                     const float4* b4 = w1 + u0 + lane;
-                    float4 b = b4[0], a = a4[0];
-                    for (uint32_t k = 0; k < full; ++k) {
-                        const uint32_t kn = k + 1 < l.K4 ? k + 1 : k;  // the next four features, loaded ahead
-                        const float4 bn = b4[(uint64_t)kn * l.HC], an = a4[kn];
-                        add_products<4>(acc, a, b, zero16);
-                        a = an;
-                        b = bn;
+                    float4 next[4];  // the next sixteen features' weights, in flight while these are added
+                    auto fetch = [&](uint32_t k) {
+#pragma unroll
+                        for (uint32_t g = 0; g < 4; ++g) next[g] = b4[(uint64_t)(k + g < l.K4 ? k + g : l.K4 - 1) * l.HC];
+                    };
+                    fetch(0);
+                    float4 tail = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    for (uint32_t k0 = 0; k0 < l.K4; k0 += 4) {
+                        float4 b[4];
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) b[g] = next[g];
+                        fetch(k0 + 4);
+                        __builtin_amdgcn_sched_barrier(0);  // the loads go out before the products
+                        if (full - k0 >= 4) {
+#pragma unroll
+                            for (uint32_t g = 0; g < 4; ++g) add_products<4>(acc, a4[k0 + g], b[g], zero16);
+                        } else {
+#pragma unroll
+                            for (uint32_t g = 0; g < 4; ++g) {
+                                if (k0 + g < full) add_products<4>(acc, a4[k0 + g], b[g], zero16);
+                                if (k0 + g == full) tail = b[g];
+                            }
+                        }
                     }
-                    add_rest(acc, a, b, zero16, rest);
+                    add_rest(acc, a4[full], tail, zero16, rest);
                 }
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -247,22 +274,46 @@ __device__ __forceinline__ void mlp_rows(uint32_t F, uint32_t H, uint32_t O, con
                     const float4* b4 = w2 + (uint64_t)(hb / 4) * l.OC + first + o4;
                     // raw: this lane's output row (the last one in place of a padded output), units past H clamped
                     const float* wr = raw.w2 + (uint64_t)(first + o4 < O ? first + o4 : O - 1) * H;
-                    auto weights = [&](uint32_t k) {
+                    auto weights = [&](uint32_t k) {  // a whole group of four units
                         if constexpr (!RAW) return b4[(uint64_t)k * l.OC];
-                        const uint32_t h = hb + 4 * k, last = H - 1;
-                        return make_float4(wr[h], wr[h + 1 < H ? h + 1 : last], wr[h + 2 < H ? h + 2 : last],
-                                           wr[h + 3 < H ? h + 3 : last]);
+                        const float* w = wr + hb + 4 * k;
+                        return make_float4(w[0], w[1], w[2], w[3]);
                     };
-                    const uint32_t full = units / 4, rest = units % 4, groups = (units + 3) / 4;
-                    float4 b = weights(0), a = a4[0];
-                    for (uint32_t k = 0; k < full; ++k) {
-                        const uint32_t kn = k + 1 < groups ? k + 1 : k;
-                        const float4 bn = weights(kn), an = a4[kn];
-                        add_products<4>(acc2[g], a, b, zero4);
-                        a = an;
-                        b = bn;
+                    const uint32_t full = units / 4, rest = units % 4;
+                    constexpr uint32_t W = 8;
+                    if (full) {
+                        float4 next[W];
+                        auto fetch = [&](uint32_t k) {
+#pragma unroll
+                            for (uint32_t e = 0; e < W; ++e) next[e] = weights(k + e < full ? k + e : full - 1);
+                        };
+                        fetch(0);
+                        for (uint32_t k0 = 0; k0 < full; k0 += W) {
+                            float4 b[W];
+#pragma unroll
+                            for (uint32_t e = 0; e < W; ++e) b[e] = next[e];
+                            fetch(k0 + W);
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (full - k0 >= W) {
+#pragma unroll
+                                for (uint32_t e = 0; e < W; ++e) add_products<4>(acc2[g], a4[k0 + e], b[e], zero4);
+                            } else {
+#pragma unroll
+                                for (uint32_t e = 0; e < W; ++e)
+                                    if (k0 + e < full) add_products<4>(acc2[g], a4[k0 + e], b[e], zero4);
+                            }
+                        }
                     }
-                    add_rest(acc2[g], a, b, zero4, rest);
+                    if (rest) {
+                        float4 b;
+                        if constexpr (RAW) {
+                            const float* w = wr + hb + 4 * full;
+                            b = make_float4(w[0], rest > 1 ? w[1] : 0.0f, rest > 2 ? w[2] : 0.0f, 0.0f);
+                        } else {
+                            b = b4[(uint64_t)full * l.OC];
+                        }
+                        add_rest(acc2[g], a4[full], b, zero4, rest);
+                    }
                 } else {
                     // a chunk's units past H hold relu(0) = 0 and meet zero weights
                     const float* wk = wp + l.w2 + ((uint64_t)(hb / 4) * l.OC + first + li) * 4 + lk;
@@ -292,12 +343,20 @@ __device__ __forceinline__ void mlp_rows(uint32_t F, uint32_t H, uint32_t O, con
 // the 16 rows of a read fall on different banks.
 __host__ __device__ inline uint32_t mlp_feature_stride(uint32_t F) { return ((F + 3) / 4 | 1u) * 4; }
 
+// A wave takes every NW-th row; features past F and rows past the last are zeros.
 template <int NW>
 __device__ __forceinline__ void stage_rows(const float* __restrict__ src, uint32_t rows, uint32_t F, float* feat,
                                            uint32_t FS) {
-    for (uint32_t t = threadIdx.x; t < kMlpRows * FS; t += NW * 64) {
-        const uint32_t r = t / FS, k = t - r * FS;
-        feat[t] = r < rows && k < F ? src[(uint64_t)r * F + k] : 0.0f;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t k = lane; k < FS; k += 64) {
+        float v[kMlpRows / NW];
+#pragma unroll
+        for (int i = 0; i < kMlpRows / NW; ++i) {
+            const uint32_t r = wave + NW * i;
+            v[i] = r < rows && k < F ? src[(uint64_t)r * F + k] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < kMlpRows / NW; ++i) feat[(wave + NW * i) * FS + k] = v[i];
     }
     __syncthreads();
 }
@@ -317,7 +376,7 @@ constexpr uint32_t kMlpUlStride = 49;  // outputs of a row in LDS (48 with the p
 
 // forward_from_features_with_eps (model.rs:867-940) for explicit feature rows [rows][F].
 template <int D, int NW>
-__global__ __launch_bounds__(NW * 64) void k_mlp_forward(StepParams P, const float* __restrict__ features, uint32_t rows,
+__global__ __launch_bounds__(NW * 64, 2) void k_mlp_forward(StepParams P, const float* __restrict__ features, uint32_t rows,
                                                          RawWeights raw, float* __restrict__ dx,
                                                          float* __restrict__ ds) {
     extern __shared__ __align__(16) float lds[];
@@ -349,7 +408,7 @@ __global__ __launch_bounds__(NW * 64) void k_mlp_forward(StepParams P, const flo
 // (model.rs:806-837) and the masked Euler step (step.rs:4-55). A row's first S features are its
 // particle's state.
 template <int D, int ENG, int NW>
-__global__ __launch_bounds__(NW * 64) void k_mlp_euler(StepParams P, const float* __restrict__ features,
+__global__ __launch_bounds__(NW * 64, 2) void k_mlp_euler(StepParams P, const float* __restrict__ features,
                                                        const uint32_t* __restrict__ perm,
                                                        const uint32_t* __restrict__ act_rows,
                                                        const uint32_t* __restrict__ row_count,
