@@ -626,7 +626,9 @@ npa_status npa_perceive_adjoint(npa_context* ctx, const float* positions, const 
     if (total) {
         NPA_HIP(ctx, npa::launch_hashgrid(plan, p.g, pos, st_in, S, B, N, ctx->ws, true, ctx->stream, &ctx->prof),
                 "hashgrid");
-        NPA_HIP(ctx, npa::launch_perceive_adjoint(p, ctx->ws, ctx->adj_ws, fa, sa, pa, ctx->stream), "adjoint");
+        NPA_HIP(ctx, npa::launch_perceive_adjoint(p, ctx->ws, ctx->adj_ws, fa, sa, pa, grid_blocks_for(ctx, plan),
+                                                 ctx->stream),
+                "adjoint");
     }
     NPA_HIP(ctx, io.finish(), "host io");
     if (!position_adjoint) {

@@ -149,4 +149,183 @@ __device__ __forceinline__ void neighbor_runs(const StepParams& P, const uint32_
     found = cell_range(P, bo, b, (int64_t)c0 + dx, (int64_t)c1 + dy, (int64_t)c2 + dz, beg, end, filter);
 }
 
+// Value of lane (group base + j) for groups of L consecutive lanes (L = 1, 2 or 4), via DPP.
+// quad_perm reads a valid lane for every lane, so bound_ctrl (zero for an invalid source lane)
+// never applies; with it set the compiler folds the permutation into the consuming VALU
+// instruction (v_mul_f32_dpp, v_add_f32_dpp) instead of issuing a separate move.
+template <int L, int J>
+__device__ __forceinline__ float group_bcast(float v) {
+    if constexpr (L == 1) {
+        return v;
+    } else if constexpr (L == 2) {
+        constexpr int c = J == 0 ? (0 | (0 << 2) | (2 << 4) | (2 << 6)) : (1 | (1 << 2) | (3 << 4) | (3 << 6));
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), c, 0xf, 0xf, true));
+    } else {
+        constexpr int c = J | (J << 2) | (J << 4) | (J << 6);
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), c, 0xf, 0xf, true));
+    }
+}
+
+// OR of a 64-bit value over each group of L consecutive lanes (L = 1, 2 or 4), via DPP.
+template <int L>
+__device__ __forceinline__ uint64_t group_or(uint64_t m) {
+    if constexpr (L == 1) return m;
+    uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+    constexpr int swap1 = 1 | (0 << 2) | (3 << 4) | (2 << 6);  // quad_perm [1,0,3,2]
+    lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, swap1, 0xf, 0xf, true);
+    hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, swap1, 0xf, 0xf, true);
+    if constexpr (L == 4) {
+        constexpr int swap2 = 2 | (3 << 2) | (0 << 4) | (1 << 6);  // quad_perm [2,3,0,1]
+        lo |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, swap2, 0xf, 0xf, true);
+        hi |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, swap2, 0xf, 0xf, true);
+    }
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Per-wave accepted-neighbour lists of the neighbour passes: the sorted slots of each target's accepted
+// candidates, appended in visit order (cells dz, dy, dx; slots ascending), so walking a list front
+// to back is the reference's neighbour order. kListBytes of LDS per wave for any targets-per-item.
+constexpr int kListBytes = 12288;
+
+template <int TPI>
+struct PerceiveLists {
+    static constexpr int CAP = kListBytes / (4 * TPI);
+    uint32_t slot[CAP][TPI];
+};
+
+// Bits k of a 64-bit chunk mask with k % L == q.
+template <int L>
+__device__ __forceinline__ uint64_t residue_mask(uint32_t q) {
+    if constexpr (L == 1) return ~0ull;
+    else if constexpr (L == 2) return 0x5555555555555555ull << q;
+    else return 0x1111111111111111ull << q;
+}
+
+// Appends each target's accepted candidates to its list in visit order: from the accept masks the
+// density pass recorded (the same test on the same candidates), or, where a target of the wave has
+// more chunks than were recorded, by testing the candidates here. Lane q of the L lanes of target t
+// holds its position pi, cell ci and compact row; `flush` consumes the lists and empties them (cnt = 0)
+// before one would overflow. The caller flushes what is left at the end.
+template <int D, int L, class Lists, class Flush>
+__device__ __forceinline__ void append_accepted(const StepParams& P, const float4* __restrict__ srec,
+                                                const int4* __restrict__ scoord, const uint32_t* __restrict__ bo,
+                                                const uint32_t* __restrict__ nb_base,
+                                                const uint64_t* __restrict__ nb_mask,
+                                                const uint32_t* __restrict__ nb_count, uint32_t row, bool active,
+                                                uint32_t b, const float* pi, const int* ci, uint32_t lane, uint32_t t,
+                                                uint32_t q, Lists& lists, uint32_t& cnt, Flush&& flush) {
+    constexpr uint32_t MAXC = max_chunks(D), CAP = Lists::CAP;
+    const uint64_t my_residue = residue_mask<L>(q);
+    // Phase A. The density pass recorded each target's accepted candidates per chunk, in visit
+    // order; the lists are built from those masks (RB chunk records loaded per batch).
+    const uint32_t nct = active ? nb_count[row] : 0u;
+    const bool recorded = !__ballot(nct > MAXC);
+    constexpr int RB = 2;  // chunk records loaded per batch
+    for (uint32_t cb = 0; recorded && __ballot(cb < nct); cb += RB) {
+        uint4 rc[RB];
+#pragma unroll
+        for (int u = 0; u < RB; ++u) {
+            const uint32_t c = cb + (uint32_t)u;
+            if (c < nct) {
+                const uint64_t mk = nb_mask[(uint64_t)row * MAXC + c];
+                rc[u] = make_uint4(nb_base[(uint64_t)row * MAXC + c], 0u, (uint32_t)mk, (uint32_t)(mk >> 32));
+            } else {
+                rc[u] = make_uint4(0u, 0u, 0u, 0u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < RB; ++u) {
+            const uint32_t c = cb + (uint32_t)u;
+            const uint64_t acc = ((uint64_t)rc[u].w << 32) | rc[u].z;  // 0 past the target's chunks
+            const uint32_t add = (uint32_t)__popcll(acc);
+            if (__ballot(cnt + add > CAP)) flush();
+            uint64_t mine = acc & my_residue;
+            while (mine) {
+                const uint32_t k = (uint32_t)__builtin_ctzll(mine);
+                mine &= mine - 1;
+                const uint32_t pos = cnt + (uint32_t)__popcll(acc & ((1ull << k) - 1ull));
+                lists.slot[pos][t] = rc[u].x + k;
+            }
+            cnt += add;
+        }
+    }
+    // Otherwise (a target with more chunks than were recorded): the coordinate groups of the
+    // item, then each group's neighbour cells in order, testing the candidates here.
+    uint64_t pending = recorded ? 0ull : __ballot(active);
+    while (pending) {
+        const int leader = __ffsll((unsigned long long)pending) - 1;
+        const int l0 = readlane_i(ci[0], leader), l1 = readlane_i(ci[1], leader);
+        const int l2 = D == 3 ? readlane_i(ci[2], leader) : 0;
+        const uint32_t lb = (uint32_t)readlane_i((int)b, leader);
+        const bool same = active && ci[0] == l0 && ci[1] == l1 && (D == 2 || ci[2] == l2) && b == lb;
+        const uint64_t group = __ballot(same) & pending;
+        pending &= ~group;
+        const bool in_group = (group >> lane) & 1ull;
+        uint32_t nb_beg, nb_end;
+        bool nb_filter, nb_found;
+        neighbor_runs<D>(P, bo, lb, l0, l1, l2, lane, nb_beg, nb_end, nb_filter, nb_found);
+        for (uint64_t cells = __ballot(nb_found); cells; cells &= cells - 1) {
+            const int nk = __ffsll((unsigned long long)cells) - 1;  // ascending = visit order
+            const int64_t n0 = (int64_t)l0 + nk % 3 - 1, n1 = (int64_t)l1 + (nk / 3) % 3 - 1;
+            const int64_t n2 = D == 3 ? (int64_t)l2 + nk / 9 - 1 : 0;
+            const uint32_t beg = (uint32_t)readlane_i((int)nb_beg, nk);
+            const uint32_t end = (uint32_t)readlane_i((int)nb_end, nk);
+            const bool filter = readlane_i((int)nb_filter, nk) != 0;
+            for (uint32_t base = beg; base < end; base += kNbChunk) {
+                const uint32_t m = end - base < (uint32_t)kNbChunk ? end - base : (uint32_t)kNbChunk;
+                // batches of 4 candidates per lane: loads first (index clamped to
+                // the chunk, so every load is in bounds), then branch-free tests
+                uint64_t acc = 0;
+                for (int i0 = 0; i0 < kNbChunk / L; i0 += 4) {
+                    if ((uint32_t)(i0 * L) >= m) break;  // wave-uniform
+                    float4 rc[4];
+                    int4 cc[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const uint32_t k = q + (uint32_t)((i0 + u) * L);
+                        const uint32_t kc = k < m ? k : m - 1;
+                        rc[u] = srec[base + kc];
+                        if constexpr (D == 3) cc[u] = scoord[base + kc];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const uint32_t k = q + (uint32_t)((i0 + u) * L);
+                        const float4 r = rc[u];
+                        bool ok = in_group & (k < m);
+                        if (filter) {
+                            if constexpr (D == 2) {
+                                ok = ok & ((int64_t)__float_as_int(r.z) == n0) &
+                                     ((int64_t)__float_as_int(r.w) == n1);
+                            } else {
+                                ok = ok & ((int64_t)cc[u].x == n0) & ((int64_t)cc[u].y == n1) &
+                                     ((int64_t)cc[u].z == n2);
+                            }
+                        }
+                        const float d0 = delta_axis(pi[0], r.x, 0, P.g);
+                        const float d1 = delta_axis(pi[1], r.y, 1, P.g);
+                        float r2 = d0 * d0;
+                        r2 += d1 * d1;
+                        if constexpr (D == 3) {
+                            const float d2 = delta_axis(pi[2], r.z, 2, P.g);
+                            r2 += d2 * d2;
+                        }
+                        acc |= (ok & (r2 < P.g.eps2)) ? (1ull << (k & 63u)) : 0ull;
+                    }
+                }
+                acc = group_or<L>(acc);
+                const uint32_t add = (uint32_t)__popcll(acc);
+                if (__ballot(cnt + add > CAP)) flush();
+                uint64_t mine = acc & my_residue;
+                while (mine) {
+                    const uint32_t k = (uint32_t)__builtin_ctzll(mine);
+                    mine &= mine - 1;
+                    const uint32_t pos = cnt + (uint32_t)__popcll(acc & ((1ull << k) - 1ull));
+                    lists.slot[pos][t] = base + k;
+                }
+                cnt += add;
+            }
+        }
+    }
+}
+
 }  // namespace npa
