@@ -45,7 +45,20 @@ struct npa_context {
     std::atomic<bool> used_noalloc{false};
     // the caller's handle plus one per live npa_state: a state keeps its context until it is destroyed
     std::atomic<int> refs{1};
+    // Device blocks of destroyed states, for the next ones: a rollout of 64 x 4,096 particles spent more
+    // time in the allocation and release of its 118 MB state than in 16 steps (6.0 ms a call, 2.8 ms of it kernels).
+    // Bounded (kPoolBlocks blocks, kPoolBytes in all), given back when an allocation fails and with the
+    // context, locked because states may be destroyed on any thread.
+    struct Block { void* ptr; size_t bytes; };
+    std::mutex pool_mutex;
+    std::vector<Block> pool;
+    size_t pool_bytes = 0;
+    std::atomic<uint32_t> stream_changes{0};  // npa_context_set_stream calls that changed the stream
+    hipError_t block_acquire(size_t bytes, Block* out);
+    void block_release(Block b);
+    void pool_clear();
     ~npa_context() {
+        pool_clear();
         ws.release();
         splat_ws.release();
         adj_ws.release();
@@ -65,18 +78,68 @@ struct npa_state {
     uint64_t seed = 0;
     uint64_t step_index = 0;
     int mlp_engine = NPA_MLP_VALU;
-    DevBuf pos[2], states[2], density, w1, b1, w2, b2;
+    npa_context::Block block{};              // one allocation; the buffers below and ws are views into it
+    uint32_t stream_changes = 0;             // the context's count when the state was created
+    bool exposed = false;                    // npa_state_buffers handed out its addresses
+    DevBuf pos[2], states[2], density, staged_weights;
     int cur = 0;
     npa::Workspace ws;
     npa::SplatWorkspace splat_ws;
     npa::HashgridPlan plan;
     int grid_blocks = 1;
-    ~npa_state() {
-        for (DevBuf* b : {&pos[0], &pos[1], &states[0], &states[1], &density, &w1, &b1, &w2, &b2}) b->release();
-        ws.release();
-        splat_ws.release();
-    }
+    ~npa_state() { splat_ws.release(); }
 };
+
+constexpr size_t kPoolBlocks = 4, kPoolBytes = (size_t)1 << 30;
+
+void npa_context::pool_clear() {
+    std::lock_guard<std::mutex> lock(pool_mutex);
+    for (const Block& b : pool) (void)hipFree(b.ptr);
+    pool.clear();
+    pool_bytes = 0;
+}
+
+// The smallest kept block that fits without wasting more than its need again, else a new one.
+hipError_t npa_context::block_acquire(size_t bytes, Block* out) {
+    constexpr size_t kGrain = (size_t)2 << 20;
+    const size_t want = (bytes + kGrain - 1) / kGrain * kGrain;
+    {
+        std::lock_guard<std::mutex> lock(pool_mutex);
+        size_t best = pool.size();
+        for (size_t k = 0; k < pool.size(); ++k)
+            if (pool[k].bytes >= want && pool[k].bytes <= 2 * want && (best == pool.size() || pool[k].bytes < pool[best].bytes))
+                best = k;
+        if (best < pool.size()) {
+            *out = pool[best];
+            pool_bytes -= out->bytes;
+            pool.erase(pool.begin() + (ptrdiff_t)best);
+            return hipSuccess;
+        }
+    }
+    *out = Block{nullptr, want};
+    hipError_t e = hipMalloc(&out->ptr, want);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        pool_clear();
+        e = hipMalloc(&out->ptr, want);
+    }
+    if (e != hipSuccess) *out = Block{nullptr, 0};
+    return e;
+}
+
+// No queued work may use the block any more.
+void npa_context::block_release(Block b) {
+    if (!b.ptr) return;
+    {
+        std::lock_guard<std::mutex> lock(pool_mutex);
+        if (pool.size() < kPoolBlocks && pool_bytes + b.bytes <= kPoolBytes) {
+            pool.push_back(b);
+            pool_bytes += b.bytes;
+            return;
+        }
+    }
+    (void)hipFree(b.ptr);
+}
 
 namespace {
 
@@ -335,6 +398,80 @@ npa_status check_flags(npa_context* ctx, npa::Workspace& ws) {
     return NPA_OK;
 }
 
+// Word copies and clears between arrays on the device in one launch (a caller's arrays need only be
+// float aligned): words [first[k-1], first[k]) belong to segment k, a null source clears.
+struct Segments {
+    static constexpr int MAX = 5;
+    uint32_t* dst[MAX];
+    const uint32_t* src[MAX];
+    uint64_t end[MAX];
+    int count = 0;
+    void add(void* d, const void* s, uint64_t words) {
+        if (!words) return;
+        dst[count] = (uint32_t*)d;
+        src[count] = (const uint32_t*)s;
+        end[count] = (count ? end[count - 1] : 0) + words;
+        ++count;
+    }
+};
+__global__ __launch_bounds__(256) void k_segments(Segments g) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    uint64_t begin = 0;
+    for (int k = 0; k < g.count; ++k) {
+        const uint64_t n = g.end[k] - begin;
+        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+            g.dst[k][i] = g.src[k] ? g.src[k][i] : 0u;
+        begin = g.end[k];
+    }
+}
+hipError_t launch_segments(const Segments& g, hipStream_t stream) {
+    if (!g.count) return hipSuccess;
+    const uint64_t words = g.end[g.count - 1];
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((words + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_segments, dim3(blocks), dim3(256), 0, stream, g);
+    return hipGetLastError();
+}
+
+// Whether a kernel on the context's device may read or write the caller's array: memory of that device.
+// Anything else (host-I/O mode, another GPU's memory, host memory) is copied by the runtime.
+bool kernel_reachable(const npa_context* ctx, const void* p) {
+    if (ctx->host_io) return false;
+    hipPointerAttribute_t attr{};
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError();  // not an address the runtime knows
+        return false;
+    }
+    return attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
+}
+
+// Lays out a model's weights for its step kernel: from the caller's arrays, or through the state's
+// staging area where a kernel cannot read them.
+hipError_t pad_state_weights(npa_state* s, const npa_weights* w, const npa::StepParams& sp) {
+    npa_context* ctx = s->ctx;
+    const uint64_t H = s->model.hidden_dims, F = sp.F, O = s->model.spatial_dims + s->model.state_dims;
+    const float *w1 = w->w1, *b1 = w->b1, *w2 = w->w2, *b2 = w->b2;
+    const hipMemcpyKind kind = ctx->host_io ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+    const uint64_t sizes[4] = {H * F, H, O * H, O};
+    const float* arrays[4] = {w1, b1, w2, b2};
+    bool direct = true;
+    for (int k = 0; k < 4; ++k) direct = direct && (!sizes[k] || kernel_reachable(ctx, arrays[k]));
+    if (!direct) {
+        float* at = s->staged_weights.as<float>();
+        auto stage = [&](const float*& src, uint64_t n) {
+            hipError_t e = n ? hipMemcpyAsync(at, src, n * 4, kind, ctx->stream) : hipSuccess;
+            src = at;
+            at += n;
+            return e;
+        };
+        hipError_t e = stage(w1, H * F);
+        if (e == hipSuccess) e = stage(b1, H);
+        if (e == hipSuccess) e = stage(w2, O * H);
+        if (e == hipSuccess) e = stage(b2, O);
+        if (e != hipSuccess) return e;
+    }
+    return npa::launch_pad_weights(sp, w1, b1, w2, b2, s->ws.wpad.as<float>(), ctx->stream);
+}
+
 npa_status set_device(npa_context* ctx) {
     NPA_HIP(ctx, hipSetDevice(ctx->device), "hipSetDevice");
     return NPA_OK;
@@ -386,6 +523,7 @@ void npa_context_destroy(npa_context* ctx) {
 
 npa_status npa_context_set_stream(npa_context* ctx, void* stream) {
     if (!ctx) return NPA_ERR_INVALID_ARGUMENT;
+    if (ctx->stream != (hipStream_t)stream) ctx->stream_changes.fetch_add(1);
     ctx->stream = (hipStream_t)stream;
     return NPA_OK;
 }
@@ -1095,38 +1233,48 @@ npa_status npa_state_create(npa_context* ctx, const npa_model_cfg* model, const 
     s->seed = seed;
     s->plan = plan;
     s->grid_blocks = grid_blocks_for(ctx, plan);
+    s->stream_changes = ctx->stream_changes.load();
     const uint32_t S = model->state_dims, F = model_perception_dims(*model), H = model->hidden_dims;
     const uint32_t O = model->spatial_dims + S;
-    const hipMemcpyKind kind = ctx->host_io ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        e = s->pos[k].reserve(total * 16);
-        if (e == hipSuccess) e = s->states[k].reserve(total * S * 4);
-    }
-    if (e == hipSuccess) e = s->density.reserve(total * 4);
-    if (e == hipSuccess) e = s->w1.reserve((uint64_t)H * F * 4 + 4);
-    if (e == hipSuccess) e = s->b1.reserve((uint64_t)H * 4 + 4);
-    if (e == hipSuccess) e = s->w2.reserve((uint64_t)O * H * 4 + 4);
-    if (e == hipSuccess) e = s->b2.reserve((uint64_t)O * 4 + 4);
     const npa::StepParams sp = [&] {
         npa::StepParams q = make_params(*grid, opts_for_model(*model), B, N, S);
         apply_model(&q, *model, grid->eps);
         return q;
     }();
-    if (e == hipSuccess) e = s->ws.reserve(plan, total, B, S, (int)grid->dim, feature_rows_for(sp));
-    if (e == hipSuccess) e = s->ws.wpad.reserve(npa::padded_weight_floats(sp) * 4);
-    if (e == hipSuccess) e = hipMemcpyAsync(s->pos[0].ptr, positions, total * 16, kind, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(s->states[0].ptr, states, total * S * 4, kind, ctx->stream);
-    if (e == hipSuccess && (uint64_t)H * F) e = hipMemcpyAsync(s->w1.ptr, w->w1, (uint64_t)H * F * 4, kind, ctx->stream);
-    if (e == hipSuccess && H) e = hipMemcpyAsync(s->b1.ptr, w->b1, (uint64_t)H * 4, kind, ctx->stream);
-    if (e == hipSuccess && (uint64_t)O * H) e = hipMemcpyAsync(s->w2.ptr, w->w2, (uint64_t)O * H * 4, kind, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(s->b2.ptr, w->b2, (uint64_t)O * 4, kind, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(s->density.ptr, 0, total * 4, ctx->stream);
-    if (e == hipSuccess)
-        e = npa::launch_pad_weights(sp, s->w1.as<float>(), s->b1.as<float>(), s->w2.as<float>(), s->b2.as<float>(),
-                                    s->ws.wpad.as<float>(), ctx->stream);
+    // one block: the workspace, then the particle buffers, each on a 256-byte boundary
+    const uint64_t weights = ((uint64_t)H * F + H + (uint64_t)O * H + O) * 4;
+    const uint64_t sizes[6] = {total * 16, total * 16, total * S * 4, total * S * 4, total * 4, weights};
+    DevBuf* const views[6] = {&s->pos[0], &s->pos[1], &s->states[0], &s->states[1], &s->density, &s->staged_weights};
+    const uint64_t wpad_bytes = npa::padded_weight_floats(sp) * 4;
+    const uint64_t ws_bytes = s->ws.carve(plan, total, B, S, (int)grid->dim, feature_rows_for(sp), wpad_bytes, nullptr, 0);
+    uint64_t need_bytes = ws_bytes;
+    for (uint64_t n : sizes) need_bytes += (n + 255) / 256 * 256;
+    hipError_t e = ctx->block_acquire(need_bytes, &s->block);
+    if (e == hipSuccess) {
+        s->ws.carve(plan, total, B, S, (int)grid->dim, feature_rows_for(sp), wpad_bytes, s->block.ptr, ws_bytes);
+        s->ws.counters_kept = true;  // cleared below; nobody else writes them
+        char* at = static_cast<char*>(s->block.ptr) + ws_bytes;
+        for (int k = 0; k < 6; ++k) {
+            views[k]->view(at, sizes[k]);
+            at += (sizes[k] + 255) / 256 * 256;
+        }
+        Segments g;
+        const hipMemcpyKind kind = ctx->host_io ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+        if (kernel_reachable(ctx, positions)) g.add(s->pos[0].ptr, positions, total * 4);
+        else e = hipMemcpyAsync(s->pos[0].ptr, positions, total * 16, kind, ctx->stream);
+        if (kernel_reachable(ctx, states)) g.add(s->states[0].ptr, states, total * S);
+        else if (e == hipSuccess) e = hipMemcpyAsync(s->states[0].ptr, states, total * S * 4, kind, ctx->stream);
+        g.add(s->density.ptr, nullptr, total);
+        g.add(s->ws.bin_count.ptr, nullptr, s->ws.bin_count.bytes / 4);
+        g.add(s->ws.flags.ptr, nullptr, s->ws.flags.bytes / 4);
+        if (e == hipSuccess) e = launch_segments(g, ctx->stream);
+    }
+    if (e == hipSuccess) e = pad_state_weights(s, w, sp);
+    // the caller's arrays have been read when this returns
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);
+        if (s->block.ptr) (void)hipFree(s->block.ptr);
         delete s;
         return hip_fail(ctx, e, "state create");
     }
@@ -1140,6 +1288,14 @@ void npa_state_destroy(npa_state* s) {
     npa_context* ctx = s->ctx;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    if (s->exposed) {
+        // others may hold the addresses and have work on streams of their own: hipFree waits for it
+        (void)hipFree(s->block.ptr);
+    } else {
+        // a state that ran on another stream as well waits for that one too before its block is reused
+        if (s->stream_changes != ctx->stream_changes.load()) (void)hipDeviceSynchronize();
+        ctx->block_release(s->block);
+    }
     delete s;
     context_release(ctx);
 }
@@ -1156,10 +1312,6 @@ npa_status npa_state_step(npa_state* s, uint32_t steps) {
     p.base_seed = base_seed(s->seed);
     p.mlp_engine = (uint32_t)s->mlp_engine;
     npa::StepIO io;
-    io.w1 = s->w1.as<float>();
-    io.b1 = s->b1.as<float>();
-    io.w2 = s->w2.as<float>();
-    io.b2 = s->b2.as<float>();
     for (uint32_t k = 0; k < steps; ++k) {
         const int c = s->cur;
         p.step_index = (uint32_t)s->step_index;
@@ -1192,13 +1344,19 @@ npa_status npa_state_read(npa_state* s, float* positions, float* states, float* 
     if (!s) return NPA_ERR_INVALID_ARGUMENT;
     npa_context* ctx = s->ctx;
     if (set_device(ctx)) return NPA_ERR_DEVICE;
-    const uint64_t total = (uint64_t)s->B * s->N;
+    const uint64_t total = (uint64_t)s->B * s->N, S = s->model.state_dims;
     const hipMemcpyKind kind = ctx->host_io ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
-    if (positions) NPA_HIP(ctx, hipMemcpyAsync(positions, s->pos[s->cur].ptr, total * 16, kind, ctx->stream), "read pos");
-    if (states)
-        NPA_HIP(ctx, hipMemcpyAsync(states, s->states[s->cur].ptr, total * s->model.state_dims * 4, kind, ctx->stream),
-                "read states");
-    if (density) NPA_HIP(ctx, hipMemcpyAsync(density, s->density.ptr, total * 4, kind, ctx->stream), "read density");
+    Segments g;
+    auto read = [&](float* dst, const DevBuf& src, uint64_t words) {
+        if (!dst) return hipSuccess;
+        if (!kernel_reachable(ctx, dst)) return hipMemcpyAsync(dst, src.ptr, words * 4, kind, ctx->stream);
+        g.add(dst, src.ptr, words);
+        return hipSuccess;
+    };
+    NPA_HIP(ctx, read(positions, s->pos[s->cur], total * 4), "read pos");
+    NPA_HIP(ctx, read(states, s->states[s->cur], total * S), "read states");
+    NPA_HIP(ctx, read(density, s->density, total), "read density");
+    NPA_HIP(ctx, launch_segments(g, ctx->stream), "read");
     return check_flags(ctx, s->ws);
 }
 
@@ -1210,16 +1368,9 @@ npa_status npa_state_update_model(npa_state* s, const npa_weights* w) {
     npa_status st = need_weights(ctx, w, F, H, O);
     if (st) return st;
     if (set_device(ctx)) return NPA_ERR_DEVICE;
-    const hipMemcpyKind kind = ctx->host_io ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    if ((uint64_t)H * F) NPA_HIP(ctx, hipMemcpyAsync(s->w1.ptr, w->w1, (uint64_t)H * F * 4, kind, ctx->stream), "w1");
-    if (H) NPA_HIP(ctx, hipMemcpyAsync(s->b1.ptr, w->b1, (uint64_t)H * 4, kind, ctx->stream), "b1");
-    if ((uint64_t)O * H) NPA_HIP(ctx, hipMemcpyAsync(s->w2.ptr, w->w2, (uint64_t)O * H * 4, kind, ctx->stream), "w2");
-    NPA_HIP(ctx, hipMemcpyAsync(s->b2.ptr, w->b2, (uint64_t)O * 4, kind, ctx->stream), "b2");
     npa::StepParams sp = make_params(s->grid, opts_for_model(m), s->B, s->N, m.state_dims);
     apply_model(&sp, m, s->grid.eps);
-    NPA_HIP(ctx, npa::launch_pad_weights(sp, s->w1.as<float>(), s->b1.as<float>(), s->w2.as<float>(),
-                                         s->b2.as<float>(), s->ws.wpad.as<float>(), ctx->stream),
-            "pad weights");
+    NPA_HIP(ctx, pad_state_weights(s, w, sp), "pad weights");
     if (ctx->host_io) NPA_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
     return NPA_OK;
 }
@@ -1232,6 +1383,7 @@ npa_status npa_state_step_index(const npa_state* s, uint64_t* step_index) {
 
 npa_status npa_state_buffers(npa_state* s, float** positions, float** states) {
     if (!s) return NPA_ERR_INVALID_ARGUMENT;
+    s->exposed = true;
     if (positions) *positions = s->pos[s->cur].as<float>();
     if (states) *states = s->states[s->cur].as<float>();
     return NPA_OK;

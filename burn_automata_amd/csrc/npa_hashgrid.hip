@@ -129,6 +129,7 @@ uint64_t Workspace::carve(const HashgridPlan& plan, uint64_t total, uint32_t bat
     });
     if (off > capacity || !base) return off;
     char* p = static_cast<char*>(base);
+    counters_kept = false;
     flags.view(p, kCarveFlagBytes);
     off = kCarveFlagBytes;
     each_buffer(*this, plan, total, batch, state_dims, dim, feature_dims, wpad_bytes, [&](DevBuf& b, uint64_t n) {
@@ -2352,7 +2353,7 @@ static hipError_t launch_bins(const HashgridPlan& plan, const GridParams& g, con
     unsigned long long* count = ws.bin_count.as<unsigned long long>();
     uint32_t* span = reinterpret_cast<uint32_t*>(count + C);
     hipError_t e;
-    if (!ws.bin_count.owned) {  // a carved workspace: its counters hold whatever the memory held
+    if (!ws.counters_kept) {  // a carved workspace: its counters hold whatever the memory held
         const uint32_t words = C + 4;  // the counters and the span words, as 64-bit words
         hipLaunchKernelGGL(k_clear_u64, dim3(std::min<uint32_t>((words + 255) / 256, 1024)), dim3(256), 0, stream,
                            count, words);

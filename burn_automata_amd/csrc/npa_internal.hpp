@@ -123,6 +123,9 @@ struct Workspace {
     // reset by the build's scan). bin_urow: per particle its target index within its bin (~0u for
     // a particle outside the mask).
     DevBuf bin_count, bin_urow;
+    // whether bin_count is zero between builds; a workspace carved from memory that others write in
+    // between clears it before each build instead
+    bool counters_kept = true;
     // Targets of the second pass and the update: particles whose update mask is not 0 (the others
     // are written to the output by the update-mask kernel). act_rows: compact row -> slot.
     // Counts (u32 words of wl_count, kWlWords): [0] density items, [1] compact rows (one 64-bit
