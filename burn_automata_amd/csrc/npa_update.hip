@@ -55,16 +55,18 @@ constexpr uint32_t kFuseHidden = 128;   // hidden units held per target (H <= 12
 constexpr uint32_t kFuseLdsBytes = 163840;
 
 // Per-variant shapes. FL: option flags fixed at compile time (bit 0 state gradient, bit 1 density
-// gradient, bit 2 moment correction, bit 3 periodic boundary; 5 = the rollout's usual set in a
-// clamped domain, 13 the same in a periodic one) or -1 (read from the params). The clamped variant
+// gradient, bit 2 moment correction, bit 3 periodic boundary; 5 = the state gradient with moment
+// correction in a clamped domain, 7 the same with the density gradient (every preset), 13 and 15 these
+// in a periodic domain) or -1 (read from the params). The clamped variant
 // carries none of the periodic wrap's loop invariants (the fmod's divisor scaling, the extents),
 // which keeps six more values out of scratch (C2 update 89 -> 87 us, 57 -> 47 MB per launch).
 template <int D, int FL>
 struct FuseShape {
     static constexpr int NMOM = D * (D + 1) / 2;            // moment matrix, upper triangle
-    static constexpr bool COMMON = FL >= 0 && (FL & 7) == 5;
-    static constexpr int SREC = COMMON ? 4 : 8;           // floats staged per entry
-    static constexpr int NX = COMMON ? NMOM : NMOM + D;   // per-target sums over entries
+    static constexpr bool COMMON = FL >= 0 && (FL & 5) == 5;
+    static constexpr bool DG = FL < 0 || (FL & 2) != 0;
+    static constexpr int SREC = COMMON ? 4 : 8;         // floats staged per entry
+    static constexpr int NX = DG ? NMOM + D : NMOM;     // per-target sums over entries
     static constexpr int CAP = D == 2 ? (COMMON ? 256 : 160) : (COMMON ? 128 : 64);  // list entries
     static constexpr int OPAD = (D + 16 + 3) / 4 * 4;      // padded update outputs
     // Per wave, one block per target group g, one after the other: its list [CAP] u32, its entry
@@ -215,10 +217,30 @@ __device__ __forceinline__ uint32_t row_last(uint32_t v) {
 //   t0 = w[E] * x, t1 = vg0[E] * diff, t2 = vg1[E] * diff (, t3 = vg2[E] * diff).
 // A DPP source must not have been written by the previous two VALU instructions (five after an
 // EXEC write): the s_nop provides those wait states, since the compiler does not see inside asm.
-template <int E, int D>
-__device__ __forceinline__ void bcast_products(float w, float g0, float g1, float g2, float x, float diff, float& t0,
-                                               float& t1, float& t2, float& t3) {
-    if constexpr (D == 2) {
+// With the density gradient the blur's term is two products, t0 = (w[E] * x) * vol[E].
+template <int E, int D, bool DG>
+__device__ __forceinline__ void bcast_products(float w, float vol, float g0, float g1, float g2, float x, float diff,
+                                               float& t0, float& t1, float& t2, float& t3) {
+    if constexpr (D == 2 && DG) {
+        asm volatile("s_nop %c9\n\t"
+                     "v_mul_f32_dpp %0, %3, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %1, %5, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %2, %6, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %0, %4, %0 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
+                     : "=&v"(t0), "=&v"(t1), "=&v"(t2)
+                     : "v"(w), "v"(vol), "v"(g0), "v"(g1), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
+        t3 = 0.0f;
+        (void)g2;
+    } else if constexpr (DG) {
+        asm volatile("s_nop %c11\n\t"
+                     "v_mul_f32_dpp %0, %4, %9 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %1, %6, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %2, %7, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %3, %8, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %0, %5, %0 row_newbcast:%c12 row_mask:0xf bank_mask:0xf"
+                     : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+                     : "v"(w), "v"(vol), "v"(g0), "v"(g1), "v"(g2), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
+    } else if constexpr (D == 2) {
         asm volatile("s_nop %c8\n\t"
                      "v_mul_f32_dpp %0, %3, %6 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n\t"
                      "v_mul_f32_dpp %1, %4, %7 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n\t"
@@ -487,8 +509,9 @@ __global__ __launch_bounds__(1024) void k_update_fused(StepParams P, const float
                             const float x = sv[e];
                             const float diff = x - si;
                             float t0, t1, t2, t3;
-                            bcast_products<e, D>(w, vg[0], vg[1], vg[2], x, diff, t0, t1, t2, t3);
-                            blur += t0;  // blur_state forward.rs:174-180 (x * w)
+                            bcast_products<e, D, Sh::DG>(Sh::DG ? smooth : w, vol, vg[0], vg[1], vg[2], x, diff, t0, t1,
+                                                         t2, t3);
+                            blur += t0;  // blur_state forward.rs:174-180 (x * w), second_pass_particle 263-270
                             gr[0] += t1;  // compute_state_gradient forward.rs:297-333 (diff * grad)
                             gr[1] += t2;
                             if constexpr (D == 3) gr[2] += t3;
@@ -995,31 +1018,35 @@ static hipError_t launch_fused_t(const StepParams& p, Workspace& ws, const StepI
 template <int D>
 static hipError_t launch_fused_d(const StepParams& p, Workspace& ws, const StepIO& io, const float* wfused,
                                  hipStream_t stream, Profiler* prof) {
-    // the usual option set (flags 5), clamped or periodic (flag 8), or every option read at run time
-    const bool common = p.state_grad && p.hybrid && !p.density_grad;
-    const bool per = p.g.boundary == 0;
+    // the state gradient with moment correction, with or without the density gradient, clamped or
+    // periodic (flags 5, 7, 13, 15: the presets and the usual rollouts), or every option read at run
+    // time. The run-time variant stages each round's scalars in LDS and spills; with the density
+    // gradient it took a step of 16,384 growing-2D particles 110 us against 87 us, and one of 1,000
+    // particles, in sixteen-wave blocks, 43 us against 33 us in four-wave ones.
+    const bool common = p.state_grad && p.hybrid;
+    const int fl = common ? 5 + (p.density_grad ? 2 : 0) + (p.g.boundary == 0 ? 8 : 0) : -1;
     constexpr int W = kFuseWaves;
+    auto launch = [&](auto engine, auto waves) {
+        constexpr int E = decltype(engine)::value, NW = decltype(waves)::value;
+        switch (fl) {
+            case 5: return launch_fused_t<D, 5, E, NW>(p, ws, io, wfused, stream, prof);
+            case 7: return launch_fused_t<D, 7, E, NW>(p, ws, io, wfused, stream, prof);
+            case 13: return launch_fused_t<D, 13, E, NW>(p, ws, io, wfused, stream, prof);
+            case 15: return launch_fused_t<D, 15, E, NW>(p, ws, io, wfused, stream, prof);
+            default: return launch_fused_t<D, -1, E, NW>(p, ws, io, wfused, stream, prof);
+        }
+    };
     if constexpr (D == 2) {  // the bf16 engine (2D; its bf16 feature parts must fit the wave's region)
-        constexpr uint32_t room = (uint32_t)std::min(FuseShape<2, 5>::WAVE_FLOATS, FuseShape<2, 13>::WAVE_FLOATS);
-        if (p.mlp_engine == NPA_MLP_MFMA_BF16 && 10 * p.FP + 4 * (16 + FuseShape<2, 5>::HSTR) <= room &&
-            10 * p.FP + 4 * (16 + FuseShape<2, -1>::HSTR) <= (uint32_t)FuseShape<2, -1>::WAVE_FLOATS)
-            return !common ? launch_fused_t<D, -1, 2, W>(p, ws, io, wfused, stream, prof)
-                   : per   ? launch_fused_t<D, 13, 2, W>(p, ws, io, wfused, stream, prof)
-                           : launch_fused_t<D, 5, 2, W>(p, ws, io, wfused, stream, prof);
+        constexpr uint32_t room = (uint32_t)std::min(FuseShape<2, 5>::WAVE_FLOATS, FuseShape<2, -1>::WAVE_FLOATS);
+        if (p.mlp_engine == NPA_MLP_MFMA_BF16 && 10 * p.FP + 4 * (16 + FuseShape<2, 5>::HSTR) <= room)
+            return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, W>{});
     }
-    if (p.mlp_engine != NPA_MLP_VALU)
-        return !common ? launch_fused_t<D, -1, 1, W>(p, ws, io, wfused, stream, prof)
-               : per   ? launch_fused_t<D, 13, 1, W>(p, ws, io, wfused, stream, prof)
-                       : launch_fused_t<D, 5, 1, W>(p, ws, io, wfused, stream, prof);
+    if (p.mlp_engine != NPA_MLP_VALU) return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, W>{});
     // a system with at most four items per CU (C1: 4,096 particles): blocks of four waves, so that
     // its items spread over every CU instead of queueing on a few
-    const bool small = ((uint64_t)p.T + 3) / 4 <= 4ull * (uint64_t)device_cu_count();
-    if (common && small)
-        return per ? launch_fused_t<D, 13, 0, 4>(p, ws, io, wfused, stream, prof)
-                   : launch_fused_t<D, 5, 0, 4>(p, ws, io, wfused, stream, prof);
-    return !common ? launch_fused_t<D, -1, 0, W>(p, ws, io, wfused, stream, prof)
-           : per   ? launch_fused_t<D, 13, 0, W>(p, ws, io, wfused, stream, prof)
-                   : launch_fused_t<D, 5, 0, W>(p, ws, io, wfused, stream, prof);
+    if (((uint64_t)p.T + 3) / 4 <= 4ull * (uint64_t)device_cu_count())
+        return launch(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+    return launch(std::integral_constant<int, 0>{}, std::integral_constant<int, W>{});
 }
 
 #if NPA_PART_DIM2
