@@ -16,6 +16,7 @@
 //                  weights in list order - the order the reference's serial loop adds them.
 #include <hip/hip_runtime.h>
 
+#include "npa_draw.hpp"
 #include "npa_internal.hpp"
 
 namespace npa {
@@ -329,6 +330,43 @@ __global__ __launch_bounds__(256) void k_splat_prep(SplatParams P, const float4*
     ntiles[n] = any ? (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1)) : 0u;
 }
 
+// The items of the matrix-core drawing (npa_draw.hip), one thread per particle: the same centre, window and
+// normaliser, its weight sum as the product of the two axes' sums (2 (2 r + 1) exponentials, not their
+// square).
+__global__ __launch_bounds__(256) void k_splat_items(SplatParams P, const float4* __restrict__ pos,
+                                                     const float* __restrict__ colors,
+                                                     const float* __restrict__ states, uint32_t count,
+                                                     DrawItem* __restrict__ out, uint32_t* __restrict__ rects) {
+    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= count) return;
+    const float4 p = pos[n];
+    const float fsz = (float)P.size;
+    const float px = (p.x - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
+    float py = (p.y - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
+    if (P.y_up) py = (fsz - 1.0f) - py;
+    const int64_t bx = f32_to_isize(floorf(px)), by = f32_to_isize(floorf(py));
+    const Footprint f = draw_footprint(px, py, P.k2, bx, by, P.radius, P.size);
+    DrawItem d;
+    d.px = px;
+    d.py = py;
+    d.k2 = P.k2;
+    d.scale = P.norm_scale / (P.normalize ? fmaxf(f.weights, 1e-8f) : 1.0f);
+    if (colors) {
+        for (int k = 0; k < 3; ++k) d.c[k] = colors[3 * (uint64_t)n + k];
+    } else {  // infer_2d.rs:20-31
+        const float* s = states + (uint64_t)n * P.S + (P.S - 3);
+        for (int k = 0; k < 3; ++k) d.c[k] = clampf_(s[k] + 0.5f, 0.0f, 1.0f);
+    }
+    d.depth = 0.0f;
+    const bool any = f.rect != kDrawNone;
+    d.x0 = any ? (int)(bx - P.radius) : 0;
+    d.y0 = any ? (int)(by - P.radius) : 0;
+    d.span = 2u * (uint32_t)P.radius;
+    d.special = draw_finite(d) ? 0u : 1u;
+    out[n] = d;
+    rects[n] = f.rect;
+}
+
 __global__ __launch_bounds__(1024) void k_scan_1block(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                       uint32_t count, uint32_t* __restrict__ total_out) {
     __shared__ uint32_t lds[32];
@@ -546,11 +584,24 @@ hipError_t launch_splat_2d(const float4* pos, const float* colors, const float* 
     const uint64_t cap64 = (uint64_t)count * max_per;
     if (cap64 >= (1ull << 31)) return hipErrorInvalidValue;
     const uint32_t cap = (uint32_t)cap64;
-    HashgridPlan plan;
-    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
     hipError_t e;
 #define NPA_RES(buf, n) \
     if ((e = (buf).reserve((size_t)(n))) != hipSuccess) return e;
+    DrawPlan draw;
+    if (make_draw_plan(P.size, windows, per_window, count, 4, win_cols, &draw)) {
+        NPA_RES(ws.params, (uint64_t)(count ? count : 1) * sizeof(DrawItem));
+        NPA_RES(ws.keys, (uint64_t)(count ? count : 1) * 4);
+        NPA_RES(ws.partials, draw.partial_floats * 4);
+        ProfScope ps(prof, NPA_KERNEL_SPLAT, stream);
+        if (count) {
+            hipLaunchKernelGGL(k_splat_items, dim3((count + 255) / 256), dim3(256), 0, stream, P, pos, colors, states, count,
+                               ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), image, stream);
+    }
+    HashgridPlan plan;
+    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
     NPA_RES(ws.params, (uint64_t)(count ? count : 1) * sizeof(SplatParticle));
     NPA_RES(ws.item_start, (uint64_t)(count ? count : 1) * 8);
     NPA_RES(ws.keys, (uint64_t)(cap ? cap : 1) * 4);
@@ -713,6 +764,42 @@ __global__ __launch_bounds__(256) void k_render_prep(RenderParams P, const float
     rp.pad = 0.0f;
     out[i] = rp;
     ntiles[i] = any ? (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1)) : 0u;
+}
+
+// The items of the matrix-core drawing (npa_draw.hip): one thread per particle-view.
+__global__ __launch_bounds__(256) void k_render_items(RenderParams P, const float4* __restrict__ pos,
+                                                      const float* __restrict__ colors,
+                                                      const float* __restrict__ opacities,
+                                                      const float* __restrict__ sigmas, DrawItem* __restrict__ out,
+                                                      uint32_t* __restrict__ rects) {
+    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= P.count) return;
+    const uint32_t v = blockIdx.y;
+    const float* B = P.basis[v];
+    const float4 p = pos[n];
+    const float x = p.x * B[0] + p.y * B[1] + p.z * B[2];
+    const float y = p.x * B[3] + p.y * B[4] + p.z * B[5];
+    const float f = p.x * B[6] + p.y * B[7] + p.z * B[8];
+    const float sigma = fmaxf(clampf_(sigmas[n], P.min_sigma, P.max_sigma), kRenderEps);
+    const int64_t radius = f32_to_isize(fmaxf(ceilf(5.0f * sigma), 1.0f));
+    const float fsz1 = (float)P.size - 1.0f;
+    DrawItem d;
+    d.px = (x + P.ws) / (2.0f * P.ws) * fsz1;
+    d.py = (P.ws - y) / (2.0f * P.ws) * fsz1;
+    d.k2 = kLog2e / (2.0f * (sigma * sigma));
+    const int64_t bx = f32_to_isize(floorf(d.px)), by = f32_to_isize(floorf(d.py));
+    const Footprint fp = draw_footprint(d.px, d.py, d.k2, bx, by, radius, P.size);
+    d.scale = P.norm_scale * clampf_(opacities[n], 0.0f, 1.0f) / fmaxf(fp.weights, kRenderEps);  // image.rs:67-69
+    for (int k = 0; k < 3; ++k) d.c[k] = colors[3 * (uint64_t)n + k];
+    d.depth = clampf_(0.5f + 0.5f * f / fmaxf(P.ws, kRenderEps), 0.0f, 1.0f);
+    const bool any = fp.rect != kDrawNone;
+    d.x0 = any ? (int)(bx - radius) : 0;
+    d.y0 = any ? (int)(by - radius) : 0;
+    d.span = 2u * (uint32_t)radius;
+    d.special = draw_finite(d) ? 0u : 1u;
+    const uint64_t i = (uint64_t)v * P.count + n;
+    out[i] = d;
+    rects[i] = fp.rect;
 }
 
 __global__ __launch_bounds__(256) void k_render_emit(RenderParams P, const RenderParticle* __restrict__ rp,
@@ -924,11 +1011,24 @@ hipError_t launch_render_views(const float4* pos, const float* colors, const flo
     const uint64_t cap64 = items64 * max_per;
     if (cap64 >= (1ull << 31)) return hipErrorInvalidValue;
     const uint32_t cap = (uint32_t)cap64;
-    HashgridPlan plan;
-    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
     hipError_t e;
 #define NPA_RES(buf, n) \
     if ((e = (buf).reserve((size_t)(n))) != hipSuccess) return e;
+    DrawPlan draw;
+    if (make_draw_plan(P.size, nviews, count, items, 5, nviews, &draw)) {
+        NPA_RES(ws.params, (uint64_t)(items ? items : 1) * sizeof(DrawItem));
+        NPA_RES(ws.keys, (uint64_t)(items ? items : 1) * 4);
+        NPA_RES(ws.partials, draw.partial_floats * 4);
+        ProfScope ps(prof, NPA_KERNEL_RENDER, stream);
+        if (count) {
+            hipLaunchKernelGGL(k_render_items, dim3((count + 255) / 256, nviews), dim3(256), 0, stream, P, pos, colors,
+                               opacities, sigmas, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), images, stream);
+    }
+    HashgridPlan plan;
+    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
     NPA_RES(ws.params, (uint64_t)(items ? items : 1) * sizeof(RenderParticle));
     NPA_RES(ws.item_start, (uint64_t)(items ? items : 1) * 8);
     NPA_RES(ws.keys, (uint64_t)(cap ? cap : 1) * 4);

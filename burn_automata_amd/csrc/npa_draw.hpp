@@ -1,0 +1,69 @@
+// npa_draw.hpp - isotropic Gaussian footprints drawn as a contraction on the matrix cores (npa_draw.hip).
+#pragma once
+
+#include "npa_internal.hpp"
+
+namespace npa {
+
+// What one item (a particle, or a particle seen through one view) adds to pixel (x, y) of its window,
+// for x0 <= x <= x0 + span and y0 <= y <= y0 + span: scale * 2^(-k2 ((x - px)^2 + (y - py)^2)) times
+// its channels (c, then 1, then depth).
+struct alignas(16) DrawItem {  // 48 bytes
+    float px, py, k2, scale;
+    float c[3], depth;
+    int x0, y0;
+    uint32_t span;
+    uint32_t special;  // a value is not finite: drawn pixel by pixel
+};
+
+// The window's 16x16 tiles an item touches, tx0 | tx1 << 8 | ty0 << 16 | ty1 << 24 (at most 256 tiles
+// per axis: image sizes up to 4096); kDrawNone touches none.
+constexpr uint32_t kDrawNone = 0x00ff00ffu;
+
+struct DrawPlan {
+    int size, tiles_x;
+    uint32_t windows, per_window, count;  // window w holds items [w * per_window, + per_window), up to count
+    uint32_t channels;                    // 4 (r, g, b, weight) or 5 (and depth)
+    uint32_t group, groups_x, splits;     // tiles per block and axis, blocks per window and axis, item ranges
+    uint32_t win_cols;                    // 4 channels: windows per image row
+    int stride;                           // 4 channels: pixels per image row
+    uint64_t partial_floats;              // of the splits' partial images (0 without splits)
+};
+
+// Lays out a drawing; false when sorting the items by tile is the faster way (see npa_draw.hip).
+bool make_draw_plan(int size, uint32_t windows, uint32_t per_window, uint32_t count, uint32_t channels, uint32_t win_cols,
+                    DrawPlan* plan);
+// image: 4 channels [rows of windows * size][win_cols * size][4], 5 channels [windows][size][size][5].
+hipError_t launch_draw(const DrawPlan& plan, const DrawItem* items, const uint32_t* rects, float* partials, float* image,
+                       hipStream_t stream);
+
+// An item's weight sum over the in-image part of its footprint, as the product of its two axes' sums, and its
+// tiles. (bx, by): the pixel of its centre.
+struct Footprint {
+    uint32_t rect;
+    float weights;
+};
+__device__ __forceinline__ float axis_weights(float p, float k2, int lo, int hi) {
+    float s = 0.0f;
+    for (int v = lo; v <= hi; ++v) {
+        const float d = (float)v - p;
+        s += __builtin_amdgcn_exp2f(-(d * d) * k2);
+    }
+    return s;
+}
+__device__ __forceinline__ Footprint draw_footprint(float px, float py, float k2, int64_t bx, int64_t by, int64_t r, int size) {
+    int64_t x0 = bx - r, x1 = bx + r, y0 = by - r, y1 = by + r;
+    if (x0 < 0) x0 = 0;
+    if (y0 < 0) y0 = 0;
+    if (x1 > size - 1) x1 = size - 1;
+    if (y1 > size - 1) y1 = size - 1;
+    if (x0 > x1 || y0 > y1) return {kDrawNone, 0.0f};
+    const uint32_t rect = (uint32_t)(x0 / 16) | (uint32_t)(x1 / 16) << 8 | (uint32_t)(y0 / 16) << 16 | (uint32_t)(y1 / 16) << 24;
+    return {rect, axis_weights(px, k2, (int)x0, (int)x1) * axis_weights(py, k2, (int)y0, (int)y1)};
+}
+__device__ __forceinline__ bool draw_finite(const DrawItem& d) {
+    return isfinite(d.px) && isfinite(d.py) && isfinite(d.k2) && isfinite(d.scale) && isfinite(d.c[0]) && isfinite(d.c[1]) &&
+           isfinite(d.c[2]) && isfinite(d.depth);
+}
+
+}  // namespace npa

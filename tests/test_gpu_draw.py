@@ -1,0 +1,84 @@
+"""The splat and the projected render drawn on the matrix cores, at the edges of their tiles, groups, batches
+of 8,192 items and item ranges, against the oracle; non-finite particles touch only their own footprint."""
+import numpy as np
+import pytest
+
+from burn_automata_amd import kernels as K
+from burn_automata_amd.config import RenderLossConfig, Splat2dConfig
+from oracle import oracle as O
+from tests.helpers import psnr, to_np
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+# The weights' exponent is evaluated by axis and the sums by matrix products: both sides round pixel
+# coordinates (up to 2^-24 of the image size, times the weight's slope) and sums of a few hundred terms.
+TOL = 1e-5
+
+
+def _err(got, want):
+    g, w = to_np(got).astype(np.float64), to_np(want).astype(np.float64).reshape(to_np(got).shape)
+    return np.max(np.abs(g - w)) / max(np.max(np.abs(w)), 1e-30)
+
+
+def _particles(n, seed, spread=1.0):
+    rng = np.random.default_rng(seed)
+    pos = np.zeros((n, 4), f32)
+    pos[:, :3] = rng.uniform(-spread, spread, (n, 3))
+    return pos, rng.random((n, 3)).astype(f32), rng.random(n).astype(f32), rng.uniform(0.5, 4.0, n).astype(f32)
+
+
+@pytest.mark.parametrize("n,size,sigma,spread", [
+    (1, 1, 0.4, 0.5), (3, 16, 1.0, 1.2), (500, 17, 2.0, 1.0), (8192, 64, 1.0, 1.0), (8193, 65, 0.7, 1.3), (20000, 300, 1.5, 1.0),
+    (3000, 500, 0.05, 1.0), (900, 128, 9.0, 1.0), (4000, 1040, 2.0, 1.0), (9000, 40, 1.0, 0.02), (0, 33, 1.0, 1.0)])
+def test_splat_matches_the_oracle(ctx, n, size, sigma, spread):
+    pos, col, _, _ = _particles(n, size, spread)
+    cfg = Splat2dConfig(image_size=size, sigma=sigma, pixel_size=2.0 / size)
+    got = K.splat_particles_2d(pos, col, cfg, ctx=ctx)
+    if n == 0:
+        assert not to_np(got).any()
+        return
+    want = O.splat_particles_2d(pos, col, cfg)
+    assert _err(got, want) <= TOL and psnr(got, to_np(want).reshape(to_np(got).shape)) >= 100
+    np.testing.assert_array_equal(to_np(K.splat_particles_2d(pos, col, cfg, ctx=ctx)), to_np(got))
+
+
+@pytest.mark.parametrize("batch,n,size,cols", [(5, 700, 48, 2), (64, 130, 128, 8), (7, 9000, 33, 3)])
+def test_tiled_windows_match_single_ones(ctx, batch, n, size, cols):
+    pos, col, _, _ = _particles(batch * n, batch)
+    cfg = Splat2dConfig(image_size=size, sigma=1.2, pixel_size=2.0 / size)
+    got = to_np(K.splat_particles_2d_tiled(pos, col, batch, n, cfg, cols, ctx=ctx))
+    for b in range(batch):
+        want = to_np(O.splat_particles_2d(pos[b * n:(b + 1) * n], col[b * n:(b + 1) * n], cfg)).reshape(size, size, 4)
+        win = got[b // cols * size:(b // cols + 1) * size, b % cols * size:(b % cols + 1) * size]
+        assert _err(win, want) <= TOL
+
+
+@pytest.mark.parametrize("n,size,views", [(1, 5, (0,)), (1500, 64, (0, 1, 2, 3)), (9000, 65, (3,)), (2500, 200, (1, 2)),
+                                          (700, 530, (0, 3))])
+def test_render_matches_the_oracle(ctx, n, size, views):
+    pos, col, op, sg = _particles(n, n, 1.1)
+    cfg = RenderLossConfig(image_size=size)
+    got = to_np(K.render_views(pos, col, op, sg, cfg, views, ctx=ctx))
+    for k, v in enumerate(views):
+        want = O.splat_projected(O.project_positions(v, pos, cfg.world_scale), col, op, sg, cfg)
+        assert _err(got[k], want) <= TOL
+    np.testing.assert_array_equal(to_np(K.render_views(pos, col, op, sg, cfg, views, ctx=ctx)), got)
+
+
+def test_non_finite_values_stay_in_their_footprint(ctx):
+    """A NaN or infinite colour reaches the pixels of its particle's footprint and no others; a particle at
+    a NaN or infinite position is drawn as the oracle draws it."""
+    pos, col, _, _ = _particles(300, 4)
+    cfg = Splat2dConfig(image_size=96, sigma=0.8, pixel_size=2.0 / 96)
+    col[7, 1] = np.nan
+    col[100, 0] = np.inf
+    col[200, 2] = -np.inf
+    pos[30, 0] = np.nan
+    pos[31, 1] = np.inf
+    got = to_np(K.splat_particles_2d(pos, col, cfg, ctx=ctx))
+    want = to_np(O.splat_particles_2d(pos, col, cfg)).reshape(got.shape)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    assert np.max(np.abs(got[fin] - want[fin])) <= TOL * np.max(np.abs(want[fin]))
