@@ -1,20 +1,15 @@
-// npa_decode.hip - Gaussian decode and tile-binned 2D splat on gfx950.
+// npa_decode.hip - Gaussian decode, the splat's and the render's items and the oriented raster on gfx950.
 //
 // decode_gaussians_3d  crates/burn_automata_kernels/src/gaussian.rs:53-223: a per-particle map.
 //
-// splat_particles_2d   crates/burn_automata_kernels/src/splat.rs:30-93, as a deterministic
-// tile-binned rasteriser:
-//   k_splat_prep   per particle: pixel-space centre, the in-bounds window weight sum
-//                  (the normaliser), colour, and how many 16x16 screen tiles the
-//                  (2r+1)^2 window touches;
-//   k_scan_1block  exclusive prefix of the per-particle tile counts;
-//   k_splat_emit   one (tile, particle) item per touched tile, in particle order;
-//   stable key sort of the items by tile (the hashgrid's counting sort) -> per-tile
-//                  particle lists in ascending particle index;
-//   k_splat_tiles  one 256-thread block per tile, one pixel per thread: the tile's list
-//                  is staged through LDS 256 particles at a time and each pixel adds its
-//                  weights in list order - the order the reference's serial loop adds them.
+// splat_particles_2d   crates/burn_automata_kernels/src/splat.rs:30-93, and the render loss's
+// project_positions + splat_projected: the particles' footprints are prepared here and drawn by
+// npa_draw.hip, deterministically.
+//
+// The oriented Gaussian raster: per-tile lists in depth order, composited front to back.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "npa_draw.hpp"
 #include "npa_internal.hpp"
@@ -208,131 +203,31 @@ hipError_t launch_write_gaussians(const float4* pos, const float* states, uint32
 // ----------------------------------------------------------------- splat
 constexpr int kTile = 16;
 
-// A Gaussian weight exp(-d2 / (2 sigma^2)) (splat.rs:71, image.rs:61) as 2^(-d2 * k2) with
+// A Gaussian weight exp(-d2 / (2 sigma^2)) (splat.rs:71, image.rs:61) is taken as 2^(-d2 * k2) with
 // k2 = log2(e) / (2 sigma^2) on the hardware exp2; it differs from expf of the IEEE quotient by a
 // few ulps at most.
 constexpr float kLog2e = 1.44269504088896340736f;
-__device__ __forceinline__ float splat_weight(float d2, float k2) { return __builtin_amdgcn_exp2f(-(d2 * k2)); }
+
+// The entry points' limits: 65,536 tiles in all, and fewer than 2^31 (item, tile) pairs at the widest
+// footprint.
+static bool draw_within_limits(int size, uint64_t windows, uint64_t items, int radius) {
+    const uint64_t tiles_x = (uint64_t)((size + kTile - 1) / kTile), tiles = tiles_x * tiles_x;
+    const uint64_t per_axis = (uint64_t)((2 * radius + 1 + kTile - 1) / kTile + 1);
+    return tiles * windows <= 65536 && items * std::min<uint64_t>(per_axis * per_axis, tiles) < (1ull << 31);
+}
 
 struct SplatParams {
     int size;
     int radius;
-    int tiles_x, tiles_y;
-    float sigma;      // pixel-space sigma after the normalize_color rescale
-    float two_sig2;   // 2 * sigma * sigma
-    float k2;         // log2(e) / two_sig2 (splat_weight)
+    float k2;
     float norm_scale;
     float lo, hi;
     int normalize, y_up;
     int S;
-    // Tiled layout: particle n belongs to window n / per_window; windows are laid out row-major,
-    // win_cols per row, each size x size pixels with tiles_x * tiles_y screen tiles; the image row
-    // stride is stride pixels. A single image is one window.
-    uint32_t per_window, win_cols, tiles_per_win;
-    int stride;
 };
 
-struct SplatParticle {  // 32 bytes
-    float fx, fy;
-    int bx, by;
-    float scale;  // norm_scale / the normaliser (1 without normalize_color)
-    float c[3];
-};
-
-__device__ __forceinline__ bool splat_tiles(const SplatParams& P, int64_t bx, int64_t by, int* tx0, int* tx1,
-                                            int* ty0, int* ty1) {
-    int64_t x0 = bx - P.radius, x1 = bx + P.radius, y0 = by - P.radius, y1 = by + P.radius;
-    if (x0 < 0) x0 = 0;
-    if (y0 < 0) y0 = 0;
-    if (x1 > P.size - 1) x1 = P.size - 1;
-    if (y1 > P.size - 1) y1 = P.size - 1;
-    if (x0 > x1 || y0 > y1) return false;
-    *tx0 = (int)(x0 / kTile);
-    *tx1 = (int)(x1 / kTile);
-    *ty0 = (int)(y0 / kTile);
-    *ty1 = (int)(y1 / kTile);
-    return true;
-}
-
-// Value of lane J of each group of four consecutive lanes (DPP quad_perm; every lane reads a valid
-// lane, so bound_ctrl never applies and the compiler folds the move into the consuming add).
-template <int J>
-__device__ __forceinline__ float quad_bcast(float v) {
-    constexpr int c = J | (J << 2) | (J << 4) | (J << 6);
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), c, 0xf, 0xf, true));
-}
-
-// Four lanes per particle: every lane derives the particle's pixel-space centre; lane q computes the
-// window weights of offsets q, q + 4, ... (row-major over (oy, ox), the reference's order), and
-// every lane adds each round's four weights in offset order, so the sum is the serial sum of the
-// reference (an out-of-image offset adds +0.0, which leaves the non-negative sum unchanged).
-__global__ __launch_bounds__(256) void k_splat_prep(SplatParams P, const float4* __restrict__ pos,
-                                                    const float* __restrict__ colors,
-                                                    const float* __restrict__ states, uint32_t count,
-                                                    SplatParticle* __restrict__ out,
-                                                    uint32_t* __restrict__ ntiles) {
-    const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t q = gt & 3u;
-    const uint32_t n = gt >> 2;
-    const bool valid = n < count;
-    const float4 p = pos[valid ? n : 0u];
-    const float fsz = (float)P.size;
-    const float px = (p.x - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
-    float py = (p.y - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
-    if (P.y_up) py = (fsz - 1.0f) - py;
-    const int64_t bx = f32_to_isize(floorf(px)), by = f32_to_isize(floorf(py));
-    const float fx = px - (float)bx, fy = py - (float)by;
-    int tx0, tx1, ty0, ty1;
-    const bool any = valid && splat_tiles(P, bx, by, &tx0, &tx1, &ty0, &ty1);
-    float weight_sum = 0.0f;
-    if (__ballot(any)) {
-        const int side = 2 * P.radius + 1;
-        const uint32_t terms = (uint32_t)side * (uint32_t)side;
-        int oy = -P.radius, ox = -P.radius + (int)q;  // offset q of the row-major window
-        while (ox > P.radius) {
-            ox -= side;
-            ++oy;
-        }
-        for (uint32_t k0 = 0; k0 < terms; k0 += 4) {
-            float wk = 0.0f;
-            const int64_t x = bx + ox, y = by + oy;
-            if (any && k0 + q < terms && x >= 0 && y >= 0 && x < P.size && y < P.size) {
-                const float dx = (float)ox - fx, dy = (float)oy - fy;
-                wk = splat_weight(dx * dx + dy * dy, P.k2);
-            }
-            weight_sum += quad_bcast<0>(wk);
-            weight_sum += quad_bcast<1>(wk);
-            weight_sum += quad_bcast<2>(wk);
-            weight_sum += quad_bcast<3>(wk);
-            ox += 4;  // the offset four places on
-            while (ox > P.radius) {
-                ox -= side;
-                ++oy;
-            }
-        }
-    }
-    if (!valid || q != 0) return;
-    SplatParticle sp;
-    sp.fx = fx;
-    sp.fy = fy;
-    sp.bx = any ? (int)bx : 0;
-    sp.by = any ? (int)by : 0;
-    sp.scale = P.norm_scale / (P.normalize ? fmaxf(weight_sum, 1e-8f) : 1.0f);
-    if (colors) {
-        sp.c[0] = colors[3 * (uint64_t)n];
-        sp.c[1] = colors[3 * (uint64_t)n + 1];
-        sp.c[2] = colors[3 * (uint64_t)n + 2];
-    } else {  // infer_2d.rs:20-31
-        const float* s = states + (uint64_t)n * P.S + (P.S - 3);
-        for (int k = 0; k < 3; ++k) sp.c[k] = clampf_(s[k] + 0.5f, 0.0f, 1.0f);
-    }
-    out[n] = sp;
-    ntiles[n] = any ? (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1)) : 0u;
-}
-
-// The items of the matrix-core drawing (npa_draw.hip), one thread per particle: the same centre, window and
-// normaliser, its weight sum as the product of the two axes' sums (2 (2 r + 1) exponentials, not their
-// square).
+// One thread per particle: its pixel-space centre, window, normaliser and colour; the window's weight sum is
+// the product of the two axes' sums (2 (2 r + 1) exponentials, not their square).
 __global__ __launch_bounds__(256) void k_splat_items(SplatParams P, const float4* __restrict__ pos,
                                                      const float* __restrict__ colors,
                                                      const float* __restrict__ states, uint32_t count,
@@ -481,63 +376,9 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
     }
 }
 
-__global__ __launch_bounds__(256) void k_splat_emit(SplatParams P, const SplatParticle* __restrict__ sp,
-                                                    const uint32_t* __restrict__ ntiles,
-                                                    const uint32_t* __restrict__ start, uint32_t count,
-                                                    uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= count || ntiles[n] == 0) return;
-    int tx0, tx1, ty0, ty1;
-    splat_tiles(P, sp[n].bx, sp[n].by, &tx0, &tx1, &ty0, &ty1);
-    uint32_t k = start[n];
-    const uint32_t win_base = (n / P.per_window) * P.tiles_per_win;
-    for (int ty = ty0; ty <= ty1; ++ty)
-        for (int tx = tx0; tx <= tx1; ++tx) {
-            keys[k] = win_base + (uint32_t)(ty * P.tiles_x + tx);
-            vals[k] = n;
-            ++k;
-        }
-}
-
-__global__ __launch_bounds__(256) void k_splat_tiles(SplatParams P, const SplatParticle* __restrict__ sp,
-                                                     const uint32_t* __restrict__ offsets,
-                                                     const uint32_t* __restrict__ sorted, float* __restrict__ image) {
-    __shared__ SplatParticle buf[256];
-    const uint32_t t = blockIdx.x;
-    const uint32_t win = t / P.tiles_per_win, lt = t - win * P.tiles_per_win;
-    const int tx = (int)(lt % P.tiles_x), ty = (int)(lt / P.tiles_x);
-    const int x = tx * kTile + (int)(threadIdx.x % kTile);
-    const int y = ty * kTile + (int)(threadIdx.x / kTile);
-    const uint32_t beg = offsets[t], end = offsets[t + 1];
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t base = beg; base < end; base += 256) {
-        const uint32_t k = base + threadIdx.x;
-        if (k < end) buf[threadIdx.x] = sp[sorted[k]];
-        __syncthreads();
-        const uint32_t m = end - base < 256 ? end - base : 256;
-        for (uint32_t q = 0; q < m; ++q) {
-            const SplatParticle& p = buf[q];
-            const int ox = x - p.bx, oy = y - p.by;
-            if (ox < -P.radius || ox > P.radius || oy < -P.radius || oy > P.radius) continue;
-            const float dx = (float)ox - p.fx, dy = (float)oy - p.fy;
-            const float w = splat_weight(dx * dx + dy * dy, P.k2) * p.scale;
-            acc[0] += p.c[0] * w;
-            acc[1] += p.c[1] * w;
-            acc[2] += p.c[2] * w;
-            acc[3] += w;
-        }
-        __syncthreads();
-    }
-    if (x < P.size && y < P.size) {
-        const uint64_t row = (uint64_t)(win / P.win_cols) * P.size + y;
-        const uint64_t col = (uint64_t)(win % P.win_cols) * P.size + x;
-        reinterpret_cast<float4*>(image)[row * P.stride + col] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    }
-}
-
 void SplatWorkspace::release() {
     for (DevBuf* b : {&params, &item_start, &keys, &vals, &sorted, &ranks, &table, &totals, &offsets, &count, &flags, &scan,
-                      &attrs, &partials, &chunks, &order, &decoded, &sort_temp})
+                      &attrs, &partials, &order, &decoded, &sort_temp})
         b->release();
 }
 
@@ -554,9 +395,7 @@ hipError_t launch_splat_2d(const float4* pos, const float* colors, const float* 
     if (!(rf >= 1.0f)) rf = rf != rf ? 1.0f : 1.0f;
     if (rf > 4096.0f) rf = 4096.0f;  // windows wider than any supported image are clipped anyway
     P.radius = (int)rf;
-    P.sigma = sigma;
-    P.two_sig2 = 2.0f * sigma * sigma;
-    P.k2 = kLog2e / P.two_sig2;
+    P.k2 = kLog2e / (2.0f * sigma * sigma);
     P.norm_scale = 1.0f;
     if (cfg.normalize_color) {
         const float t = fsz * cfg.pixel_size / (cfg.hi - cfg.lo);
@@ -567,206 +406,39 @@ hipError_t launch_splat_2d(const float4* pos, const float* colors, const float* 
     P.normalize = cfg.normalize_color ? 1 : 0;
     P.y_up = cfg.y_up ? 1 : 0;
     P.S = (int)S;
-    P.tiles_x = (P.size + kTile - 1) / kTile;
-    P.tiles_y = P.tiles_x;
     if (windows == 0 || win_cols == 0 || per_window == 0) return hipErrorInvalidValue;
     if ((uint64_t)per_window * windows < count) return hipErrorInvalidValue;
-    P.per_window = per_window;
-    P.win_cols = win_cols;
-    P.tiles_per_win = (uint32_t)(P.tiles_x * P.tiles_y);
-    P.stride = (int)(win_cols * (uint32_t)P.size);
-    const uint64_t ntile64 = (uint64_t)P.tiles_per_win * windows;
-    if (ntile64 > 65536) return hipErrorInvalidValue;  // the key sort's bin limit
-    const uint32_t ntile_total = (uint32_t)ntile64;
-    const uint32_t ntile_win = P.tiles_per_win;
-    const uint64_t per_axis = (uint64_t)((2 * P.radius + 1 + kTile - 1) / kTile + 1);
-    const uint64_t max_per = std::min<uint64_t>(per_axis * per_axis, ntile_win);
-    const uint64_t cap64 = (uint64_t)count * max_per;
-    if (cap64 >= (1ull << 31)) return hipErrorInvalidValue;
-    const uint32_t cap = (uint32_t)cap64;
+    if (!draw_within_limits(P.size, windows, count, P.radius)) return hipErrorInvalidValue;
     hipError_t e;
-#define NPA_RES(buf, n) \
-    if ((e = (buf).reserve((size_t)(n))) != hipSuccess) return e;
     DrawPlan draw;
-    if (make_draw_plan(P.size, windows, per_window, count, 4, win_cols, &draw)) {
-        NPA_RES(ws.params, (uint64_t)(count ? count : 1) * sizeof(DrawItem));
-        NPA_RES(ws.keys, (uint64_t)(count ? count : 1) * 4);
-        NPA_RES(ws.partials, draw.partial_floats * 4);
-        ProfScope ps(prof, NPA_KERNEL_SPLAT, stream);
-        if (count) {
-            hipLaunchKernelGGL(k_splat_items, dim3((count + 255) / 256), dim3(256), 0, stream, P, pos, colors, states, count,
-                               ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), image, stream);
-    }
-    HashgridPlan plan;
-    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
-    NPA_RES(ws.params, (uint64_t)(count ? count : 1) * sizeof(SplatParticle));
-    NPA_RES(ws.item_start, (uint64_t)(count ? count : 1) * 8);
-    NPA_RES(ws.keys, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.vals, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.sorted, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.ranks, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.table, plan.table_entries * 4);
-    NPA_RES(ws.totals, (uint64_t)ntile_total * 4);
-    NPA_RES(ws.offsets, ((uint64_t)ntile_total + 1) * 4);
-    NPA_RES(ws.count, 64);
-    NPA_RES(ws.scan, (2 * ((uint64_t)count / kScanBlock + 1) + 2) * 4);
-    NPA_RES(ws.flags, 64);
-#undef NPA_RES
+    if (!make_draw_plan(P.size, P.radius, windows, per_window, count, 4, win_cols, &draw)) return hipErrorInvalidValue;
+    if ((e = ws.params.reserve((uint64_t)(count ? count : 1) * sizeof(DrawItem))) != hipSuccess) return e;
+    if ((e = ws.keys.reserve((uint64_t)(count ? count : 1) * 4)) != hipSuccess) return e;
+    if ((e = ws.partials.reserve(draw.partial_floats * 4)) != hipSuccess) return e;
     ProfScope ps(prof, NPA_KERNEL_SPLAT, stream);
-    uint32_t* ntiles = ws.item_start.as<uint32_t>() + (count ? count : 1);
-    uint32_t* start = ws.item_start.as<uint32_t>();
     if (count) {
-        hipLaunchKernelGGL(k_splat_prep, dim3((uint32_t)(((uint64_t)count * 4 + 255) / 256)), dim3(256), 0, stream, P,
-                           pos, colors, states, count, ws.params.as<SplatParticle>(), ntiles);
+        hipLaunchKernelGGL(k_splat_items, dim3((count + 255) / 256), dim3(256), 0, stream, P, pos, colors, states, count,
+                           ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    {  // start = exclusive prefix of ntiles, total item count into ws.count
-        const uint32_t nb = (count + kScanBlock - 1) / kScanBlock;
-        uint32_t* sums = ws.scan.as<uint32_t>();
-        if (nb) {
-            hipLaunchKernelGGL(k_scan_partials, dim3(nb), dim3(256), 0, stream, ntiles, count, sums);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(k_scan_1block, dim3(1), dim3(1024), 0, stream, sums, sums + nb + 1, nb,
-                           ws.count.as<uint32_t>());
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (nb) {
-            hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, stream, ntiles, start, count, sums + nb + 1);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-    }
-    if (count) {
-        hipLaunchKernelGGL(k_splat_emit, dim3((count + 255) / 256), dim3(256), 0, stream, P,
-                           ws.params.as<SplatParticle>(), ntiles, start, count, ws.keys.as<uint32_t>(),
-                           ws.vals.as<uint32_t>());
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    e = launch_key_sort(plan, ws.keys.as<uint32_t>(), ws.vals.as<uint32_t>(), ws.count.as<uint32_t>(), cap,
-                        ws.ranks.as<uint32_t>(), ws.table.as<uint32_t>(), ws.totals.as<uint32_t>(),
-                        ws.offsets.as<uint32_t>(), ws.sorted.as<uint32_t>(), ws.flags.as<uint32_t>(), stream);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_splat_tiles, dim3(ntile_total), dim3(256), 0, stream, P, ws.params.as<SplatParticle>(),
-                       ws.offsets.as<uint32_t>(), ws.sorted.as<uint32_t>(), image);
-    return hipGetLastError();
+    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), image, stream);
 }
 
 // ------------------------------------------------------- projected 3D render
 // project_positions (render_loss/projection.rs:11-29) + splat_projected (render_loss/image.rs:18-79)
-// for up to kMaxRenderViews views in one pipeline: item i = v * count + n is particle n seen
-// through view v; its screen tiles get keys v * tiles_per_view + tile, so one stable key sort
-// bins every view, and one tile kernel draws them all. Within a tile the items keep ascending
-// n, so every pixel sums its particles in the reference's order.
+// for up to kMaxRenderViews views at once: item v * count + n is particle n seen through view v, drawn
+// into window v.
 constexpr float kRenderEps = 1.0e-8f;
 
 struct RenderParams {
-    int size, tiles_x;
-    uint32_t tiles_per_view, count;
+    int size;
+    uint32_t count;
     float ws, min_sigma, max_sigma, norm_scale;
     float basis[kMaxRenderViews][9];  // right, up, forward of each view
 };
 
-struct alignas(16) RenderParticle {  // 48 bytes
-    float px, py;     // projected pixel coordinates
-    int x0, y0;       // first column / row of the (2 radius + 1)^2 footprint (image.rs:41-53)
-    uint32_t span;    // 2 radius
-    float k2;         // log2(e) / (2 sigma^2)
-    float scale;      // norm_scale * clamp(opacity, 0, 1) / max(in-bounds weight sum, EPS)
-    float depth;
-    float c[3];
-    float pad;
-};
-
-
-__device__ __forceinline__ bool render_tiles(const RenderParams& P, int64_t bx, int64_t by, int64_t r, int* tx0,
-                                             int* tx1, int* ty0, int* ty1) {
-    int64_t x0 = bx - r, x1 = bx + r, y0 = by - r, y1 = by + r;
-    if (x0 < 0) x0 = 0;
-    if (y0 < 0) y0 = 0;
-    if (x1 > P.size - 1) x1 = P.size - 1;
-    if (y1 > P.size - 1) y1 = P.size - 1;
-    if (x0 > x1 || y0 > y1) return false;
-    *tx0 = (int)(x0 / kTile);
-    *tx1 = (int)(x1 / kTile);
-    *ty0 = (int)(y0 / kTile);
-    *ty1 = (int)(y1 / kTile);
-    return true;
-}
-
-// kPrepLanes lanes per particle-view; grid (ceil(count * kPrepLanes / 256), nviews): blockIdx.y is
-// the view, so its basis is a uniform load. The lanes split the in-bounds footprint by rows (lane
-// l sums rows l, l + kPrepLanes, ... left to right) and combine their sums in a fixed butterfly,
-// so the weight sum is deterministic; it differs from the reference's single running sum only
-// by rounding.
-constexpr uint32_t kPrepLanes = 16;
-
-__global__ __launch_bounds__(256) void k_render_prep(RenderParams P, const float4* __restrict__ pos,
-                                                     const float* __restrict__ colors,
-                                                     const float* __restrict__ opacities,
-                                                     const float* __restrict__ sigmas,
-                                                     RenderParticle* __restrict__ out,
-                                                     uint32_t* __restrict__ ntiles) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = g / kPrepLanes, lane = g % kPrepLanes;
-    const bool live = n < P.count;  // the whole group agrees: count * kPrepLanes threads are live
-    const uint32_t nn = live ? n : 0;
-    const uint32_t v = blockIdx.y;
-    const float* B = P.basis[v];
-    const float4 p = pos[nn];
-    // dot3 (math.rs:20-22) in the reference's order, then the depth of projection.rs:20-21
-    const float x = p.x * B[0] + p.y * B[1] + p.z * B[2];
-    const float y = p.x * B[3] + p.y * B[4] + p.z * B[5];
-    const float f = p.x * B[6] + p.y * B[7] + p.z * B[8];
-    const float depth = clampf_(0.5f + 0.5f * f / fmaxf(P.ws, kRenderEps), 0.0f, 1.0f);
-    const float sigma = fmaxf(clampf_(sigmas[nn], P.min_sigma, P.max_sigma), kRenderEps);
-    const float sigma2 = sigma * sigma;
-    const float k2 = kLog2e / (2.0f * sigma2);
-    const int64_t radius = f32_to_isize(fmaxf(ceilf(5.0f * sigma), 1.0f));
-    const float fsz1 = (float)P.size - 1.0f;
-    const float px = (x + P.ws) / (2.0f * P.ws) * fsz1;
-    const float py = (P.ws - y) / (2.0f * P.ws) * fsz1;
-    const int64_t bx = f32_to_isize(floorf(px)), by = f32_to_isize(floorf(py));
-    const float fx = px - (float)bx, fy = py - (float)by;
-    int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;
-    const bool any = live && render_tiles(P, bx, by, radius, &tx0, &tx1, &ty0, &ty1);
-    float part = 0.0f;
-    if (any) {  // the in-bounds part of the footprint (image.rs:49-63)
-        const int oy0 = (int)(by - radius < 0 ? -by : -radius);
-        const int oy1 = (int)(by + radius > P.size - 1 ? P.size - 1 - by : radius);
-        const int ox0 = (int)(bx - radius < 0 ? -bx : -radius);
-        const int ox1 = (int)(bx + radius > P.size - 1 ? P.size - 1 - bx : radius);
-        for (int oy = oy0 + (int)lane; oy <= oy1; oy += (int)kPrepLanes) {
-            const float dy = (float)oy - fy;
-            for (int ox = ox0; ox <= ox1; ++ox) {
-                const float dx = (float)ox - fx;
-                part += splat_weight(dx * dx + dy * dy, k2);
-            }
-        }
-    }
-#pragma unroll
-    for (uint32_t m = kPrepLanes / 2; m >= 1; m >>= 1) part += __shfl_xor(part, (int)m, (int)kPrepLanes);
-    if (!live || lane != 0) return;
-    const uint64_t i = (uint64_t)v * P.count + n;
-    RenderParticle rp;
-    rp.px = px;
-    rp.py = py;
-    rp.x0 = any ? (int)(bx - radius) : 0;
-    rp.y0 = any ? (int)(by - radius) : 0;
-    rp.span = any ? (uint32_t)(2 * radius) : 0u;
-    rp.k2 = k2;
-    rp.scale = P.norm_scale * clampf_(opacities[n], 0.0f, 1.0f) / fmaxf(part, kRenderEps);  // image.rs:67-69
-    rp.depth = depth;
-    rp.c[0] = colors[3 * (uint64_t)n];
-    rp.c[1] = colors[3 * (uint64_t)n + 1];
-    rp.c[2] = colors[3 * (uint64_t)n + 2];
-    rp.pad = 0.0f;
-    out[i] = rp;
-    ntiles[i] = any ? (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1)) : 0u;
-}
-
-// The items of the matrix-core drawing (npa_draw.hip): one thread per particle-view.
+// One thread per particle-view (blockIdx.y is the view, so its basis is a uniform load): dot3 (math.rs:20-22) in
+// the reference's order, the depth of projection.rs:20-21, the footprint of image.rs:41-69.
 __global__ __launch_bounds__(256) void k_render_items(RenderParams P, const float4* __restrict__ pos,
                                                       const float* __restrict__ colors,
                                                       const float* __restrict__ opacities,
@@ -800,156 +472,6 @@ __global__ __launch_bounds__(256) void k_render_items(RenderParams P, const floa
     const uint64_t i = (uint64_t)v * P.count + n;
     out[i] = d;
     rects[i] = fp.rect;
-}
-
-__global__ __launch_bounds__(256) void k_render_emit(RenderParams P, const RenderParticle* __restrict__ rp,
-                                                     const uint32_t* __restrict__ ntiles,
-                                                     const uint32_t* __restrict__ start, uint32_t items,
-                                                     uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= items || ntiles[i] == 0) return;
-    const RenderParticle q = rp[i];
-    const int64_t r = q.span / 2;
-    int tx0, tx1, ty0, ty1;
-    render_tiles(P, (int64_t)q.x0 + r, (int64_t)q.y0 + r, r, &tx0, &tx1, &ty0, &ty1);
-    uint32_t k = start[i];
-    const uint32_t base = (i / P.count) * P.tiles_per_view;
-    for (int ty = ty0; ty <= ty1; ++ty)
-        for (int tx = tx0; tx <= tx1; ++tx) {
-            keys[k] = base + (uint32_t)(ty * P.tiles_x + tx);
-            vals[k] = i;
-            ++k;
-        }
-}
-
-// The sorted particle list of each screen tile is cut into chunks of kChunk particles; a block
-// draws one chunk of one tile (thread = pixel, the chunk staged in LDS), summing its particles in
-// ascending index order into a partial tile. k_render_reduce then adds each tile's partials in
-// chunk order. A tile of one chunk is thus exactly the reference's running sum; a longer list
-// differs from it only by the rounding of the chunk boundaries.
-constexpr uint32_t kChunk = 256;
-
-// One block: nch[t] = ceil(tile t's key count / kChunk), chunk_start = its exclusive prefix, and
-// the total into *total. ntiles <= 65536, so each thread owns at most 64 consecutive tiles.
-__global__ __launch_bounds__(1024) void k_render_chunk_scan(const uint32_t* __restrict__ offsets, uint32_t ntiles,
-                                                            uint32_t* __restrict__ nch,
-                                                            uint32_t* __restrict__ chunk_start,
-                                                            uint32_t* __restrict__ total) {
-    __shared__ uint32_t lds[16];
-    const uint32_t per = (ntiles + blockDim.x - 1) / blockDim.x;
-    const uint32_t t0 = threadIdx.x * per;
-    const uint32_t t1 = t0 + per < ntiles ? t0 + per : ntiles;
-    uint32_t sum = 0;
-    for (uint32_t t = t0; t < t1; ++t) {
-        const uint32_t c = (offsets[t + 1] - offsets[t] + kChunk - 1) / kChunk;
-        nch[t] = c;
-        sum += c;
-    }
-    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    uint32_t x = sum;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= (uint32_t)off) x += y;
-    }
-    if (lane == 63) lds[wid] = x;
-    __syncthreads();
-    uint32_t base = 0, all = 0;
-    for (uint32_t w = 0; w < nw; ++w) {
-        const uint32_t v = lds[w];
-        if (w < wid) base += v;
-        all += v;
-    }
-    uint32_t run = base + x - sum;
-    for (uint32_t t = t0; t < t1; ++t) {
-        chunk_start[t] = run;
-        run += nch[t];
-    }
-    if (threadIdx.x == 0) *total = all;
-}
-
-// Grid-stride over the chunks; thread = pixel, the chunk's particles staged in LDS. dx = x - px
-// is the reference's (x - base_x) - frac_x exactly: both are one rounding of the same real number.
-// partials[c][5][256] (channel-planar, so the stores coalesce).
-__global__ __launch_bounds__(256) void k_render_chunks(RenderParams P, const RenderParticle* __restrict__ rp,
-                                                       const uint32_t* __restrict__ offsets,
-                                                       const uint32_t* __restrict__ sorted,
-                                                       const uint32_t* __restrict__ chunk_start,
-                                                       const uint32_t* __restrict__ total_chunks, uint32_t ntiles,
-                                                       float* __restrict__ partials) {
-    __shared__ RenderParticle buf[kChunk];
-    const uint32_t total = *total_chunks;
-    for (uint32_t c = blockIdx.x; c < total; c += gridDim.x) {
-        // the tile: the last t with chunk_start[t] <= c (tiles without chunks share the next start)
-        uint32_t lo = 0, hi = ntiles - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) / 2;
-            if (chunk_start[mid] <= c) lo = mid;
-            else hi = mid - 1;
-        }
-        const uint32_t t = lo;
-        const uint32_t v = t / P.tiles_per_view, lt = t - v * P.tiles_per_view;
-        const int x = (int)(lt % (uint32_t)P.tiles_x) * kTile + (int)(threadIdx.x % kTile);
-        const int y = (int)(lt / (uint32_t)P.tiles_x) * kTile + (int)(threadIdx.x / kTile);
-        const float xf = (float)x, yf = (float)y;
-        const uint32_t beg = offsets[t] + (c - chunk_start[t]) * kChunk;
-        const uint32_t end = min(beg + kChunk, offsets[t + 1]);
-        if (beg + threadIdx.x < end) buf[threadIdx.x] = rp[sorted[beg + threadIdx.x]];
-        __syncthreads();
-        float acc[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        const uint32_t m = end - beg;
-        for (uint32_t q = 0; q < m; ++q) {
-            const RenderParticle& p = buf[q];
-            if ((uint32_t)(x - p.x0) > p.span || (uint32_t)(y - p.y0) > p.span) continue;
-            const float dx = xf - p.px, dy = yf - p.py;
-            const float w = splat_weight(dx * dx + dy * dy, p.k2) * p.scale;  // image.rs:61, 69
-            acc[0] += p.c[0] * w;
-            acc[1] += p.c[1] * w;
-            acc[2] += p.c[2] * w;
-            acc[3] += w;
-            acc[4] += p.depth * w;
-        }
-        float* o = partials + (uint64_t)c * (5 * kChunk) + threadIdx.x;
-#pragma unroll
-        for (int ch = 0; ch < 5; ++ch) o[ch * kChunk] = acc[ch];
-        __syncthreads();  // buf is refilled by the next chunk
-    }
-}
-
-// One tile per block, thread = pixel: the tile's partials in chunk order (zero for an empty tile).
-__global__ __launch_bounds__(256) void k_render_reduce(RenderParams P, const uint32_t* __restrict__ chunk_start,
-                                                       const uint32_t* __restrict__ nch,
-                                                       const float* __restrict__ partials,
-                                                       float* __restrict__ images) {
-    const uint32_t t = blockIdx.x;
-    const uint32_t v = t / P.tiles_per_view, lt = t - v * P.tiles_per_view;
-    const int x = (int)(lt % (uint32_t)P.tiles_x) * kTile + (int)(threadIdx.x % kTile);
-    const int y = (int)(lt / (uint32_t)P.tiles_x) * kTile + (int)(threadIdx.x / kTile);
-    float acc[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t c0 = chunk_start[t], c1 = c0 + nch[t];
-    uint32_t c = c0;
-    for (; c + 4 <= c1; c += 4) {  // four chunks' loads in flight, then added in chunk order
-        float v[4][5];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float* q = partials + (uint64_t)(c + u) * (5 * kChunk) + threadIdx.x;
-#pragma unroll
-            for (int ch = 0; ch < 5; ++ch) v[u][ch] = q[ch * kChunk];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int ch = 0; ch < 5; ++ch) acc[ch] += v[u][ch];
-    }
-    for (; c < c1; ++c) {
-        const float* q = partials + (uint64_t)c * (5 * kChunk) + threadIdx.x;
-#pragma unroll
-        for (int ch = 0; ch < 5; ++ch) acc[ch] += q[ch * kChunk];
-    }
-    if (x < P.size && y < P.size) {
-        float* o = images + (((uint64_t)v * P.size + y) * P.size + x) * 5;
-#pragma unroll
-        for (int ch = 0; ch < 5; ++ch) o[ch] = acc[ch];
-    }
 }
 
 // view_basis (render_loss/projection.rs:31-43) with normalize3 / cross3 (render_loss/math.rs:24-39).
@@ -988,8 +510,6 @@ hipError_t launch_render_views(const float4* pos, const float* colors, const flo
     if (nviews == 0 || nviews > kMaxRenderViews || !views) return hipErrorInvalidValue;
     RenderParams P{};
     P.size = (int)cfg.image_size;
-    P.tiles_x = (P.size + kTile - 1) / kTile;
-    P.tiles_per_view = (uint32_t)(P.tiles_x * P.tiles_x);
     P.count = count;
     P.ws = cfg.world_scale;
     P.min_sigma = cfg.min_sigma;
@@ -997,104 +517,28 @@ hipError_t launch_render_views(const float4* pos, const float* colors, const flo
     P.norm_scale = 1.0f / (float)(count > 1 ? count : 1);  // image.rs:29
     for (uint32_t v = 0; v < nviews; ++v)
         if (!render_view_basis(views[v], P.basis[v])) return hipErrorInvalidValue;
-    const uint64_t ntile64 = (uint64_t)P.tiles_per_view * nviews;
-    if (ntile64 > 65536) return hipErrorInvalidValue;  // the key sort's bin limit
-    const uint32_t ntile_total = (uint32_t)ntile64;
     const uint64_t items64 = (uint64_t)count * nviews;
-    if (items64 >= (1ull << 31) || (uint64_t)count * kPrepLanes >= (1ull << 32)) return hipErrorInvalidValue;
+    if (items64 >= (1ull << 31) || (uint64_t)count * 16 >= (1ull << 32)) return hipErrorInvalidValue;
     const uint32_t items = (uint32_t)items64;
     // the widest footprint: sigma <= max(max_sigma, EPS)
     const float rmaxf = fmaxf(ceilf(5.0f * fmaxf(cfg.max_sigma, kRenderEps)), 1.0f);
     if (!(rmaxf <= 1024.0f)) return hipErrorInvalidValue;
-    const uint64_t per_axis = (uint64_t)((2 * (int)rmaxf + 1 + kTile - 1) / kTile + 1);
-    const uint64_t max_per = std::min<uint64_t>(per_axis * per_axis, P.tiles_per_view);
-    const uint64_t cap64 = items64 * max_per;
-    if (cap64 >= (1ull << 31)) return hipErrorInvalidValue;
-    const uint32_t cap = (uint32_t)cap64;
+    if (!draw_within_limits(P.size, nviews, items64, (int)rmaxf)) return hipErrorInvalidValue;
     hipError_t e;
-#define NPA_RES(buf, n) \
-    if ((e = (buf).reserve((size_t)(n))) != hipSuccess) return e;
     DrawPlan draw;
-    if (make_draw_plan(P.size, nviews, count, items, 5, nviews, &draw)) {
-        NPA_RES(ws.params, (uint64_t)(items ? items : 1) * sizeof(DrawItem));
-        NPA_RES(ws.keys, (uint64_t)(items ? items : 1) * 4);
-        NPA_RES(ws.partials, draw.partial_floats * 4);
-        ProfScope ps(prof, NPA_KERNEL_RENDER, stream);
-        if (count) {
-            hipLaunchKernelGGL(k_render_items, dim3((count + 255) / 256, nviews), dim3(256), 0, stream, P, pos, colors,
-                               opacities, sigmas, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), images, stream);
-    }
-    HashgridPlan plan;
-    if (!make_key_sort_plan(cap, ntile_total, &plan)) return hipErrorInvalidValue;
-    NPA_RES(ws.params, (uint64_t)(items ? items : 1) * sizeof(RenderParticle));
-    NPA_RES(ws.item_start, (uint64_t)(items ? items : 1) * 8);
-    NPA_RES(ws.keys, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.vals, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.sorted, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.ranks, (uint64_t)(cap ? cap : 1) * 4);
-    NPA_RES(ws.table, plan.table_entries * 4);
-    NPA_RES(ws.totals, (uint64_t)ntile_total * 4);
-    NPA_RES(ws.offsets, ((uint64_t)ntile_total + 1) * 4);
-    NPA_RES(ws.count, 64);
-    NPA_RES(ws.scan, (2 * ((uint64_t)items / kScanBlock + 1) + 2) * 4);
-    NPA_RES(ws.flags, 64);
-    // chunks: at most one partial per kChunk keys plus one per tile
-    const uint64_t max_chunks = (uint64_t)cap / kChunk + ntile_total;
-    NPA_RES(ws.partials, max_chunks * 5 * kChunk * 4);
-    NPA_RES(ws.chunks, (2 * (uint64_t)ntile_total + 1) * 4);
-#undef NPA_RES
+    const float typical = fminf(fmaxf(cfg.sigma, cfg.min_sigma), cfg.max_sigma);  // (each particle has its own)
+    const int radius = typical > 0.0f ? (int)ceilf(5.0f * typical) : 1;
+    if (!make_draw_plan(P.size, radius, nviews, count, items, 5, nviews, &draw)) return hipErrorInvalidValue;
+    if ((e = ws.params.reserve((uint64_t)(items ? items : 1) * sizeof(DrawItem))) != hipSuccess) return e;
+    if ((e = ws.keys.reserve((uint64_t)(items ? items : 1) * 4)) != hipSuccess) return e;
+    if ((e = ws.partials.reserve(draw.partial_floats * 4)) != hipSuccess) return e;
     ProfScope ps(prof, NPA_KERNEL_RENDER, stream);
-    uint32_t* ntiles = ws.item_start.as<uint32_t>() + (items ? items : 1);
-    uint32_t* start = ws.item_start.as<uint32_t>();
-    RenderParticle* rp = ws.params.as<RenderParticle>();
     if (count) {
-        hipLaunchKernelGGL(k_render_prep, dim3((uint32_t)(((uint64_t)count * kPrepLanes + 255) / 256), nviews), dim3(256),
-                           0, stream, P, pos, colors,
-                           opacities, sigmas, rp, ntiles);
+        hipLaunchKernelGGL(k_render_items, dim3((count + 255) / 256, nviews), dim3(256), 0, stream, P, pos, colors, opacities,
+                           sigmas, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    {  // start = exclusive prefix of ntiles, total key count into ws.count
-        const uint32_t nb = (items + kScanBlock - 1) / kScanBlock;
-        uint32_t* sums = ws.scan.as<uint32_t>();
-        if (nb) {
-            hipLaunchKernelGGL(k_scan_partials, dim3(nb), dim3(256), 0, stream, ntiles, items, sums);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(k_scan_1block, dim3(1), dim3(1024), 0, stream, sums, sums + nb + 1, nb,
-                           ws.count.as<uint32_t>());
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (nb) {
-            hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, stream, ntiles, start, items, sums + nb + 1);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-    }
-    if (items) {
-        hipLaunchKernelGGL(k_render_emit, dim3((items + 255) / 256), dim3(256), 0, stream, P, rp, ntiles, start, items,
-                           ws.keys.as<uint32_t>(), ws.vals.as<uint32_t>());
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    e = launch_key_sort(plan, ws.keys.as<uint32_t>(), ws.vals.as<uint32_t>(), ws.count.as<uint32_t>(), cap,
-                        ws.ranks.as<uint32_t>(), ws.table.as<uint32_t>(), ws.totals.as<uint32_t>(),
-                        ws.offsets.as<uint32_t>(), ws.sorted.as<uint32_t>(), ws.flags.as<uint32_t>(), stream);
-    if (e != hipSuccess) return e;
-    {  // chunks per tile, their exclusive prefix and total, then the chunks and the reduction
-        uint32_t* nch = ws.chunks.as<uint32_t>();
-        uint32_t* cstart = nch + ntile_total;
-        uint32_t* ctotal = cstart + ntile_total;
-        hipLaunchKernelGGL(k_render_chunk_scan, dim3(1), dim3(1024), 0, stream, ws.offsets.as<uint32_t>(), ntile_total,
-                           nch, cstart, ctotal);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        const uint32_t grid = (uint32_t)std::min<uint64_t>(max_chunks, 4096);
-        hipLaunchKernelGGL(k_render_chunks, dim3(grid), dim3(256), 0, stream, P, rp, ws.offsets.as<uint32_t>(),
-                           ws.sorted.as<uint32_t>(), cstart, ctotal, ntile_total, ws.partials.as<float>());
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_render_reduce, dim3(ntile_total), dim3(256), 0, stream, P, cstart, nch,
-                           ws.partials.as<float>(), images);
-    }
-    return hipGetLastError();
+    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), images, stream);
 }
 
 // state_tail_render_attributes (render_loss/attributes.rs:15-87): one thread per particle.

@@ -393,7 +393,7 @@ hipError_t launch_write_gaussians(const float4* pos, const float* states, uint32
 struct SplatWorkspace {
     DevBuf params, item_start, keys, vals, sorted, ranks, table, totals, offsets, count, flags, scan;
     DevBuf attrs;  // render attributes of a state's particles: colours [n][3], opacities [n], sigmas [n]
-    DevBuf partials, chunks;  // render: per-chunk partial tiles; chunk counts, starts and total
+    DevBuf partials;  // the drawing's partial images, one per item range
     DevBuf order;      // oriented raster: depth order
     DevBuf sort_temp;  // oriented raster: the radix sort's temporary storage
     DevBuf decoded;  // oriented raster of a state: its decoded Gaussians

@@ -1,5 +1,5 @@
-"""The splat and the projected render drawn on the matrix cores, at the edges of their tiles, groups, batches
-of 8,192 items and item ranges, against the oracle; non-finite particles touch only their own footprint."""
+"""The splat and the projected render drawn on the matrix cores, at the edges of their tiles, groups, the
+waves' shares of the items and item ranges, against the oracle; non-finite particles touch only their own footprint."""
 import numpy as np
 import pytest
 
