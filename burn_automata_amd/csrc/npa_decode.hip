@@ -603,10 +603,15 @@ hipError_t launch_render_attributes(const float* states, uint32_t count, uint32_
 //   k_raster_emit      the (tile, Gaussian) items in depth order, after a prefix of the tile
 //                      counts (its total read back to size the item buffers);
 //   stable key sort    by tile (the hashgrid's counting sort) -> per-tile lists in depth order;
-//   k_raster_tiles     one 256-thread block per 16x16 tile, one pixel per thread: the list is
-//                      staged through LDS 256 Gaussians at a time; each pixel composites front to
-//                      back and stops at the transmittance cut; the block leaves when every pixel
-//                      has stopped.
+//   k_raster_tiles     one 256-thread block per 16x16 tile; each wave draws an 8x8 block of its pixels
+//                      by itself, without barriers: of 64 Gaussians of the list it keeps those that
+//                      reach the 1/255 floor on its block (a lane tests one), and each pixel composites
+//                      those front to back and stops at the transmittance cut; the wave leaves when
+//                      every pixel has stopped.
+// Bound: vector instructions, about 20 per pixel and kept Gaussian. A 3-sigma tile rectangle holds two
+// to three times the pixels that its Gaussian's 1/255 contour does; testing each 8x8 block (about 30
+// lane instructions a Gaussian, for the 1,280 it saves) draws 16,384 oriented Gaussians at 1024x768 in
+// 71 us where evaluating every listed Gaussian in every pixel took 142 us; the frame is bit-identical.
 struct RasterParams {
     float view[12];
     float fx, fy, cx, cy, limx, limy, near_plane, far_plane;
@@ -819,58 +824,104 @@ __global__ __launch_bounds__(256) void k_raster_emit(RasterParams P, const Raste
     }
 }
 
+// Whether a Gaussian can reach the 1/255 floor on an 8x8 pixel block whose first pixel centre is
+// (x, y): the largest exponent over the block, from the edges facing the mean, against
+// log2(1 / (255 opacity)).  False only where every pixel would drop it: the slack is over ten times
+// the rounding of the pixels' own exponents, and a conic near singular (where the edges that do not
+// face the mean could hold the maximum), an infinity or a NaN is kept for the pixels to decide.
+__device__ __forceinline__ bool raster_reaches(const float4& A, const float4& B, float x, float y) {
+    const float x0 = A.x - (x + 7.0f), x1 = A.x - x, y0 = A.y - (y + 7.0f), y1 = A.y - y;
+    const float nx = __builtin_amdgcn_fmed3f(0.0f, x0, x1), ny = __builtin_amdgcn_fmed3f(0.0f, y0, y1);
+    const float ax = fmaxf(fabsf(x0), fabsf(x1)), ay = fmaxf(fabsf(y0), fabsf(y1));
+    const float qa = A.z, qb = A.w, qc = B.x;
+    // along the edge dx = nx the exponent is largest at dy = -qb nx / 2 qc, along dy = ny likewise
+    const float ey = __builtin_amdgcn_fmed3f(-0.5f * qb * nx * __builtin_amdgcn_rcpf(qc), y0, y1);
+    const float ex = __builtin_amdgcn_fmed3f(-0.5f * qb * ny * __builtin_amdgcn_rcpf(qa), x0, x1);
+    const float pa = qa * nx * nx + qb * nx * ey + qc * ey * ey;
+    const float pb = qa * ex * ex + qb * ex * ny + qc * ny * ny;
+    const float size = fabsf(qa) * ax * ax + fabsf(qb) * ax * ay + fabsf(qc) * ay * ay;
+    const float least = __builtin_amdgcn_logf(__builtin_amdgcn_rcpf(255.0f * B.y)) - (1e-3f + 1e-5f * size);
+    const bool sound = 4.0f * qa * qc - qb * qb > 4e-3f * qa * qc;  // qa, qc < 0
+    const bool inside = nx == 0.0f && ny == 0.0f;
+    return !(sound && !inside && pa < least && pb < least);
+}
+
 __global__ __launch_bounds__(256) void k_raster_tiles(RasterParams P, const RasterSplat* __restrict__ sp,
                                                       const uint32_t* __restrict__ offsets,
                                                       const uint32_t* __restrict__ sorted, float4* __restrict__ image) {
-    __shared__ float4 la[256], lb[256];
-    __shared__ float lc[256];
-    const uint32_t tile = blockIdx.x;
-    const uint32_t px = (tile % P.tiles_x) * 16 + (threadIdx.x & 15);
-    const uint32_t py = (tile / P.tiles_x) * 16 + (threadIdx.x >> 4);
+    __shared__ float4 la[4][68], lb[4][68];
+    __shared__ float lc[4][68];
+    const uint32_t tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t bx = (tile % P.tiles_x) * 16 + (wave & 1) * 8, by = (tile / P.tiles_x) * 16 + (wave >> 1) * 8;
+    const uint32_t px = bx + (lane & 7), py = by + (lane >> 3);
     const bool inside = px < P.width && py < P.height;
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
+    const float bxc = (float)bx + 0.5f, byc = (float)by + 0.5f;
     const uint32_t begin = offsets[tile], end = offsets[tile + 1];
     float T = 1.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;
-    int done = inside ? 0 : 1;
-    for (uint32_t base = begin; base < end; base += 256) {
-        if (__syncthreads_count(done) == (int)blockDim.x) break;
-        const uint32_t k = base + threadIdx.x;
-        if (k < end) {
-            const float4* s4 = reinterpret_cast<const float4*>(sp + sorted[k]);
-            la[threadIdx.x] = s4[0];
-            lb[threadIdx.x] = s4[1];
-            lc[threadIdx.x] = s4[2].x;
+    bool done = !inside;
+    // the next round's record and the index of the one after are in flight while a round is drawn
+    float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A;
+    float C = 0.0f;
+    uint32_t g = 0;
+    if (begin + lane < end) {
+        const float4* s4 = reinterpret_cast<const float4*>(sp + sorted[begin + lane]);
+        A = s4[0];
+        B = s4[1];
+        C = s4[2].x;
+    }
+    if (begin + 64 + lane < end) g = sorted[begin + 64 + lane];
+    for (uint32_t base = begin; base < end && !__all(done); base += 64) {
+        const bool keep = base + lane < end && raster_reaches(A, B, bxc, byc);
+        const uint64_t kept = __ballot(keep);
+        const uint32_t n = (uint32_t)__popcll(kept);
+        if (keep) {
+            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0));
+            la[wave][at] = A;
+            lb[wave][at] = B;
+            lc[wave][at] = C;
         }
-        __syncthreads();
-        const uint32_t n = end - base < 256 ? end - base : 256;
+        if (lane < 4) {  // opacity 0: nothing drawn
+            la[wave][n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+            lb[wave][n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+            lc[wave][n + lane] = 0.0f;
+        }
+        if (base + 64 + lane < end) {
+            const float4* s4 = reinterpret_cast<const float4*>(sp + g);
+            A = s4[0];
+            B = s4[1];
+            C = s4[2].x;
+        }
+        if (base + 128 + lane < end) g = sorted[base + 128 + lane];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         // Branch-free: every lane evaluates every entry and the tests become selects (the same
         // comparisons, so NaN behaves as in a branching loop); a stopped lane keeps its values.
-        // The wave leaves the batch once all of its lanes have stopped.
         for (uint32_t u0 = 0; u0 < n; u0 += 4) {
 #pragma unroll
             for (uint32_t du = 0; du < 4; ++du) {
-                const uint32_t u = u0 + du;
-                if (u >= n) break;  // wave-uniform
-                const float4 A = la[u], B = lb[u];  // (mx, my, qa, qb), (qc, opacity, r, g)
-                const float C = lc[u];
-                const float dx = A.x - pxc, dy = A.y - pyc;
+                const float4 a = la[wave][u0 + du], b = lb[wave][u0 + du];  // (mx, my, qa, qb), (qc, opacity, r, g)
+                const float c = lc[wave][u0 + du];
+                const float dx = a.x - pxc, dy = a.y - pyc;
                 // power * log2(e), with the oracle's fused operations
-                const float p2 = __builtin_fmaf(A.z * dx, dx, __builtin_fmaf(B.x * dy, dy, A.w * dx * dy));
+                const float p2 = __builtin_fmaf(a.z * dx, dx, __builtin_fmaf(b.x * dy, dy, a.w * dx * dy));
                 // the hardware 2^x: below 2^-126 alpha is far under the 1/255 floor either way
-                const float alpha = fminf(0.99f, B.y * __builtin_amdgcn_exp2f(p2));
+                const float alpha = fminf(0.99f, b.y * __builtin_amdgcn_exp2f(p2));
                 const float next = T * (1.0f - alpha);
                 const bool ok = !done && !(p2 > 0.0f) && !(alpha < 1.0f / 255.0f);
                 const bool stop = ok && next < 0.0001f;
                 const bool apply = ok && !stop;
                 const float wgt = alpha * T;
-                cr = apply ? __builtin_fmaf(B.z, wgt, cr) : cr;
-                cg = apply ? __builtin_fmaf(B.w, wgt, cg) : cg;
-                cb = apply ? __builtin_fmaf(C, wgt, cb) : cb;
+                cr = apply ? __builtin_fmaf(b.z, wgt, cr) : cr;
+                cg = apply ? __builtin_fmaf(b.w, wgt, cg) : cg;
+                cb = apply ? __builtin_fmaf(c, wgt, cb) : cb;
                 T = apply ? next : T;
                 done = done || stop;
             }
             if (__all(done)) break;
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
     if (inside) image[(uint64_t)py * P.width + px] = make_float4(cr, cg, cb, 1.0f - T);
 }
