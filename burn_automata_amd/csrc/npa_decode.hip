@@ -600,14 +600,20 @@ hipError_t launch_render_attributes(const float* states, uint32_t count, uint32_
 //                      (spherical harmonics or RGB), the tile count and the depth key;
 //   depth order        a stable radix sort of the indices by the positive depth's float bits
 //                      (rocPRIM): depth ascending, ties by index;
-//   k_raster_emit      the (tile, Gaussian) items in depth order, after a prefix of the tile
-//                      counts (its total read back to size the item buffers);
-//   stable key sort    by tile (the hashgrid's counting sort) -> per-tile lists in depth order;
+//   k_raster_lists     up to kRasterListMax Gaussians: a block per group of tiles lists those whose
+//                      rectangles touch it, in depth order; nothing is read back;
+//   or, for more, k_raster_emit (the (tile, Gaussian) items in depth order, after a prefix of the tile
+//                      counts; its total read back to size the item buffers) and a stable key sort by
+//                      tile (the hashgrid's counting sort) -> per-tile lists in depth order;
 //   k_raster_tiles     one 256-thread block per 16x16 tile; each wave draws an 8x8 block of its pixels
 //                      by itself, without barriers: of 64 Gaussians of the list it keeps those that
 //                      reach the 1/255 floor on its block (a lane tests one), and each pixel composites
 //                      those front to back and stops at the transmittance cut; the wave leaves when
 //                      every pixel has stopped.
+// Both give a tile the same Gaussians in the same order. 65,536 Gaussians (one more for the items):
+// 285 us with lists at 640x480 and 228 us at 1280x1024, 341 and 322 us with items; at 4096x4096, with
+// groups of 16x16 tiles, 2,691 and 2,698 us. 16,384 at 1024x768, decode included: 124 and 186 us. Past 16
+// bits of Gaussians an entry would double and the lists, each as long as all Gaussians, outgrow the items.
 // Bound: vector instructions, about 20 per pixel and kept Gaussian. A 3-sigma tile rectangle holds two
 // to three times the pixels that its Gaussian's 1/255 contour does; testing each 8x8 block (about 30
 // lane instructions a Gaussian, for the 1,280 it saves) draws 16,384 oriented Gaussians at 1024x768 in
@@ -637,10 +643,12 @@ __device__ __forceinline__ float raster_clamp(float v, float lo, float hi) { ret
 __global__ __launch_bounds__(256) void k_raster_prep(RasterParams P, const float4* __restrict__ pv,
                                                      const float* __restrict__ sh, const float4* __restrict__ rot,
                                                      const float4* __restrict__ so, RasterSplat* __restrict__ out,
-                                                     uint32_t* __restrict__ ntiles, uint32_t* __restrict__ dkey) {
+                                                     uint32_t* __restrict__ ntiles, uint2* __restrict__ rects,
+                                                     uint32_t* __restrict__ dkey) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P.count) return;
-    ntiles[i] = 0;
+    if (rects) rects[i] = make_uint2(0u, 0u);
+    else ntiles[i] = 0;
     dkey[i] = kDepthCulled;
     const float4 p = pv[i];
     if (!(p.w > 0.0f)) return;
@@ -762,9 +770,80 @@ __global__ __launch_bounds__(256) void k_raster_prep(RasterParams P, const float
         o.b = rgb[2];
     }
     out[i] = o;
-    ntiles[i] = (x1 - x0) * (y1 - y0);
+    if (rects) rects[i] = make_uint2(o.rx, o.ry);
+    else ntiles[i] = (x1 - x0) * (y1 - y0);
     dkey[i] = __float_as_uint(tz);
 }
+
+// ---- Up to kRasterListMax Gaussians: one list per group of (1 << shift)^2 tiles.
+constexpr uint32_t kRasterListMax = 65536;  // an entry holds its Gaussian in 16 bits
+constexpr uint32_t kRasterGroups = 512;     // at most this many groups
+
+__global__ __launch_bounds__(256) void k_raster_order_rects(const uint2* __restrict__ rects,
+                                                            const uint32_t* __restrict__ order, uint32_t count,
+                                                            uint2* __restrict__ out) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < count) out[j] = rects[order[j]];
+}
+
+// One block per group: the Gaussians whose rectangles touch it, in depth order, at lists[group * count].
+// An entry is the Gaussian << 16 | the group's tiles that it covers as four inclusive 4-bit bounds
+// (x first, x last, y first, y last). Each wave tests a consecutive range of the depth order and
+// keeps the hits as bits, then writes its entries after those of the waves before it.
+// Bound: the latency of a wave's loads, kRasterAhead in flight: 16 waves test 16,384 in four batches each
+// (13 us for 192 groups, against 45 us for the counts, their prefix and total, the items and their sort).
+constexpr int kRasterAhead = 4;
+
+__global__ __launch_bounds__(1024) void k_raster_lists(const uint2* __restrict__ orects,
+                                                       const uint32_t* __restrict__ order, uint32_t count,
+                                                       uint32_t shift, uint32_t groups_x, uint32_t* __restrict__ lists,
+                                                       uint32_t* __restrict__ counts) {
+    __shared__ uint64_t masks[kRasterListMax / 64];
+    __shared__ uint32_t wave_hits[16];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t gx = (blockIdx.x % groups_x) << shift, gy = (blockIdx.x / groups_x) << shift, side = 1u << shift;
+    const uint32_t chunks = (count + 63) / 64, per = (chunks + 15) / 16;
+    const uint32_t c0 = min(wave * per, chunks), c1 = min(c0 + per, chunks);
+    uint32_t hits = 0;
+    for (uint32_t c = c0; c < c1; c += kRasterAhead) {
+        uint2 r[kRasterAhead];
+#pragma unroll
+        for (int u = 0; u < kRasterAhead; ++u) {
+            const uint32_t j = (c + u) * 64 + lane;
+            r[u] = c + u < c1 && j < count ? orects[j] : make_uint2(0u, 0u);
+        }
+#pragma unroll
+        for (int u = 0; u < kRasterAhead; ++u) {
+            const uint64_t m = __ballot((r[u].x & 0xffffu) < gx + side && (r[u].x >> 16) > gx &&
+                                        (r[u].y & 0xffffu) < gy + side && (r[u].y >> 16) > gy);
+            if (c + u < c1 && lane == 0) masks[c + u] = m;
+            hits += (uint32_t)__popcll(m);
+        }
+    }
+    if (lane == 0) wave_hits[wave] = hits;
+    __syncthreads();
+    uint32_t at = 0, total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) {
+        at += w < wave ? wave_hits[w] : 0u;
+        total += wave_hits[w];
+    }
+    if (threadIdx.x == 0) counts[blockIdx.x] = total;
+    uint32_t* list = lists + (uint64_t)blockIdx.x * count;
+    for (uint32_t c = c0; c < c1; ++c) {
+        const uint64_t m = masks[c];
+        if ((m >> lane) & 1ull) {  // j < count: only such lanes hit
+            const uint32_t j = c * 64 + lane;
+            const uint2 r = orects[j];
+            const uint32_t xa = max(r.x & 0xffffu, gx) - gx, xb = min(r.x >> 16, gx + side) - gx - 1;
+            const uint32_t ya = max(r.y & 0xffffu, gy) - gy, yb = min(r.y >> 16, gy + side) - gy - 1;
+            list[at + (uint32_t)__popcll(m & lanemask_lt())] = (order[j] << 16) | xa | (xb << 4) | (ya << 8) | (yb << 12);
+        }
+        at += (uint32_t)__popcll(m);
+    }
+}
+
+// ---- More Gaussians: (tile, Gaussian) items, sorted by tile.
 
 __global__ __launch_bounds__(256) void k_raster_gather_counts(const uint32_t* __restrict__ ntiles,
                                                               const uint32_t* __restrict__ order, uint32_t count,
@@ -846,37 +925,90 @@ __device__ __forceinline__ bool raster_reaches(const float4& A, const float4& B,
     return !(sound && !inside && pa < least && pb < least);
 }
 
+// LISTS: `lists` holds the groups' entries (k_raster_lists), of which a wave keeps its tile's; otherwise
+// `lists` holds the items' Gaussians sorted by tile, from offsets[tile].
+template <bool LISTS>
 __global__ __launch_bounds__(256) void k_raster_tiles(RasterParams P, const RasterSplat* __restrict__ sp,
                                                       const uint32_t* __restrict__ offsets,
-                                                      const uint32_t* __restrict__ sorted, float4* __restrict__ image) {
+                                                      const uint32_t* __restrict__ lists, uint32_t shift,
+                                                      uint32_t groups_x, float4* __restrict__ image) {
     __shared__ float4 la[4][68], lb[4][68];
     __shared__ float lc[4][68];
+    __shared__ uint32_t waiting_g[LISTS ? 4 : 1][LISTS ? 128 : 1];
     const uint32_t tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t bx = (tile % P.tiles_x) * 16 + (wave & 1) * 8, by = (tile / P.tiles_x) * 16 + (wave >> 1) * 8;
+    const uint32_t tx = tile % P.tiles_x, ty = tile / P.tiles_x;
+    const uint32_t bx = tx * 16 + (wave & 1) * 8, by = ty * 16 + (wave >> 1) * 8;
     const uint32_t px = bx + (lane & 7), py = by + (lane >> 3);
     const bool inside = px < P.width && py < P.height;
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
     const float bxc = (float)bx + 0.5f, byc = (float)by + 0.5f;
-    const uint32_t begin = offsets[tile], end = offsets[tile + 1];
+    auto wave_fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    uint32_t pos, end, lx = 0, ly = 0;  // of the list; the tile within its group
+    if constexpr (LISTS) {
+        const uint32_t group = (ty >> shift) * groups_x + (tx >> shift);
+        pos = 0;
+        end = offsets[group];
+        lists += (uint64_t)group * P.count;
+        lx = tx & ((1u << shift) - 1);
+        ly = ty & ((1u << shift) - 1);
+    } else {
+        pos = offsets[tile];
+        end = offsets[tile + 1];
+    }
+    uint32_t ahead = pos + lane < end ? lists[pos + lane] : 0u;  // the list's next 64 entries
+    uint32_t waiting = 0;
+    // the next up to 64 Gaussians of the tile: lane l's in g for l < the count returned
+    auto take = [&](uint32_t& g) {
+        if constexpr (LISTS) {
+            while (waiting < 64 && pos < end) {
+                const uint32_t e = ahead;
+                const bool hit = pos + lane < end && lx >= (e & 15u) && lx <= ((e >> 4) & 15u) &&
+                                 ly >= ((e >> 8) & 15u) && ly <= ((e >> 12) & 15u);
+                pos += 64;
+                if (pos + lane < end) ahead = lists[pos + lane];
+                const uint64_t m = __ballot(hit);
+                if (hit) waiting_g[wave][waiting + (uint32_t)__popcll(m & lanemask_lt())] = e >> 16;
+                waiting += (uint32_t)__popcll(m);
+            }
+            wave_fence();
+            const uint32_t n = min(waiting, 64u);
+            g = waiting_g[wave][lane];
+            const uint32_t rest = waiting_g[wave][64 + lane];
+            waiting -= n;
+            wave_fence();
+            if (lane < waiting) waiting_g[wave][lane] = rest;
+            wave_fence();
+            return n;
+        } else {
+            const uint32_t n = min(end - pos, 64u);
+            g = ahead;
+            pos += n;
+            if (pos + lane < end) ahead = lists[pos + lane];
+            return n;
+        }
+    };
     float T = 1.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;
     bool done = !inside;
-    // the next round's record and the index of the one after are in flight while a round is drawn
     float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A;
     float C = 0.0f;
-    uint32_t g = 0;
-    if (begin + lane < end) {
-        const float4* s4 = reinterpret_cast<const float4*>(sp + sorted[begin + lane]);
+    auto load = [&](uint32_t g) {
+        const float4* s4 = reinterpret_cast<const float4*>(sp + g);
         A = s4[0];
         B = s4[1];
         C = s4[2].x;
-    }
-    if (begin + 64 + lane < end) g = sorted[begin + 64 + lane];
-    for (uint32_t base = begin; base < end && !__all(done); base += 64) {
-        const bool keep = base + lane < end && raster_reaches(A, B, bxc, byc);
+    };
+    uint32_t g;
+    uint32_t have = take(g);
+    if (lane < have) load(g);
+    while (have && !__all(done)) {
+        const bool keep = lane < have && raster_reaches(A, B, bxc, byc);
         const uint64_t kept = __ballot(keep);
         const uint32_t n = (uint32_t)__popcll(kept);
         if (keep) {
-            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0));
+            const uint32_t at = (uint32_t)__popcll(kept & lanemask_lt());
             la[wave][at] = A;
             lb[wave][at] = B;
             lc[wave][at] = C;
@@ -886,15 +1018,9 @@ __global__ __launch_bounds__(256) void k_raster_tiles(RasterParams P, const Rast
             lb[wave][n + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
             lc[wave][n + lane] = 0.0f;
         }
-        if (base + 64 + lane < end) {
-            const float4* s4 = reinterpret_cast<const float4*>(sp + g);
-            A = s4[0];
-            B = s4[1];
-            C = s4[2].x;
-        }
-        if (base + 128 + lane < end) g = sorted[base + 128 + lane];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        have = take(g);  // the next round's records are in flight while this one is drawn
+        if (lane < have) load(g);
+        wave_fence();
         // Branch-free: every lane evaluates every entry and the tests become selects (the same
         // comparisons, so NaN behaves as in a branching loop); a stopped lane keeps its values.
         for (uint32_t u0 = 0; u0 < n; u0 += 4) {
@@ -920,8 +1046,7 @@ __global__ __launch_bounds__(256) void k_raster_tiles(RasterParams P, const Rast
             }
             if (__all(done)) break;
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_fence();
     }
     if (inside) image[(uint64_t)py * P.width + px] = make_float4(cr, cg, cb, 1.0f - T);
 }
@@ -964,9 +1089,28 @@ hipError_t launch_raster_gaussians(const float4* pv, const float* sh, const floa
     NPA_RES(ws.item_start, (4 * n1 + 1) * 4);  // ntiles, depth keys, ordered counts, starts (+1)
     NPA_RES(ws.order, n1 * 4);
     NPA_RES(ws.keys, n1 * 4);
-    NPA_RES(ws.offsets, ((uint64_t)ntile_total + 1) * 4);
-    NPA_RES(ws.count, 64);
-    NPA_RES(ws.scan, (2 * (n1 / kScanBlock + 1) + 2) * 4);
+    // Groups of the smallest size that gives at most kRasterGroups of them (16x16 tiles at the image
+    // limit, 256 of those), so that a block per group about fills the chip. Lists hold up to
+    // kRasterListMax Gaussians, and take no more items than the sorted way accepts.
+    uint32_t shift = 0;
+    auto groups_along = [&](uint32_t tiles) { return (tiles + (1u << shift) - 1) >> shift; };
+    while (groups_along(P.tiles_x) * groups_along(P.tiles_y) > kRasterGroups && shift < 4) ++shift;
+    const uint32_t groups_x = groups_along(P.tiles_x), groups = groups_x * groups_along(P.tiles_y);
+    const bool lists = count && count <= kRasterListMax && groups <= kRasterGroups &&
+                       (uint64_t)count * ntile_total < (1ull << 31);
+    uint2 *rects = nullptr, *orects = nullptr;
+    if (lists) {
+        NPA_RES(ws.vals, n1 * 8);
+        NPA_RES(ws.sorted, n1 * 8);
+        NPA_RES(ws.table, (uint64_t)groups * count * 4);
+        NPA_RES(ws.totals, (uint64_t)groups * 4);
+        rects = ws.vals.as<uint2>();
+        orects = ws.sorted.as<uint2>();
+    } else {
+        NPA_RES(ws.offsets, ((uint64_t)ntile_total + 1) * 4);
+        NPA_RES(ws.count, 64);
+        NPA_RES(ws.scan, (2 * (n1 / kScanBlock + 1) + 2) * 4);
+    }
     ProfScope ps(prof, NPA_KERNEL_RASTER, stream);
     RasterSplat* sp = ws.params.as<RasterSplat>();
     uint32_t* ntiles = ws.item_start.as<uint32_t>();
@@ -977,13 +1121,25 @@ hipError_t launch_raster_gaussians(const float4* pv, const float* sh, const floa
     unsigned long long* d_total64 = reinterpret_cast<unsigned long long*>(ws.count.as<uint32_t>() + 2);
     if (count) {
         hipLaunchKernelGGL(k_raster_prep, dim3((count + 255) / 256), dim3(256), 0, stream, P, pv, sh, rot, so, sp,
-                           ntiles, dkey);
+                           ntiles, rects, dkey);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     // depth order: stable radix sort of the indices by the depth keys' bits 0-30 (non-negative floats)
     if ((e = sort_index_by_key(dkey, ws.keys.as<uint32_t>(), ord_a, count, 31, ws.sort_temp, stream)) != hipSuccess)
         return e;
     const uint32_t* order = ord_a;
+    if (lists) {
+        hipLaunchKernelGGL(k_raster_order_rects, dim3((count + 255) / 256), dim3(256), 0, stream, rects, order, count,
+                           orects);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_raster_lists, dim3(groups), dim3(1024), 0, stream, orects, order, count, shift, groups_x,
+                           ws.table.as<uint32_t>(), ws.totals.as<uint32_t>());
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_raster_tiles<true>, dim3(ntile_total), dim3(256), 0, stream, P, sp,
+                           ws.totals.as<uint32_t>(), ws.table.as<uint32_t>(), shift, groups_x,
+                           reinterpret_cast<float4*>(image));
+        return hipGetLastError();
+    }
     if (count) {
         hipLaunchKernelGGL(k_raster_gather_counts, dim3((count + 255) / 256), dim3(256), 0, stream, ntiles, order,
                            count, ocounts);
@@ -1031,8 +1187,8 @@ hipError_t launch_raster_gaussians(const float4* pv, const float* sh, const floa
                         ws.ranks.as<uint32_t>(), ws.table.as<uint32_t>(), ws.totals.as<uint32_t>(),
                         ws.offsets.as<uint32_t>(), ws.sorted.as<uint32_t>(), ws.flags.as<uint32_t>(), stream);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_raster_tiles, dim3(ntile_total), dim3(256), 0, stream, P, sp, ws.offsets.as<uint32_t>(),
-                       ws.sorted.as<uint32_t>(), reinterpret_cast<float4*>(image));
+    hipLaunchKernelGGL(k_raster_tiles<false>, dim3(ntile_total), dim3(256), 0, stream, P, sp,
+                       ws.offsets.as<uint32_t>(), ws.sorted.as<uint32_t>(), 0u, 0u, reinterpret_cast<float4*>(image));
     return hipGetLastError();
 }
 

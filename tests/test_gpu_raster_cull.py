@@ -38,3 +38,35 @@ def test_blocks_leave_out_only_what_every_pixel_drops(ctx, n, width, height, sca
     want = O.raster_gaussians_3d(pv, sh, rot, so, cam)
     assert np.isfinite(want).all()
     _check(K.raster_gaussians_3d(pv, sh, rot, so, cam, ctx=ctx), want, f"n={n} {width}x{height}")
+
+
+@pytest.mark.parametrize("n,width,height", [
+    (1, 16, 16), (64, 33, 400), (1023, 640, 20),  # a tile a group, single rows and columns of tiles
+    (1025, 368, 368),  # 23 x 23 tiles: groups of 2x2, the last ones partial
+    (16384, 1024, 768), (30001, 1500, 1100),  # 4x4
+    (5000, 2500, 1600),  # 8x8
+    (3000, 4096, 4096), (3000, 16384, 1024),  # 16x16, the tile limit
+    (65536, 300, 200),  # the most that the lists hold
+])
+def test_lists_by_group_draw_what_lists_by_tile_draw(ctx, n, width, height):
+    """Hidden Gaussians appended until the count is past the group lists' take the same frame to the sorted items:
+    the same Gaussians in the same order in every tile, so the images are equal bit for bit."""
+    rng = np.random.default_rng(n)
+    pv = np.ones((n, 4), f32)
+    pv[:, :3] = rng.uniform(-0.9, 0.9, (n, 3))
+    pv[: n // 3, 2] = 0.25  # equal positions along one axis
+    sh = rng.uniform(0.0, 1.0, (n, 1, 3)).astype(f32)
+    rot = rng.normal(size=(n, 4)).astype(f32)
+    so = np.exp(rng.uniform(math.log(0.002), math.log(0.05), (n, 4))).astype(f32)
+    so[:, 3] = rng.uniform(0.02, 1.0, n)
+    so[:: 500, :3] = 0.6  # some cover many groups
+    cam = RasterCamera.look_at((0.0, 0.1, 2.2), width=width, height=height, color_mode=RasterColor.Rgb)
+
+    def padded(a):
+        more = np.zeros((65537 - n, *a.shape[1:]), f32)
+        return np.concatenate([a, more])
+
+    got = K.raster_gaussians_3d(pv, sh, rot, so, cam, ctx=ctx).cpu().numpy()
+    want = K.raster_gaussians_3d(padded(pv), padded(sh), padded(rot), padded(so), cam, ctx=ctx).cpu().numpy()
+    assert (want[..., 3] > 0).any()
+    np.testing.assert_array_equal(got, want)
