@@ -217,30 +217,10 @@ __device__ __forceinline__ uint32_t row_last(uint32_t v) {
 //   t0 = w[E] * x, t1 = vg0[E] * diff, t2 = vg1[E] * diff (, t3 = vg2[E] * diff).
 // A DPP source must not have been written by the previous two VALU instructions (five after an
 // EXEC write): the s_nop provides those wait states, since the compiler does not see inside asm.
-// With the density gradient the blur's term is two products, t0 = (w[E] * x) * vol[E].
-template <int E, int D, bool DG>
-__device__ __forceinline__ void bcast_products(float w, float vol, float g0, float g1, float g2, float x, float diff,
-                                               float& t0, float& t1, float& t2, float& t3) {
-    if constexpr (D == 2 && DG) {
-        asm volatile("s_nop %c9\n\t"
-                     "v_mul_f32_dpp %0, %3, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %1, %5, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %2, %6, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %0, %4, %0 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
-                     : "=&v"(t0), "=&v"(t1), "=&v"(t2)
-                     : "v"(w), "v"(vol), "v"(g0), "v"(g1), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
-        t3 = 0.0f;
-        (void)g2;
-    } else if constexpr (DG) {
-        asm volatile("s_nop %c11\n\t"
-                     "v_mul_f32_dpp %0, %4, %9 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %1, %6, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %2, %7, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %3, %8, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
-                     "v_mul_f32_dpp %0, %5, %0 row_newbcast:%c12 row_mask:0xf bank_mask:0xf"
-                     : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
-                     : "v"(w), "v"(vol), "v"(g0), "v"(g1), "v"(g2), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
-    } else if constexpr (D == 2) {
+template <int E, int D>
+__device__ __forceinline__ void bcast_products(float w, float g0, float g1, float g2, float x, float diff, float& t0,
+                                               float& t1, float& t2, float& t3) {
+    if constexpr (D == 2) {
         asm volatile("s_nop %c8\n\t"
                      "v_mul_f32_dpp %0, %3, %6 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n\t"
                      "v_mul_f32_dpp %1, %4, %7 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n\t"
@@ -257,6 +237,33 @@ __device__ __forceinline__ void bcast_products(float w, float vol, float g0, flo
                      "v_mul_f32_dpp %3, %7, %9 row_newbcast:%c11 row_mask:0xf bank_mask:0xf"
                      : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
                      : "v"(w), "v"(g0), "v"(g1), "v"(g2), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
+    }
+}
+
+// With the density gradient the blur's term is two products, t0 = (smooth[E] * x) * vol[E].
+template <int E, int D>
+__device__ __forceinline__ void bcast_products_dg(float smooth, float vol, float g0, float g1, float g2, float x,
+                                                  float diff, float& t0, float& t1, float& t2, float& t3) {
+    if constexpr (D == 2) {
+        asm volatile("s_nop %c9\n\t"
+                     "v_mul_f32_dpp %0, %3, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %1, %5, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %2, %6, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %0, %4, %0 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
+                     : "=&v"(t0), "=&v"(t1), "=&v"(t2)
+                     : "v"(smooth), "v"(vol), "v"(g0), "v"(g1), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1), "n"(E));
+        t3 = 0.0f;
+        (void)g2;
+    } else {
+        asm volatile("s_nop %c11\n\t"
+                     "v_mul_f32_dpp %0, %4, %9 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %1, %6, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %2, %7, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %3, %8, %10 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n\t"
+                     "v_mul_f32_dpp %0, %5, %0 row_newbcast:%c12 row_mask:0xf bank_mask:0xf"
+                     : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+                     : "v"(smooth), "v"(vol), "v"(g0), "v"(g1), "v"(g2), "v"(x), "v"(diff), "n"(E == 0 ? 4 : 1),
+                       "n"(E));
     }
 }
 
@@ -509,8 +516,10 @@ __global__ __launch_bounds__(1024) void k_update_fused(StepParams P, const float
                             const float x = sv[e];
                             const float diff = x - si;
                             float t0, t1, t2, t3;
-                            bcast_products<e, D, Sh::DG>(Sh::DG ? smooth : w, vol, vg[0], vg[1], vg[2], x, diff, t0, t1,
-                                                         t2, t3);
+                            if constexpr (Sh::DG)
+                                bcast_products_dg<e, D>(smooth, vol, vg[0], vg[1], vg[2], x, diff, t0, t1, t2, t3);
+                            else
+                                bcast_products<e, D>(w, vg[0], vg[1], vg[2], x, diff, t0, t1, t2, t3);
                             blur += t0;  // blur_state forward.rs:174-180 (x * w), second_pass_particle 263-270
                             gr[0] += t1;  // compute_state_gradient forward.rs:297-333 (diff * grad)
                             gr[1] += t2;
