@@ -354,7 +354,7 @@ def bench_raster(args, torch) -> int:
                    "particles": n, "image_size": size, "coverage": coverage},
         "roofline": {"bound": "mfma", "achieved": None, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": None, "traffic": None,
-                     "kernel": "raster pipeline (prep + depth sort + scans + emit + tile sort + tiles)",
+                     "kernel": "raster pipeline (prep + depth sort + tile groups' lists + tiles)",
                      "engine": "fp32 VALU; exp counted as one operation",
                      "mean_launch_ms": pipe_ms,
                      "timing": "HIP events around the raster pipeline of every timed call, on the "
@@ -432,7 +432,7 @@ def bench_adjoint(args, torch) -> int:
                    "particles": n, "pairs": pairs, "outputs_finite": finite},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": None,
-                     "kernel": "whole call (hashgrid build + k_adj_density, k_adj_prep, k_adj_gather, "
+                     "kernel": "whole call (hashgrid build + density pass, k_adj_prep, k_adj_gather, "
                                "k_adj_density_kernel)",
                      "engine": "fp32 VALU", "mean_launch_ms": ms, "flops_per_launch": flops,
                      "timing": "wall clock over the timed calls (synchronised on both sides)"},
