@@ -432,16 +432,22 @@ hipError_t launch_segments(const Segments& g, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Whether a kernel on the context's device may read or write the caller's array: memory of that device.
-// Anything else (host-I/O mode, another GPU's memory, host memory) is copied by the runtime.
-bool kernel_reachable(const npa_context* ctx, const void* p) {
-    if (ctx->host_io) return false;
+// Whether a kernel on the context's device may read or write the caller's array: `bytes` of one
+// allocation of that device, on a word boundary. Anything else (host-I/O mode, another GPU's memory, host
+// memory, an odd address, an array that ends before `bytes`) is left to the runtime's copy, which takes
+// or refuses it.
+bool kernel_reachable(const npa_context* ctx, const void* p, uint64_t bytes) {
+    if (ctx->host_io || (reinterpret_cast<uintptr_t>(p) & 3)) return false;
     hipPointerAttribute_t attr{};
-    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess || attr.type != hipMemoryTypeDevice ||
+        attr.device != ctx->device || hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
         (void)hipGetLastError();  // not an address the runtime knows
         return false;
     }
-    return attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
+    const size_t at = (size_t)(static_cast<const char*>(p) - static_cast<const char*>(base));
+    return at <= size && bytes <= size - at;
 }
 
 // Lays out a model's weights for its step kernel: from the caller's arrays, or through the state's
@@ -454,7 +460,7 @@ hipError_t pad_state_weights(npa_state* s, const npa_weights* w, const npa::Step
     const uint64_t sizes[4] = {H * F, H, O * H, O};
     const float* arrays[4] = {w1, b1, w2, b2};
     bool direct = true;
-    for (int k = 0; k < 4; ++k) direct = direct && (!sizes[k] || kernel_reachable(ctx, arrays[k]));
+    for (int k = 0; k < 4; ++k) direct = direct && (!sizes[k] || kernel_reachable(ctx, arrays[k], sizes[k] * 4));
     if (!direct) {
         float* at = s->staged_weights.as<float>();
         auto stage = [&](const float*& src, uint64_t n) {
@@ -1260,9 +1266,9 @@ npa_status npa_state_create(npa_context* ctx, const npa_model_cfg* model, const 
         }
         Segments g;
         const hipMemcpyKind kind = ctx->host_io ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-        if (kernel_reachable(ctx, positions)) g.add(s->pos[0].ptr, positions, total * 4);
+        if (kernel_reachable(ctx, positions, total * 16)) g.add(s->pos[0].ptr, positions, total * 4);
         else e = hipMemcpyAsync(s->pos[0].ptr, positions, total * 16, kind, ctx->stream);
-        if (kernel_reachable(ctx, states)) g.add(s->states[0].ptr, states, total * S);
+        if (kernel_reachable(ctx, states, total * S * 4)) g.add(s->states[0].ptr, states, total * S);
         else if (e == hipSuccess) e = hipMemcpyAsync(s->states[0].ptr, states, total * S * 4, kind, ctx->stream);
         g.add(s->density.ptr, nullptr, total);
         g.add(s->ws.bin_count.ptr, nullptr, s->ws.bin_count.bytes / 4);
@@ -1349,7 +1355,7 @@ npa_status npa_state_read(npa_state* s, float* positions, float* states, float* 
     Segments g;
     auto read = [&](float* dst, const DevBuf& src, uint64_t words) {
         if (!dst) return hipSuccess;
-        if (!kernel_reachable(ctx, dst)) return hipMemcpyAsync(dst, src.ptr, words * 4, kind, ctx->stream);
+        if (!kernel_reachable(ctx, dst, words * 4)) return hipMemcpyAsync(dst, src.ptr, words * 4, kind, ctx->stream);
         g.add(dst, src.ptr, words);
         return hipSuccess;
     };

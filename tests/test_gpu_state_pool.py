@@ -116,3 +116,24 @@ def test_weights_staged_after_a_mode_change():
     a.close()
     b.close()
     ctx.close()
+
+
+def test_read_into_an_odd_address():
+    """A destination off the word boundary goes through the runtime's copy, one on it through the library's kernel."""
+    from burn_automata_amd._lib import lib
+
+    w = syn.workload("c1", particles=700)
+    ctx = Context()
+    ex = HipAutomataExecutor(ctx=ctx)
+    s = ex.create_state(NpaModel(w["model"], w["weights"]), w["positions"], w["states"], 1, w["n"], w["grid"], 1.0, 0.5, 7)
+    ex.step_state_many(s, 2)
+    want = to_np(ex.read_state(s)[2])
+    for offset in (1, 2, 4):
+        buf = torch.zeros(4 * w["n"] + 8, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        ctx.check(lib().npa_state_read(s.handle, None, None, buf.data_ptr() + offset))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(buf[offset: offset + 4 * w["n"]].cpu().numpy().view(np.float32), want)
+        assert not buf[4 * w["n"] + offset:].any() and not buf[:offset].any()
+    s.close()
+    ctx.close()
