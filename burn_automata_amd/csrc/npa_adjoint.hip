@@ -152,12 +152,16 @@ struct AdjPair {
         }
         x = g.eps2 - r2;
         const bool ok = other && r2 > 0.0f;
-        // r and 1 / r from the hardware's reciprocal square root, each refined once
-        const float z = ok ? r2 : 1.0f;
+        // r and 1 / r from the hardware's reciprocal square root, each refined once. It takes a subnormal
+        // for zero, so the squares of distances below 2^-50 are scaled by 2^64, exactly, around it.
+        const bool tiny = r2 < 0x1p-100f;
+        const float z = ok ? (tiny ? r2 * 0x1p64f : r2) : 1.0f;
         float y = __builtin_amdgcn_rsqf(z);
         y = fmaf(0.5f * y, fmaf(-z * y, y, 1.0f), y);
         const float w = z * y;
         r = fmaf(fmaf(-w, w, z), 0.5f * y, w);
+        r = tiny ? r * 0x1p-32f : r;
+        y = tiny ? y * 0x1p32f : y;
         ir = y;
         const float t = g.eps - r, k = ok ? 3.0f * g.k5 : 0.0f;
         f = k * (t * t);

@@ -49,3 +49,31 @@ def test_adjoint_shapes_match_the_oracle(ctx, name):
     again = K.perceive_adjoint_with_options(pos, st, batch, n, S, cfg, opts, fa, ctx=ctx)
     np.testing.assert_array_equal(to_np(again.state), to_np(got.state))
     np.testing.assert_array_equal(to_np(again.position), to_np(got.position))
+
+
+@pytest.mark.parametrize("dim,S", [(2, 16), (3, 5)])
+def test_nearly_coincident_particles(ctx, dim, S):
+    """Pairs from exactly coincident to 1e-15 apart, next to the origin, the squares of whose distances are
+    subnormal or vanish. Below 1.5e-17 the oracle's position terms overflow in 32 bits; its state adjoint does not."""
+    cfg = HashGridConfig(dim, Boundary.Clamped, HashGridMode.Particle, (8, 8, 8 if dim == 3 else 1), 0.25, 32)
+    rng = np.random.default_rng(S)
+    gaps = [0.0, 1e-30, 2e-23, 5e-23, 3e-20, 1e-19, 1.2e-19, 5e-18, 1e-16, 1e-15]
+    B, N = len(gaps), 8  # one system per pair: its particles at 0 and at the gap, and six others around them
+    pos = np.zeros((B, N, 4), f32)
+    pos[:, 2:, :dim] = rng.uniform(-0.2, 0.2, (B, N - 2, dim))
+    pos[:, 1, 0] = gaps
+    pos = pos.reshape(B * N, 4)
+    st = rng.normal(0, 0.5, B * N * S).astype(f32)
+    opts = PerceptionOptions(state_grad=True, density_grad=True, eps0=0.25, hybrid_state_gradient=True,
+                             log_norm_grad=False, log_norm_density_grad=False, position_features=False)
+    fa = rng.normal(0, 0.1, B * N * opts.feature_dims(S, dim)).astype(f32)
+    want = O.perceive_adjoint_with_options(pos, st, B, N, S, cfg, opts, fa)
+    got = K.perceive_adjoint_with_options(pos, st, B, N, S, cfg, opts, fa, ctx=ctx)
+    ws, gs = np.asarray(want.state).reshape(B, -1), to_np(got.state).reshape(B, -1)
+    wp, gp = np.asarray(want.position).reshape(B, -1), to_np(got.position).reshape(B, -1)
+    assert np.isfinite(ws).all() and np.isfinite(gs).all() and np.isfinite(gp).all()
+    for k in range(B):
+        es = rel_err(gs[k], ws[k])
+        ep = rel_err(gp[k], wp[k]) if np.isfinite(wp[k]).all() else 0.0
+        print(f"gap {gaps[k]:.1e}: state {es:.2e}, position {ep:.2e}")
+        assert es <= TOL and ep <= TOL
