@@ -215,6 +215,7 @@ __device__ __forceinline__ void append_accepted(const StepParams& P, const float
                                                 uint32_t b, const float* pi, const int* ci, uint32_t lane, uint32_t t,
                                                 uint32_t q, Lists& lists, uint32_t& cnt, Flush&& flush) {
     constexpr uint32_t MAXC = max_chunks(D), CAP = Lists::CAP;
+    static_assert(CAP >= (uint32_t)kNbChunk, "an emptied list takes a whole chunk");
     const uint64_t my_residue = residue_mask<L>(q);
     // Phase A. The density pass recorded each target's accepted candidates per chunk, in visit
     // order; the lists are built from those masks (RB chunk records loaded per batch).

@@ -55,10 +55,12 @@ namespace npa {
 // sum is unchanged.
 constexpr int kChunk = kNbChunk;
 
-// Lanes per target for a sorted-state row width SM (each lane owns SM / L state channels).
+// Lanes per target for a sorted-state row width SM (each lane owns SM / L state channels). Two lanes
+// also for the narrowest rows: a chunk's 64 accepted candidates have to fit a target's list, which 64
+// targets a wave would leave 48 entries.
 template <int SM>
 struct LanesPerTarget {
-    static constexpr int L = SM >= 16 ? 4 : SM / 4;
+    static constexpr int L = SM >= 16 ? 4 : 2;
     static constexpr int CPL = SM / L;
 };
 

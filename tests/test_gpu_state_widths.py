@@ -70,3 +70,29 @@ def test_rollout_state_width(ctx, name):
     # clamped) exactly: the rollout is the oracle's bit for bit
     np.testing.assert_array_equal(to_np(gp), want_p)
     np.testing.assert_array_equal(to_np(gs), want_s)
+
+
+@pytest.mark.parametrize("dim,S,n,side", [(2, 4, 90, 0.1), (2, 1, 300, 0.1), (3, 3, 200, 0.08), (2, 3, 2500, 0.5),
+                                          (3, 2, 1800, 0.2)])
+def test_narrow_rows_of_crowded_cells(ctx, dim, S, n, side):
+    """State rows of one float4 where whole chunks of 64 candidates are accepted: with the chunks recorded
+    by the density pass, and with more of them than it records."""
+    from burn_automata_amd.config import Boundary, HashGridMode
+    g = HashGridConfig(dim, Boundary.Clamped, HashGridMode.Particle, (16, 16, 16 if dim == 3 else 1), 0.25, 32)
+    m = NpaConfig(spatial_dims=dim, state_dims=S, hidden_dims=32, density_grad=dim == 2)
+    rng = np.random.default_rng(n)
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :dim] = 0.125 + rng.uniform(-side / 2, side / 2, (n, dim))
+    st = syn.normal_states(n, S, n)
+    want = O.perceive_with_options(pos, st, 1, n, S, g, m.perception_options())
+    got = K.perceive_with_options(pos, st, 1, n, S, g, m.perception_options(), ctx=ctx)
+    np.testing.assert_array_equal(to_np(got.density), want.density)
+    for field in ("features", "blurred_state", "state_gradient", "density_gradient"):
+        if getattr(want, field) is not None and np.size(getattr(want, field)):
+            e = rel_err(getattr(got, field), getattr(want, field))
+            assert e <= STEP_TOL, f"{field}: {e}"
+    w = syn.seeded_weights(m, 3)
+    ref = O.step(m, w, pos, st, 1, n, g, 1.0, None)
+    res = NpaModel(m, w).step(pos, st, 1, n, g, 1.0, ctx=ctx)
+    np.testing.assert_array_equal(to_np(res.next_positions), ref.next_positions)
+    np.testing.assert_array_equal(to_np(res.next_states), ref.next_states)
