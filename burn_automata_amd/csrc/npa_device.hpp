@@ -202,13 +202,18 @@ __device__ __forceinline__ uint32_t cell_of_coords(const int64_t c[3], const Gri
 // neighbor_delta  hashgrid.rs:165-181, component a.
 // Branch-free: both wrapped candidates are computed and one is selected (same values as the
 // reference's if / else-if, NaN included).
-__device__ __forceinline__ float delta_axis(float pi, float pj, int a, const GridParams& g) {
+template <bool PERIODIC>
+__device__ __forceinline__ float delta_axis_as(float pi, float pj, int a, const GridParams& g) {
     const float v = pj - pi;
-    if (g.boundary == 0) {  // wave-uniform
+    if constexpr (PERIODIC) {
         const float up = v - g.extent[a], dn = v + g.extent[a];
         return v > g.half[a] ? up : (v < -g.half[a] ? dn : v);
     }
     return v;
+}
+__device__ __forceinline__ float delta_axis(float pi, float pj, int a, const GridParams& g) {
+    if (g.boundary == 0) return delta_axis_as<true>(pi, pj, a, g);  // wave-uniform
+    return pj - pi;
 }
 
 // smoothing_poly6_kernel  crates/burn_automata_kernels/src/reference/kernels.rs:51-58

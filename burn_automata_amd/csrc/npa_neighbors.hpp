@@ -275,43 +275,50 @@ __device__ __forceinline__ void append_accepted(const StepParams& P, const float
             for (uint32_t base = beg; base < end; base += kNbChunk) {
                 const uint32_t m = end - base < (uint32_t)kNbChunk ? end - base : (uint32_t)kNbChunk;
                 // batches of 4 candidates per lane: loads first (index clamped to
-                // the chunk, so every load is in bounds), then branch-free tests
+                // the chunk, so every load is in bounds), then branch-free tests. The boundary and the
+                // bin's filter are chosen per chunk: tested by candidate the compiler turns both into
+                // selects for every one of them (a dense 2D cloud's second pass 1,122 -> 1,220 us).
                 uint64_t acc = 0;
-                for (int i0 = 0; i0 < kNbChunk / L; i0 += 4) {
-                    if ((uint32_t)(i0 * L) >= m) break;  // wave-uniform
-                    float4 rc[4];
-                    int4 cc[4];
+                auto tests = [&](auto periodic, auto filtered) {
+#pragma unroll 1
+                    for (int i0 = 0; i0 < kNbChunk / L; i0 += 4) {
+                        if ((uint32_t)(i0 * L) >= m) break;  // wave-uniform
+                        float4 rc[4];
+                        int4 cc[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const uint32_t k = q + (uint32_t)((i0 + u) * L);
-                        const uint32_t kc = k < m ? k : m - 1;
-                        rc[u] = srec[base + kc];
-                        if constexpr (D == 3) cc[u] = scoord[base + kc];
-                    }
+                        for (int u = 0; u < 4; ++u) {
+                            const uint32_t k = q + (uint32_t)((i0 + u) * L);
+                            const uint32_t kc = k < m ? k : m - 1;
+                            rc[u] = srec[base + kc];
+                            if constexpr (D == 3 && filtered) cc[u] = scoord[base + kc];
+                        }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const uint32_t k = q + (uint32_t)((i0 + u) * L);
-                        const float4 r = rc[u];
-                        bool ok = in_group & (k < m);
-                        if (filter) {
-                            if constexpr (D == 2) {
-                                ok = ok & ((int64_t)__float_as_int(r.z) == n0) &
-                                     ((int64_t)__float_as_int(r.w) == n1);
-                            } else {
-                                ok = ok & ((int64_t)cc[u].x == n0) & ((int64_t)cc[u].y == n1) &
-                                     ((int64_t)cc[u].z == n2);
+                        for (int u = 0; u < 4; ++u) {
+                            const uint32_t k = q + (uint32_t)((i0 + u) * L);
+                            const float4 r = rc[u];
+                            bool ok = in_group & (k < m);
+                            if constexpr (filtered && D == 2)
+                                ok = ok & ((int64_t)__float_as_int(r.z) == n0) & ((int64_t)__float_as_int(r.w) == n1);
+                            if constexpr (filtered && D == 3)
+                                ok = ok & ((int64_t)cc[u].x == n0) & ((int64_t)cc[u].y == n1) & ((int64_t)cc[u].z == n2);
+                            const float d0 = delta_axis_as<periodic>(pi[0], r.x, 0, P.g);
+                            const float d1 = delta_axis_as<periodic>(pi[1], r.y, 1, P.g);
+                            float r2 = d0 * d0;
+                            r2 += d1 * d1;
+                            if constexpr (D == 3) {
+                                const float d2 = delta_axis_as<periodic>(pi[2], r.z, 2, P.g);
+                                r2 += d2 * d2;
                             }
+                            acc |= (ok & (r2 < P.g.eps2)) ? (1ull << (k & 63u)) : 0ull;
                         }
-                        const float d0 = delta_axis(pi[0], r.x, 0, P.g);
-                        const float d1 = delta_axis(pi[1], r.y, 1, P.g);
-                        float r2 = d0 * d0;
-                        r2 += d1 * d1;
-                        if constexpr (D == 3) {
-                            const float d2 = delta_axis(pi[2], r.z, 2, P.g);
-                            r2 += d2 * d2;
-                        }
-                        acc |= (ok & (r2 < P.g.eps2)) ? (1ull << (k & 63u)) : 0ull;
                     }
+                };
+                if (P.g.boundary == 0) {
+                    if (filter) tests(std::true_type{}, std::true_type{});
+                    else tests(std::true_type{}, std::false_type{});
+                } else {
+                    if (filter) tests(std::false_type{}, std::true_type{});
+                    else tests(std::false_type{}, std::false_type{});
                 }
                 acc = group_or<L>(acc);
                 const uint32_t add = (uint32_t)__popcll(acc);

@@ -96,3 +96,26 @@ def test_narrow_rows_of_crowded_cells(ctx, dim, S, n, side):
     res = NpaModel(m, w).step(pos, st, 1, n, g, 1.0, ctx=ctx)
     np.testing.assert_array_equal(to_np(res.next_positions), ref.next_positions)
     np.testing.assert_array_equal(to_np(res.next_states), ref.next_states)
+
+
+@pytest.mark.parametrize("dim,boundary,mode,gs,eps,n,side", [
+    (2, "Periodic", "Grid", 5, 0.2, 3500, 0.99), (2, "Clamped", "Grid", 4, 0.2, 3000, 0.7),
+    (2, "Clamped", "Particle", 2, 0.5, 4000, 6.0), (3, "Clamped", "Particle", 2, 0.5, 7000, 4.0),
+    (3, "Periodic", "Grid", 4, 0.25, 6000, 0.99), (3, "Clamped", "Particle", 8, 0.3, 5000, 0.8)])
+def test_candidates_tested_by_boundary_and_filter(ctx, dim, boundary, mode, gs, eps, n, side):
+    """More chunks than the density pass records, so the second pass tests the candidates itself: over both
+    boundaries, for cells with runs of their own and for bins that several cells share."""
+    from burn_automata_amd.config import Boundary, HashGridMode
+    g = HashGridConfig(dim, getattr(Boundary, boundary), getattr(HashGridMode, mode), (gs, gs, gs if dim == 3 else 1), eps, 32)
+    S = 6
+    m = NpaConfig(spatial_dims=dim, state_dims=S, hidden_dims=24, density_grad=True)
+    rng = np.random.default_rng(n)
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :dim] = rng.uniform(-side / 2, side / 2, (n, dim))
+    st = syn.normal_states(n, S, n)
+    want = O.perceive_with_options(pos, st, 1, n, S, g, m.perception_options())
+    got = K.perceive_with_options(pos, st, 1, n, S, g, m.perception_options(), ctx=ctx)
+    np.testing.assert_array_equal(to_np(got.density), want.density)
+    for field in ("features", "blurred_state", "state_gradient", "density_gradient"):
+        e = rel_err(getattr(got, field), getattr(want, field))
+        assert e <= STEP_TOL, f"{field}: {e}"
