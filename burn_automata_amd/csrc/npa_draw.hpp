@@ -13,7 +13,7 @@ struct alignas(16) DrawItem {  // 48 bytes
     float c[3], depth;
     int x0, y0;
     uint32_t span;
-    uint32_t special;  // a value is not finite: drawn pixel by pixel
+    uint32_t special;  // a value, or a product of scale and a channel, is not finite: drawn pixel by pixel
 };
 
 // The window's 16x16 tiles an item touches (pairs of them, where an axis has more than 127), as four
@@ -72,8 +72,11 @@ __device__ __forceinline__ Footprint draw_footprint(float px, float py, float k2
     const uint32_t rect = draw_rect((uint32_t)x0 >> sh, (uint32_t)x1 >> sh, (uint32_t)y0 >> sh, (uint32_t)y1 >> sh);
     return {rect, axis_weights(px, k2, (int)x0, (int)x1) * axis_weights(py, k2, (int)y0, (int)y1)};
 }
+// Whether the item can be drawn as matrix products: its values are finite, and so is every operand
+// (e(y) scale) c, which scale * c bounds (an infinite one would meet the zeros outside the footprint).
 __device__ __forceinline__ bool draw_finite(const DrawItem& d) {
-    return isfinite(d.px) && isfinite(d.py) && isfinite(d.k2) && isfinite(d.scale) && isfinite(d.c[0]) && isfinite(d.c[1]) &&
+    return isfinite(d.px) && isfinite(d.py) && isfinite(d.k2) && isfinite(d.scale) && isfinite(d.scale * d.c[0]) &&
+           isfinite(d.scale * d.c[1]) && isfinite(d.scale * d.c[2]) && isfinite(d.c[0]) && isfinite(d.c[1]) &&
            isfinite(d.c[2]) && isfinite(d.depth);
 }
 

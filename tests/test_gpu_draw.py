@@ -82,3 +82,37 @@ def test_non_finite_values_stay_in_their_footprint(ctx):
     np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
     fin = np.isfinite(want)
     assert np.max(np.abs(got[fin] - want[fin])) <= TOL * np.max(np.abs(want[fin]))
+
+
+def test_huge_finite_colours_stay_in_their_footprint(ctx):
+    """Finite colours whose product with the particle's scale overflows, where the footprint is all but outside the
+    image or falls between the pixels: finite in its own pixels, and nothing in any other."""
+    pos, col, op, sg = _particles(60, 4, 0.9)
+    size = 64
+    px = lambda p: f32(2 * p / (size - 1) - 1)  # noqa: E731  (the inverse of the splat's pixel coordinates)
+    pos[3, :2] = px(-3.6), px(size + 2.6)
+    pos[4, :2] = px(20.0), px(-3.7)
+    pos[5, :2] = px(size + 2.7), px(33.0)
+    col[3], col[4, 1], col[5] = (1e31, 2e31, -1e31), 3e38, -3e38
+    cfg = Splat2dConfig(image_size=size, sigma=0.8, pixel_size=2.0 / size)
+    cfg_n = Splat2dConfig(image_size=size, sigma=0.1, pixel_size=2.0 / size)
+    pos2, col2 = pos.copy(), col.copy()
+    pos2[7, :2] = px(40.5), px(17.5)
+    col2[7] = 1e32
+    for p, c, cf in ((pos, col, cfg), (pos2, col2, cfg_n)):
+        got = to_np(K.splat_particles_2d(p, c, cf, ctx=ctx))
+        want = to_np(O.splat_particles_2d(p, c, cf)).reshape(got.shape)
+        assert np.isfinite(want).all() and np.isfinite(got).all()
+        for ch in range(4):
+            g, w = got[..., ch].astype(np.float64), want[..., ch].astype(np.float64)
+            np.testing.assert_allclose(g, w, rtol=2e-4, atol=1e-4)
+    rc = RenderLossConfig(image_size=size)
+    rpos, rcol = pos.copy(), col.copy()
+    rpos[3, :2] = rc.world_scale * 1.13, -rc.world_scale * 1.13
+    rcol[4], rcol[5] = 0.5, 0.5
+    rcol[3] = 1e35
+    got = to_np(K.render_views(rpos, rcol, op, np.full_like(sg, 0.9), rc, (0,), ctx=ctx))[0]
+    want = O.splat_projected(O.project_positions(0, rpos, rc.world_scale), rcol, op, np.full_like(sg, 0.9), rc)
+    want = to_np(want).reshape(got.shape)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    np.testing.assert_allclose(got.astype(np.float64), want.astype(np.float64), rtol=2e-4, atol=1e-4)
