@@ -53,7 +53,6 @@ struct npa_context {
     std::mutex pool_mutex;
     std::vector<Block> pool;
     size_t pool_bytes = 0;
-    std::atomic<uint32_t> stream_changes{0};  // npa_context_set_stream calls that changed the stream
     hipError_t block_acquire(size_t bytes, Block* out);
     void block_release(Block b);
     void pool_clear();
@@ -79,7 +78,6 @@ struct npa_state {
     uint64_t step_index = 0;
     int mlp_engine = NPA_MLP_VALU;
     npa_context::Block block{};              // one allocation; the buffers below and ws are views into it
-    uint32_t stream_changes = 0;             // the context's count when the state was created
     bool exposed = false;                    // npa_state_buffers handed out its addresses
     DevBuf pos[2], states[2], density, staged_weights;
     int cur = 0;
@@ -529,7 +527,6 @@ void npa_context_destroy(npa_context* ctx) {
 
 npa_status npa_context_set_stream(npa_context* ctx, void* stream) {
     if (!ctx) return NPA_ERR_INVALID_ARGUMENT;
-    if (ctx->stream != (hipStream_t)stream) ctx->stream_changes.fetch_add(1);
     ctx->stream = (hipStream_t)stream;
     return NPA_OK;
 }
@@ -1239,7 +1236,6 @@ npa_status npa_state_create(npa_context* ctx, const npa_model_cfg* model, const 
     s->seed = seed;
     s->plan = plan;
     s->grid_blocks = grid_blocks_for(ctx, plan);
-    s->stream_changes = ctx->stream_changes.load();
     const uint32_t S = model->state_dims, F = model_perception_dims(*model), H = model->hidden_dims;
     const uint32_t O = model->spatial_dims + S;
     const npa::StepParams sp = [&] {
@@ -1293,14 +1289,14 @@ void npa_state_destroy(npa_state* s) {
     if (!s) return;
     npa_context* ctx = s->ctx;
     (void)hipSetDevice(ctx->device);
-    (void)hipStreamSynchronize(ctx->stream);
-    if (s->exposed) {
-        // others may hold the addresses and have work on streams of their own: hipFree waits for it
-        (void)hipFree(s->block.ptr);
-    } else {
-        // a state that ran on another stream as well waits for that one too before its block is reused
-        if (s->stream_changes != ctx->stream_changes.load()) (void)hipDeviceSynchronize();
+    // As freeing it would, wait for everything queued on the device before the block can be another
+    // state's: work of this state may be on streams that the context was never given (a captured step
+    // replayed elsewhere).
+    if (hipDeviceSynchronize() == hipSuccess && !s->exposed) {
         ctx->block_release(s->block);
+    } else {
+        (void)hipGetLastError();
+        (void)hipFree(s->block.ptr);  // others hold its addresses, or the wait was refused
     }
     delete s;
     context_release(ctx);

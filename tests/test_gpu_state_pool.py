@@ -137,3 +137,35 @@ def test_read_into_an_odd_address():
         assert not buf[4 * w["n"] + offset:].any() and not buf[:offset].any()
     s.close()
     ctx.close()
+
+
+def test_destroy_waits_for_work_on_other_streams():
+    """A state's captured step, replayed on a stream that the context was never given, has finished when the state is
+    destroyed: its block may be the next state's."""
+    w = syn.workload("c1", particles=4096)
+    ref = _fresh(w, 8)
+    ctx = Context()
+    ex = HipAutomataExecutor(ctx=ctx)
+    m = NpaModel(w["model"], w["weights"])
+    make = lambda: ex.create_state(m, w["positions"], w["states"], 1, w["n"], w["grid"], 1.0, 0.5, 7)  # noqa: E731
+    capture, other = torch.cuda.Stream(), torch.cuda.Stream()
+    ctx.set_stream(capture.cuda_stream)
+    s = make()
+    ex.step_state_many(s, 2)  # eager, outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=capture):
+        ex.step_state_many(s, 2)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        for _ in range(500):  # about 40 ms of steps
+            graph.replay()
+    queued = not other.query()
+    s.close()
+    assert queued and other.query()
+    t = make()
+    ex.step_state_many(t, 8)
+    for x, y in zip(ex.read_state(t), ref):
+        np.testing.assert_array_equal(to_np(x), y)
+    t.close()
+    ctx.close()
