@@ -45,19 +45,8 @@ struct npa_context {
     std::atomic<bool> used_noalloc{false};
     // the caller's handle plus one per live npa_state: a state keeps its context until it is destroyed
     std::atomic<int> refs{1};
-    // Device blocks of destroyed states, for the next ones: a rollout of 64 x 4,096 particles spent more
-    // time in the allocation and release of its 118 MB state than in 16 steps (6.0 ms a call, 2.8 ms of it kernels).
-    // Bounded (kPoolBlocks blocks, kPoolBytes in all), given back when an allocation fails and with the
-    // context, locked because states may be destroyed on any thread.
-    struct Block { void* ptr; size_t bytes; };
-    std::mutex pool_mutex;
-    std::vector<Block> pool;
-    size_t pool_bytes = 0;
-    hipError_t block_acquire(size_t bytes, Block* out);
-    void block_release(Block b);
-    void pool_clear();
+    npa::DeviceBlocks blocks;  // of destroyed states, for the next ones
     ~npa_context() {
-        pool_clear();
         ws.release();
         splat_ws.release();
         adj_ws.release();
@@ -77,7 +66,7 @@ struct npa_state {
     uint64_t seed = 0;
     uint64_t step_index = 0;
     int mlp_engine = NPA_MLP_VALU;
-    npa_context::Block block{};              // one allocation; the buffers below and ws are views into it
+    npa::DeviceBlocks::Block block{};              // one allocation; the buffers below and ws are views into it
     bool exposed = false;                    // npa_state_buffers handed out its addresses
     DevBuf pos[2], states[2], density, staged_weights;
     int cur = 0;
@@ -87,57 +76,6 @@ struct npa_state {
     int grid_blocks = 1;
     ~npa_state() { splat_ws.release(); }
 };
-
-constexpr size_t kPoolBlocks = 4, kPoolBytes = (size_t)1 << 30;
-
-void npa_context::pool_clear() {
-    std::lock_guard<std::mutex> lock(pool_mutex);
-    for (const Block& b : pool) (void)hipFree(b.ptr);
-    pool.clear();
-    pool_bytes = 0;
-}
-
-// The smallest kept block that fits without wasting more than its need again, else a new one.
-hipError_t npa_context::block_acquire(size_t bytes, Block* out) {
-    constexpr size_t kGrain = (size_t)2 << 20;
-    const size_t want = (bytes + kGrain - 1) / kGrain * kGrain;
-    {
-        std::lock_guard<std::mutex> lock(pool_mutex);
-        size_t best = pool.size();
-        for (size_t k = 0; k < pool.size(); ++k)
-            if (pool[k].bytes >= want && pool[k].bytes <= 2 * want && (best == pool.size() || pool[k].bytes < pool[best].bytes))
-                best = k;
-        if (best < pool.size()) {
-            *out = pool[best];
-            pool_bytes -= out->bytes;
-            pool.erase(pool.begin() + (ptrdiff_t)best);
-            return hipSuccess;
-        }
-    }
-    *out = Block{nullptr, want};
-    hipError_t e = hipMalloc(&out->ptr, want);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        pool_clear();
-        e = hipMalloc(&out->ptr, want);
-    }
-    if (e != hipSuccess) *out = Block{nullptr, 0};
-    return e;
-}
-
-// No queued work may use the block any more.
-void npa_context::block_release(Block b) {
-    if (!b.ptr) return;
-    {
-        std::lock_guard<std::mutex> lock(pool_mutex);
-        if (pool.size() < kPoolBlocks && pool_bytes + b.bytes <= kPoolBytes) {
-            pool.push_back(b);
-            pool_bytes += b.bytes;
-            return;
-        }
-    }
-    (void)hipFree(b.ptr);
-}
 
 namespace {
 
@@ -1251,7 +1189,7 @@ npa_status npa_state_create(npa_context* ctx, const npa_model_cfg* model, const 
     const uint64_t ws_bytes = s->ws.carve(plan, total, B, S, (int)grid->dim, feature_rows_for(sp), wpad_bytes, nullptr, 0);
     uint64_t need_bytes = ws_bytes;
     for (uint64_t n : sizes) need_bytes += (n + 255) / 256 * 256;
-    hipError_t e = ctx->block_acquire(need_bytes, &s->block);
+    hipError_t e = ctx->blocks.acquire(need_bytes, &s->block);
     if (e == hipSuccess) {
         s->ws.carve(plan, total, B, S, (int)grid->dim, feature_rows_for(sp), wpad_bytes, s->block.ptr, ws_bytes);
         s->ws.counters_kept = true;  // cleared below; nobody else writes them
@@ -1293,7 +1231,7 @@ void npa_state_destroy(npa_state* s) {
     // state's: work of this state may be on streams that the context was never given (a captured step
     // replayed elsewhere).
     if (hipDeviceSynchronize() == hipSuccess && !s->exposed) {
-        ctx->block_release(s->block);
+        ctx->blocks.release(s->block);
     } else {
         (void)hipGetLastError();
         (void)hipFree(s->block.ptr);  // others hold its addresses, or the wait was refused

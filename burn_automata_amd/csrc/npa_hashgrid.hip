@@ -33,7 +33,7 @@ hipError_t DevBuf::reserve(size_t want) {
     if (want <= bytes && ptr) return hipSuccess;
     release();
     size_t b = want ? want : 16;
-    hipError_t e = hipMalloc(&ptr, b);
+    hipError_t e = DeviceBlocks::allocate(&ptr, b);
     if (e != hipSuccess) {
         ptr = nullptr;
         bytes = 0;

@@ -11,9 +11,24 @@
 #include <vector>
 
 #include "../../include/npa_abi.h"
+#include "npa_blocks.hpp"
 #include "npa_device.hpp"
 
 namespace npa {
+
+// The device memory of npa_blocks.hpp.
+struct HipMemory {
+    using Error = hipError_t;
+    static Error alloc(void** p, size_t bytes) { return hipMalloc(p, bytes); }
+    static void free(void* p) { (void)hipFree(p); }
+    static bool ok(Error e) { return e == hipSuccess; }
+    static bool out_of_memory(Error e) {
+        if (e != hipErrorOutOfMemory) return false;
+        (void)hipGetLastError();  // the call after the blocks were given back reports it again
+        return true;
+    }
+};
+using DeviceBlocks = BlockPool<HipMemory>;
 
 // Grow-only device allocation, or a view into memory the library does not allocate (view(); never
 // freed).
