@@ -11,8 +11,9 @@ namespace npa {
 
 // Device blocks of one context's destroyed states: a rollout of 64 x 4,096 particles spent more time in the
 // allocation and release of its 118 MB state than in 16 steps (6.0 ms a call, 2.8 ms of it kernels).
-// Bounded (kBlocks blocks, kBytes in all), locked because states may be destroyed on any thread, and given back with
-// the pool and wherever an allocation of this library, through whichever context, finds no memory left (allocate()).
+// Bounded (kBlocks blocks, kBytes in all; the block kept longest goes first), locked because states may be
+// destroyed on any thread, and given back with the pool and wherever an allocation of this library, through
+// whichever context, finds no memory left (allocate()).
 //
 // Mem: Error; Error alloc(void**, size_t); void free(void*); bool ok(Error), out_of_memory(Error).
 template <class Mem>
@@ -72,19 +73,26 @@ class BlockPool {
         return e;
     }
 
-    // Keeps the block for the next acquire, if there is room; no queued work may use it any more.
+    // Keeps the block for the next acquire; no queued work may use it any more.
     void release(Block b) {
         if (!b.ptr) return;
+        std::vector<Block> gone;
         {
             std::lock_guard<std::mutex> lock(mutex_);
-            size_t total = b.bytes;
-            for (const Block& k : kept_) total += k.bytes;
-            if (kept_.size() < kBlocks && total <= kBytes) {
+            if (b.bytes > kBytes) {
+                gone.push_back(b);
+            } else {
+                size_t total = b.bytes;
+                for (const Block& k : kept_) total += k.bytes;
+                while (kept_.size() >= kBlocks || total > kBytes) {  // the oldest: sizes no longer asked for leave
+                    total -= kept_.front().bytes;
+                    gone.push_back(kept_.front());
+                    kept_.erase(kept_.begin());
+                }
                 kept_.push_back(b);
-                return;
             }
         }
-        Mem::free(b.ptr);
+        for (const Block& g : gone) Mem::free(g.ptr);
     }
 
     void clear() {

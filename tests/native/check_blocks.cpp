@@ -110,6 +110,23 @@ static void bounds() {
     CHECK(FakeMemory::used <= Pool::kBytes);
 }
 
+static void oldest_leaves() {  // sizes that are no longer asked for make room
+    FakeMemory::budget = 100000 * MB;
+    Pool pool;
+    Block b[5];
+    for (int k = 0; k < 4; ++k) b[k] = take(pool, (size_t)(k + 1) * 4 * MB);
+    for (int k = 0; k < 4; ++k) pool.release(b[k]);
+    b[4] = take(pool, 200 * MB);
+    pool.release(b[4]);
+    CHECK(FakeMemory::live.size() == 4 && !FakeMemory::live.count(b[0].ptr));
+    CHECK(take(pool, 200 * MB).ptr == b[4].ptr);
+    pool.release(b[4]);
+    Block wide = take(pool, 900 * MB);
+    pool.release(wide);
+    CHECK(FakeMemory::used <= Pool::kBytes && take(pool, 900 * MB).ptr == wide.ptr);
+    pool.release(wide);
+}
+
 static void threads() {
     FakeMemory::budget = 2000 * MB;
     Pool one, two;
@@ -127,7 +144,7 @@ static void threads() {
 }
 
 int main() {
-    for (auto f : {reuse, out_of_memory, bounds, threads}) {
+    for (auto f : {reuse, out_of_memory, bounds, oldest_leaves, threads}) {
         f();
         CHECK(FakeMemory::live.empty() && FakeMemory::used == 0);  // the pools gave everything back
     }
