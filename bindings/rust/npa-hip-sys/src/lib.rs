@@ -214,6 +214,7 @@ extern "C" {
     pub fn npa_context_set_stream(ctx: *mut npa_context, stream: *mut c_void) -> npa_status;
     pub fn npa_context_set_host_io(ctx: *mut npa_context, host_io: c_int) -> npa_status;
     pub fn npa_context_set_mlp_engine(ctx: *mut npa_context, engine: c_int) -> npa_status;
+    pub fn npa_context_trim(ctx: *mut npa_context) -> npa_status;
     pub fn npa_context_synchronize(ctx: *mut npa_context) -> npa_status;
     pub fn npa_last_error(ctx: *const npa_context) -> *const c_char;
     pub fn npa_version() -> *const c_char;

@@ -30,6 +30,7 @@ def _decl(L):
     L.npa_context_set_stream.argtypes = [P, P]
     L.npa_context_set_host_io.argtypes = [P, C.c_int]
     L.npa_context_synchronize.argtypes = [P]
+    L.npa_context_trim.argtypes = [P]
     L.npa_last_error.argtypes = [P]
     L.npa_last_error.restype = C.c_char_p
     L.npa_build_hashgrid.argtypes = [P, P, u32, u32, ptr(_abi.NpaGridCfg), P, sz, P, P, sz]
@@ -86,7 +87,7 @@ def _decl(L):
     L.npa_profile_read.argtypes = [P, C.c_int, ptr(C.c_double), ptr(u64)]
     L.npa_state_pair_counts.argtypes = [P, ptr(u64), ptr(u64), ptr(u64), ptr(u64), ptr(u64)]
     for name in ("npa_context_create", "npa_context_set_stream", "npa_context_set_host_io",
-                 "npa_context_synchronize", "npa_build_hashgrid", "npa_neighbor_lists",
+                 "npa_context_synchronize", "npa_context_trim", "npa_build_hashgrid", "npa_neighbor_lists",
                  "npa_perceive", "npa_mlp_forward", "npa_euler_step", "npa_step",
                  "npa_update_mask", "npa_decode_gaussians_3d", "npa_splat_2d", "npa_state_create",
                  "npa_state_step", "npa_state_read", "npa_state_update_model",
@@ -105,7 +106,7 @@ def _decl(L):
 
 EXPORTED = (
     "npa_context_create", "npa_context_destroy", "npa_context_set_stream", "npa_context_set_host_io",
-    "npa_context_synchronize", "npa_last_error", "npa_version", "npa_build_hashgrid",
+    "npa_context_synchronize", "npa_context_trim", "npa_last_error", "npa_version", "npa_build_hashgrid",
     "npa_neighbor_lists", "npa_perceive", "npa_mlp_forward", "npa_euler_step", "npa_step",
     "npa_update_mask", "npa_decode_gaussians_3d", "npa_splat_2d", "npa_state_create",
     "npa_state_destroy", "npa_state_step", "npa_state_read", "npa_state_update_model",

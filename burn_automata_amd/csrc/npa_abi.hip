@@ -469,6 +469,13 @@ npa_status npa_context_set_stream(npa_context* ctx, void* stream) {
     return NPA_OK;
 }
 
+npa_status npa_context_trim(npa_context* ctx) {
+    if (!ctx) return NPA_ERR_INVALID_ARGUMENT;
+    if (set_device(ctx)) return NPA_ERR_DEVICE;
+    ctx->blocks.clear();
+    return NPA_OK;
+}
+
 npa_status npa_context_set_host_io(npa_context* ctx, int host_io) {
     if (!ctx) return NPA_ERR_INVALID_ARGUMENT;
     ctx->host_io = host_io != 0;

@@ -12,8 +12,8 @@ namespace npa {
 // Device blocks of one context's destroyed states: a rollout of 64 x 4,096 particles spent more time in the
 // allocation and release of its 118 MB state than in 16 steps (6.0 ms a call, 2.8 ms of it kernels).
 // Bounded (kBlocks blocks, kBytes in all; the block kept longest goes first), locked because states may be
-// destroyed on any thread, and given back with the pool and wherever an allocation of this library, through
-// whichever context, finds no memory left (allocate()).
+// destroyed on any thread, and given back with the pool, by clear(), and wherever an allocation of this library,
+// through whichever context, finds no memory left (allocate()).
 //
 // Mem: Error; Error alloc(void**, size_t); void free(void*); bool ok(Error), out_of_memory(Error).
 template <class Mem>

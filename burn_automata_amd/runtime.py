@@ -54,6 +54,10 @@ class Context:
     def synchronize(self):
         self.check(lib().npa_context_synchronize(self.handle))
 
+    def trim(self):
+        """Gives the device memory kept from destroyed states back."""
+        self.check(lib().npa_context_trim(self.handle))
+
     def close(self):
         if getattr(self, "handle", None) is not None and self.handle.value:
             lib().npa_context_destroy(self.handle)

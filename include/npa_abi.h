@@ -195,6 +195,9 @@ npa_status npa_context_set_host_io(npa_context* ctx, int host_io);
 enum { NPA_MLP_VALU = 0, NPA_MLP_MFMA = 1, NPA_MLP_MFMA_BF16 = 2 };
 npa_status npa_context_set_mlp_engine(npa_context* ctx, int engine);
 
+/* Gives the device memory kept from destroyed states (see npa_state_destroy) back, for programs
+ * that share the GPU with other allocators. Workspaces and live states are not touched. */
+npa_status npa_context_trim(npa_context* ctx);
 /* Blocks until all work queued on the context's stream has finished. */
 npa_status npa_context_synchronize(npa_context* ctx);
 /* Message of the last failing call on this context ("" when none). */
@@ -358,6 +361,9 @@ npa_status npa_state_create(npa_context* ctx, const npa_model_cfg* model,
                             const float* positions, const float* states,
                             uint32_t batch_size, uint32_t particle_count, float dt,
                             float update_prob, uint64_t seed, npa_state** out);
+/* Waits for all work queued on the device. The state's memory is kept for the context's next
+ * states (at most four blocks and 1 GiB, without those whose addresses npa_state_buffers gave out)
+ * until a call of this library needs it elsewhere, npa_context_trim or the context's release. */
 void npa_state_destroy(npa_state* state);
 /* step_state / step_state_many (crates/burn_automata/src/gpu/executor/steps.rs:6-69). */
 npa_status npa_state_step(npa_state* state, uint32_t steps);

@@ -169,3 +169,29 @@ def test_destroy_waits_for_work_on_other_streams():
         np.testing.assert_array_equal(to_np(x), y)
     t.close()
     ctx.close()
+
+
+def test_trim_gives_the_kept_memory_back():
+    """The memory of destroyed states, and no live state's, is free again for other allocators after a trim."""
+    w = syn.workload("c2", particles=200000)
+    ctx = Context()
+    ex = HipAutomataExecutor(ctx=ctx)
+    m = NpaModel(w["model"], w["weights"])
+    make = lambda: ex.create_state(m, w["positions"], w["states"], 1, w["n"], w["grid"], 1.0, 0.5, 7)  # noqa: E731
+    live = make()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    a, b = make(), make()
+    two = before - torch.cuda.mem_get_info()[0]
+    assert two > 100 << 20
+    a.close()
+    b.close()
+    kept = before - torch.cuda.mem_get_info()[0]
+    assert kept > two // 2
+    ctx.trim()
+    assert before - torch.cuda.mem_get_info()[0] <= two // 16
+    ex.step_state_many(live, 6)
+    for x, y in zip(ex.read_state(live), _fresh(w)):
+        np.testing.assert_array_equal(to_np(x), y)
+    live.close()
+    ctx.close()
