@@ -499,9 +499,17 @@ hipError_t launch_mlp_forward(const StepParams& p, const float* features, uint32
     const int nw = mlp_waves(p);
     auto k = p.g.dim == 2 ? (nw == 2 ? k_mlp_forward<2, 2> : k_mlp_forward<2, 4>)
                           : (nw == 2 ? k_mlp_forward<3, 2> : k_mlp_forward<3, 4>);
-    hipLaunchKernelGGL(k, dim3((rows - 1) / kMlpRows + 1), dim3(nw * 64), mlp_lds_bytes(p, nw, true), stream, p, features,
-                       rows, RawWeights{io.w1, io.b1, io.w2, io.b2}, dx, ds);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 threads
+    constexpr uint32_t kMost = 1u << 26;
+    for (uint32_t first = 0; first < rows; first += std::min(rows - first, kMost)) {
+        const uint32_t n = std::min(rows - first, kMost);
+        hipLaunchKernelGGL(k, dim3((n - 1) / kMlpRows + 1), dim3(nw * 64), mlp_lds_bytes(p, nw, true), stream, p,
+                           features + (uint64_t)first * p.F, n, RawWeights{io.w1, io.b1, io.w2, io.b2},
+                           dx + 4 * (uint64_t)first, ds + (uint64_t)first * p.S);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int D, int ENG>

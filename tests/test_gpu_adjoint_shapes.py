@@ -77,3 +77,22 @@ def test_nearly_coincident_particles(ctx, dim, S):
         ep = rel_err(gp[k], wp[k]) if np.isfinite(wp[k]).all() else 0.0
         print(f"gap {gaps[k]:.1e}: state {es:.2e}, position {ep:.2e}")
         assert es <= TOL and ep <= TOL
+
+
+def test_more_particles_than_one_launch_takes(ctx):
+    """Past 2^24 particles a block takes several of them: 4,097 copies of one system give its result 4,097 times."""
+    import torch
+    B, N, S = 4097, 4096, 1
+    cfg = HashGridConfig(2, Boundary.Clamped, HashGridMode.Particle, (16, 16, 1), 0.05, 32)
+    rng = np.random.default_rng(5)
+    pos = np.zeros((N, 4), f32)
+    pos[:, :2] = rng.uniform(-0.9, 0.9, (N, 2))
+    st = rng.normal(0, 0.5, N * S).astype(f32)
+    opts = PerceptionOptions(state_grad=True, density_grad=False, eps0=0.05, hybrid_state_gradient=False)
+    fa = rng.normal(0, 0.1, N * opts.feature_dims(S, 2)).astype(f32)
+    want = O.perceive_adjoint_with_options(pos, st, 1, N, S, cfg, opts, fa)
+    many = lambda a: torch.from_numpy(a).cuda().reshape(1, -1).expand(B, -1).contiguous()  # noqa: E731
+    got = K.perceive_adjoint_with_options(many(pos).reshape(B * N, 4), many(st), B, N, S, cfg, opts, many(fa), ctx=ctx)
+    for g, w in ((got.state, want.state), (got.position, want.position)):
+        g = g.reshape(B, -1)
+        assert rel_err(to_np(g[0]), w) <= TOL and torch.equal(g, g[:1].expand(B, -1))

@@ -52,3 +52,18 @@ def test_two_kernel_step_bit_exact(ctx, d, S, H, n, periodic):
     got = NpaModel(m, w).step(pos, st, 1, n, g, 1.0, update_mask=mask, ctx=ctx)
     np.testing.assert_array_equal(to_np(got.next_positions), want.next_positions)
     np.testing.assert_array_equal(to_np(got.next_states), want.next_states)
+
+
+def test_more_rows_than_one_launch_takes(ctx):
+    """Rows past 2^26 go to another launch: the same results as the same rows of a short call."""
+    import torch
+    m = NpaConfig(spatial_dims=2, state_dims=1, hidden_dims=130, state_grad=False, density_grad=False)
+    mod = NpaModel(m, _weights(m, 3))
+    F, short, rows = m.perception_dims(), 4001, (1 << 26) + 37
+    feats = torch.randn(short, F, generator=torch.Generator().manual_seed(1)).cuda()
+    dx, ds = mod.forward_from_features_with_eps(feats.repeat(rows // short + 1, 1)[:rows], 0.1, ctx=ctx)
+    want_dx, want_ds = mod.forward_from_features_with_eps(feats, 0.1, ctx=ctx)
+    for got, want in ((dx.reshape(rows, 4), want_dx.reshape(short, 4)), (ds.reshape(rows, 1), want_ds.reshape(short, 1))):
+        for first in (0, rows // short * short - 3 * short, rows // short * short):
+            n = min(short, rows - first)
+            assert torch.equal(got[first:first + n], want[:n])
