@@ -404,6 +404,51 @@ __global__ __launch_bounds__(NW * 64, 2) void k_mlp_forward(StepParams P, const 
     }
 }
 
+// The same for networks of a few dozen products a row, of whose hidden units a wave of the kernel above
+// would use a few of its 64: a thread per row, 64 rows per block, their features staged in LDS (rows read
+// from memory by thread touch a cache line each) and the hidden units held there. The weights are uniform loads.
+template <int D>
+__global__ __launch_bounds__(64) void k_mlp_forward_narrow(StepParams P, const float* __restrict__ features, uint32_t rows,
+                                                           RawWeights raw, float* __restrict__ dx,
+                                                           float* __restrict__ ds) {
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t F = P.F, H = P.H, S = P.S, FS = F | 1u, lane = threadIdx.x;
+    const uint32_t row0 = blockIdx.x * 64, n = rows - row0 < 64 ? rows - row0 : 64;
+    float* hid = lds + 64 * FS;  // [H][64]
+    const float* src = features + (uint64_t)row0 * F;
+    uint32_t r = lane / F, k = lane % F;
+    for (uint32_t t = lane; t < n * F; t += 64) {
+        lds[r * FS + k] = src[t];
+        r += 64 / F;
+        k += 64 % F;
+        if (k >= F) {
+            k -= F;
+            ++r;
+        }
+    }
+    __syncthreads();
+    if (lane >= n) return;
+    const float* f = lds + lane * FS;
+    for (uint32_t h = 0; h < H; ++h) {
+        float sum = raw.b1[h];
+        for (uint32_t i = 0; i < F; ++i) sum += raw.w1[h * F + i] * f[i];
+        hid[h * 64 + lane] = fmaxf(sum, 0.0f);
+    }
+    auto output = [&](uint32_t o) {
+        float u = raw.b2[o];
+        for (uint32_t h = 0; h < H; ++h) u += raw.w2[o * H + h] * hid[h * 64 + lane];
+        return u;
+    };
+    float v[D], px[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int a = 0; a < D; ++a) v[a] = output(a);
+    motion<D>(P, v, px);
+    float* o = dx + 4 * (uint64_t)(row0 + lane);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) o[a] = px[a];
+    for (uint32_t c = 0; c < S; ++c) ds[(uint64_t)(row0 + lane) * S + c] = output(D + c);
+}
+
 // The update of the particles of 16 compact feature rows [rows][F]: MLP, motion scaling, 3D gates
 // (model.rs:806-837) and the masked Euler step (step.rs:4-55). A row's first S features are its
 // particle's state.
@@ -493,17 +538,29 @@ static uint32_t mlp_lds_bytes(const StepParams& p, int waves, bool raw) {
     return ((rows + 3) / 4 * 4 + (raw ? (uint32_t)waves * 64 * kTileS : 0u)) * 4;
 }
 
+// Networks of at most 400 products a row on rows that fill the chip: 600,000 rows of F = 6, H = 8 take 20 us with a
+// thread per row and 135 us with sixteen rows per block, of F = 66, H = 4 174 and 315 us. Above, or with few rows,
+// the rows' own chain sets the time (4,000 rows of F = 66, H = 4: 21 and 14 us; 60,000 of F = 18, H = 32: 29 and 24 us),
+// and wide rows leave too few waves (600,000 of F = 123, H = 2: 502 and 455 us).
+static bool mlp_narrow(const StepParams& p, uint32_t rows) {
+    return rows > 16384 && p.F <= 72 && (uint64_t)(p.F + p.g.dim + p.S) * p.H <= 400;
+}
+
 hipError_t launch_mlp_forward(const StepParams& p, const float* features, uint32_t rows, const StepIO& io,
                               float* dx, float* ds, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
     const int nw = mlp_waves(p);
-    auto k = p.g.dim == 2 ? (nw == 2 ? k_mlp_forward<2, 2> : k_mlp_forward<2, 4>)
-                          : (nw == 2 ? k_mlp_forward<3, 2> : k_mlp_forward<3, 4>);
+    const bool narrow = mlp_narrow(p, rows);
+    auto k = narrow ? (p.g.dim == 2 ? k_mlp_forward_narrow<2> : k_mlp_forward_narrow<3>)
+             : p.g.dim == 2 ? (nw == 2 ? k_mlp_forward<2, 2> : k_mlp_forward<2, 4>)
+                            : (nw == 2 ? k_mlp_forward<3, 2> : k_mlp_forward<3, 4>);
+    const uint32_t per = narrow ? 64u : (uint32_t)kMlpRows, threads = narrow ? 64u : (uint32_t)nw * 64;
+    const uint32_t lds = narrow ? 64 * ((p.F | 1u) + p.H) * 4 : mlp_lds_bytes(p, nw, true);
     // a launch holds fewer than 2^32 threads
     constexpr uint32_t kMost = 1u << 26;
     for (uint32_t first = 0; first < rows; first += std::min(rows - first, kMost)) {
         const uint32_t n = std::min(rows - first, kMost);
-        hipLaunchKernelGGL(k, dim3((n - 1) / kMlpRows + 1), dim3(nw * 64), mlp_lds_bytes(p, nw, true), stream, p,
+        hipLaunchKernelGGL(k, dim3((n - 1) / per + 1), dim3(threads), lds, stream, p,
                            features + (uint64_t)first * p.F, n, RawWeights{io.w1, io.b1, io.w2, io.b2},
                            dx + 4 * (uint64_t)first, ds + (uint64_t)first * p.S);
         const hipError_t e = hipGetLastError();

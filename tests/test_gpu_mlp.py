@@ -38,6 +38,22 @@ def test_mlp_forward_bit_exact(ctx, rows, d, S, H, dgrad):
     np.testing.assert_array_equal(to_np(ds), np.asarray(want_ds).reshape(rows, S))
 
 
+@pytest.mark.parametrize("rows,d,S,H,sgrad,dgrad", [
+    (16385, 2, 1, 16, True, True), (16448, 2, 16, 4, True, True), (16400, 3, 8, 7, True, False), (20001, 3, 13, 4, True, True),
+    (16449, 2, 32, 4, False, False), (16385, 3, 1, 1, False, False), (17000, 2, 4, 16, True, True)])
+def test_narrow_networks_bit_exact(ctx, rows, d, S, H, sgrad, dgrad):
+    """A thread per row: at most 400 products a row, more than 16,384 rows, feature counts on both sides of 64."""
+    m = NpaConfig(spatial_dims=d, state_dims=S, hidden_dims=H, state_grad=sgrad, density_grad=dgrad)
+    F = m.perception_dims()
+    assert F <= 72 and (F + m.update_dims()) * H <= 400
+    w = _weights(m, rows)
+    feats = np.random.default_rng(rows + H).normal(size=(rows, F)).astype(f32)
+    want_dx, want_ds = O.forward_from_features_with_eps(m, w, feats, 0.1)
+    dx, ds = NpaModel(m, w).forward_from_features_with_eps(feats, 0.1, ctx=ctx)
+    np.testing.assert_array_equal(to_np(dx), np.asarray(want_dx).reshape(rows, 4))
+    np.testing.assert_array_equal(to_np(ds), np.asarray(want_ds).reshape(rows, S))
+
+
 @pytest.mark.parametrize("d,S,H,n,periodic", [(2, 16, 256, 333, False), (2, 8, 129, 65, True), (3, 24, 256, 500, False),
                                               (3, 32, 300, 47, False), (2, 5, 1, 15, False)])
 def test_two_kernel_step_bit_exact(ctx, d, S, H, n, periodic):
