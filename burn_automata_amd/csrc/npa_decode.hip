@@ -231,11 +231,26 @@ struct SplatParams {
 __global__ __launch_bounds__(256) void k_splat_items(SplatParams P, const float4* __restrict__ pos,
                                                      const float* __restrict__ colors,
                                                      const float* __restrict__ states, uint32_t count,
-                                                     DrawItem* __restrict__ out, uint32_t* __restrict__ rects) {
-    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+                                                     DrawItem* __restrict__ out, uint32_t* __restrict__ rects,
+                                                     DrawPlan draw, uint32_t* __restrict__ crowd) {
+    const float fsz = (float)P.size;
+    const uint32_t planner = draw.extra ? 1u : 0u;  // the first block finds the crowded groups
+    if (blockIdx.x < planner) {
+        const float to_px = (fsz - 1.0f) / (P.hi - P.lo);
+        draw_crowd(draw, crowd, [&](uint32_t, uint32_t i, float* box) {
+            const float4 p = pos[i];
+            const float x = floorf((p.x - P.lo) * to_px), y0 = (p.y - P.lo) * to_px;
+            const float y = floorf(P.y_up ? fsz - 1.0f - y0 : y0), r = (float)P.radius;
+            box[0] = x - r;
+            box[1] = x + r;
+            box[2] = y - r;
+            box[3] = y + r;
+        });
+        return;
+    }
+    const uint32_t n = (blockIdx.x - planner) * blockDim.x + threadIdx.x;
     if (n >= count) return;
     const float4 p = pos[n];
-    const float fsz = (float)P.size;
     const float px = (p.x - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
     float py = (p.y - P.lo) / (P.hi - P.lo) * (fsz - 1.0f);
     if (P.y_up) py = (fsz - 1.0f) - py;
@@ -378,7 +393,7 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
 
 void SplatWorkspace::release() {
     for (DevBuf* b : {&params, &item_start, &keys, &vals, &sorted, &ranks, &table, &totals, &offsets, &count, &flags, &scan,
-                      &attrs, &partials, &order, &decoded, &sort_temp})
+                      &attrs, &partials, &crowd, &order, &decoded, &sort_temp})
         b->release();
 }
 
@@ -414,14 +429,15 @@ hipError_t launch_splat_2d(const float4* pos, const float* colors, const float* 
     if (!make_draw_plan(P.size, P.radius, windows, per_window, count, 4, win_cols, &draw)) return hipErrorInvalidValue;
     if ((e = ws.params.reserve((uint64_t)(count ? count : 1) * sizeof(DrawItem))) != hipSuccess) return e;
     if ((e = ws.keys.reserve((uint64_t)(count ? count : 1) * 4)) != hipSuccess) return e;
-    if ((e = ws.partials.reserve(draw.partial_floats * 4)) != hipSuccess) return e;
+    if ((e = reserve_draw(draw, ws, stream)) != hipSuccess) return e;
     ProfScope ps(prof, NPA_KERNEL_SPLAT, stream);
     if (count) {
-        hipLaunchKernelGGL(k_splat_items, dim3((count + 255) / 256), dim3(256), 0, stream, P, pos, colors, states, count,
-                           ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
+        hipLaunchKernelGGL(k_splat_items, dim3((count + 255) / 256 + (draw.extra ? 1 : 0)), dim3(256), 0, stream, P, pos,
+                           colors, states, count, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), draw,
+                           ws.crowd.as<uint32_t>());
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), image, stream);
+    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws, image, stream);
 }
 
 // ------------------------------------------------------- projected 3D render
@@ -443,8 +459,28 @@ __global__ __launch_bounds__(256) void k_render_items(RenderParams P, const floa
                                                       const float* __restrict__ colors,
                                                       const float* __restrict__ opacities,
                                                       const float* __restrict__ sigmas, DrawItem* __restrict__ out,
-                                                      uint32_t* __restrict__ rects) {
-    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+                                                      uint32_t* __restrict__ rects, DrawPlan draw,
+                                                      uint32_t* __restrict__ crowd) {
+    const float fsz1 = (float)P.size - 1.0f;
+    const uint32_t planner = draw.extra ? 1u : 0u;  // the first block finds the crowded groups
+    if (blockIdx.x < planner) {
+        if (blockIdx.y != 0) return;
+        const float to_px = fsz1 / (2.0f * P.ws);
+        draw_crowd(draw, crowd, [&](uint32_t v, uint32_t i, float* box) {
+            const float* B = P.basis[v];
+            const uint32_t n = i - v * P.count;
+            const float4 p = pos[n];
+            const float r = ceilf(5.0f * clampf_(sigmas[n], P.min_sigma, P.max_sigma));
+            const float x = floorf((P.ws + (p.x * B[0] + p.y * B[1] + p.z * B[2])) * to_px);
+            const float y = floorf((P.ws - (p.x * B[3] + p.y * B[4] + p.z * B[5])) * to_px);
+            box[0] = x - r;
+            box[1] = x + r;
+            box[2] = y - r;
+            box[3] = y + r;
+        });
+        return;
+    }
+    const uint32_t n = (blockIdx.x - planner) * blockDim.x + threadIdx.x;
     if (n >= P.count) return;
     const uint32_t v = blockIdx.y;
     const float* B = P.basis[v];
@@ -454,7 +490,6 @@ __global__ __launch_bounds__(256) void k_render_items(RenderParams P, const floa
     const float f = p.x * B[6] + p.y * B[7] + p.z * B[8];
     const float sigma = fmaxf(clampf_(sigmas[n], P.min_sigma, P.max_sigma), kRenderEps);
     const int64_t radius = f32_to_isize(fmaxf(ceilf(5.0f * sigma), 1.0f));
-    const float fsz1 = (float)P.size - 1.0f;
     DrawItem d;
     d.px = (x + P.ws) / (2.0f * P.ws) * fsz1;
     d.py = (P.ws - y) / (2.0f * P.ws) * fsz1;
@@ -531,14 +566,15 @@ hipError_t launch_render_views(const float4* pos, const float* colors, const flo
     if (!make_draw_plan(P.size, radius, nviews, count, items, 5, nviews, &draw)) return hipErrorInvalidValue;
     if ((e = ws.params.reserve((uint64_t)(items ? items : 1) * sizeof(DrawItem))) != hipSuccess) return e;
     if ((e = ws.keys.reserve((uint64_t)(items ? items : 1) * 4)) != hipSuccess) return e;
-    if ((e = ws.partials.reserve(draw.partial_floats * 4)) != hipSuccess) return e;
+    if ((e = reserve_draw(draw, ws, stream)) != hipSuccess) return e;
     ProfScope ps(prof, NPA_KERNEL_RENDER, stream);
     if (count) {
-        hipLaunchKernelGGL(k_render_items, dim3((count + 255) / 256, nviews), dim3(256), 0, stream, P, pos, colors, opacities,
-                           sigmas, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>());
+        hipLaunchKernelGGL(k_render_items, dim3((count + 255) / 256 + (draw.extra ? 1 : 0), nviews), dim3(256), 0, stream, P,
+                           pos, colors, opacities, sigmas, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), draw,
+                           ws.crowd.as<uint32_t>());
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws.partials.as<float>(), images, stream);
+    return launch_draw(draw, ws.params.as<DrawItem>(), ws.keys.as<uint32_t>(), ws, images, stream);
 }
 
 // state_tail_render_attributes (render_loss/attributes.rs:15-87): one thread per particle.

@@ -12,15 +12,17 @@
 // No sort either: a block covers a group of G x G tiles; its waves test the packed tile rectangles of
 // their shares of the window's items and keep the indices of those that touch the group, in ascending
 // order; then they draw the group's tiles from the kept items (several waves per tile for small groups,
-// their sums added in a fixed order). So items are added in a fixed order and the image is deterministic;
-// it differs from the reference's running sums only by rounding.
+// their sums added in a fixed order). The items of crowded groups are divided among further blocks, by a sample
+// of the items alone. So items are added in a fixed order and the image is deterministic; it differs from the
+// reference's running sums only by rounding.
 //
 // Bound: the matrix instructions, 32 cycles per channel and four items (160 cycles for five channels), and
 // the tests, about twelve instructions per 64 items and group. Against the former passes (items sorted by
 // tile, a wave evaluating every pixel's exponential): four 64x64 views of 16,384 particles 161 -> 45 us with
 // their preparation, a 512x512 splat of 65,536 89 -> 28 us, a 160x160 view of 4,000 102 -> 35 us, 300,000
-// at 2048x2048 1,094 -> 405 us, 500,000 at 4096x4096 8.5 -> 1.7 ms; faster at every size measured, so the
-// sorted passes are gone.
+// at 2048x2048 1,094 -> 405 us, 500,000 at 4096x4096 8.5 -> 1.7 ms, and on a part of the image 300,000 at 2048x2048
+// 1,519 -> 433 us, four 512x512 views of 100,000 790 -> 608 us. At most a sixth slower where all items lie on a few
+// pixels of a large image (20,000 on a fiftieth of four 512x512 views 255 -> 288 us); the sorted passes are gone.
 #include "npa_draw.hpp"
 
 #include <algorithm>
@@ -101,25 +103,53 @@ struct DrawTile {
     }
 };
 
-// Grid: x = window * groups_x^2 + group, y = split of the window's items.
+// Which items a block draws: range `range` of `ranges` of the items of group `blk`'s window; the second range's
+// partial tiles are at `slot` and so on.
+struct DrawShare {
+    uint32_t blk, range, ranges, slot;
+};
+
+// Grid: single tiles (G = 1): x = window * groups_x^2 + group, y = split of the window's items. Groups: the first
+// P.groups blocks take one each, the others the further ranges of crowded groups (draw_crowd's jobs), and the
+// block that finishes such a group last adds up its ranges, in order.
 // NW waves per block: sixteen for groups of tiles, whose waves share the tests of every item of the window;
 // four for single tiles, whose blocks are short and hide each other's latencies (four of them per CU).
 template <int NCH, int G, int NW>
 __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const float4* __restrict__ items,
                                                         const uint32_t* __restrict__ rects,
-                                                        float* __restrict__ partials, float* __restrict__ image) {
+                                                        float* partials, uint32_t* crowd, float* image) {
     constexpr uint32_t TILES = G * G, WPT = NW / TILES;  // tiles per block, waves per tile
     constexpr uint32_t NR = NCH * 4;                             // accumulated values per lane
     // the waves' kept items (rectangle, index), then their queues; the sums of the waves at the end
     constexpr uint32_t LIST = NW * kDrawSeg * 2, QUEUE = NW * kDrawQueue, SUMS = NW * NR * 64;
     __shared__ uint32_t lds[LIST + QUEUE > SUMS ? LIST + QUEUE : SUMS];
-    __shared__ uint32_t counts[NW], unfinished;
+    __shared__ uint32_t counts[NW], unfinished, last_ticket;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t per_win = P.groups_x * P.groups_x;
-    // the ranges of one crowded tile go to different CUs: each range's blocks start at another tile (a CU
-    // gets about every 256th block)
-    const uint32_t blk = (uint32_t)((blockIdx.x + (uint64_t)blockIdx.y * (gridDim.x * 5 / 8 | 1u) + blockIdx.y / 4) % gridDim.x);
+    DrawShare share;
+    uint32_t crowded = 0;
+    if constexpr (G == 1) {
+        // the ranges of one crowded tile go to different CUs: each range's blocks start at another tile (a CU
+        // gets about every 256th block)
+        share.blk = (uint32_t)((blockIdx.x + (uint64_t)blockIdx.y * (gridDim.x * 5 / 8 | 1u) + blockIdx.y / 4) % gridDim.x);
+        share.range = blockIdx.y;
+        share.ranges = P.splits;
+        share.slot = 0;
+    } else {
+        share = {blockIdx.x, 0u, 1u, 0u};
+        if (P.extra) {
+            if (blockIdx.x >= P.groups) {
+                const uint32_t job = blockIdx.x - P.groups;
+                if (job >= crowd[kCrowdJobs]) return;  // whole block
+                const uint32_t j = crowd[kCrowdJobs + 1 + job];
+                share.blk = j & 0xffffu;
+                share.range = j >> 16;
+            }
+            crowded = crowd[kCrowdGroups + share.blk];
+        }
+    }
+    const uint32_t blk = share.blk;
     const uint32_t win = blk / per_win, grp = blk - win * per_win;
     const uint32_t gx0 = grp % P.groups_x * G, gy0 = grp / P.groups_x * G;
     const uint32_t tg = wave % TILES, part = wave / TILES;
@@ -135,12 +165,31 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
     const uint64_t win_beg = (uint64_t)win * P.per_window;
     const uint64_t win_end = win_beg + P.per_window < P.count ? win_beg + P.per_window : P.count;
     const uint32_t n = win_end > win_beg ? (uint32_t)(win_end - win_beg) : 0u;
-    const uint32_t share = (n + P.splits - 1) / P.splits;
-    const uint32_t first = min(n, blockIdx.y * share), last = min(n, first + share);
-    const uint32_t mine = (last - first + NW - 1) / NW;
-    uint32_t pos = min(last, first + wave * mine);
-    const uint32_t end = min(last, pos + mine);
+    uint32_t pos, end;
+    auto take_share = [&] {
+        const uint32_t part_n = (n + share.ranges - 1) / share.ranges;
+        const uint32_t first = min(n, share.range * part_n), last = min(n, first + part_n);
+        const uint32_t mine = (last - first + NW - 1) / NW;
+        pos = min(last, first + wave * mine);
+        end = min(last, pos + mine);
+    };
+    take_share();
     const uint32_t* rw = rects + win_beg;
+    uint32_t r[kDrawPer];
+    auto fetch = [&](uint32_t at) {
+#pragma unroll
+        for (uint32_t i = 0; i < kDrawPer; ++i) {
+            const uint32_t k = at + i * 64 + lane;
+            r[i] = k < end ? rw[k] : kDrawNone;
+        }
+    };
+    fetch(pos);
+    if (crowded & 0xffu) {  // known by now: few groups are, and start again with their range
+        share.ranges = (crowded & 0xffu) + 1;
+        share.slot = crowded >> 8;
+        take_share();
+        fetch(pos);
+    }
     auto wave_fence = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -155,6 +204,7 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
     } E0, E1;
     uint32_t waiting = 0;  // entries in this wave's queue
     bool ahead = false;    // E0 holds eight entries not drawn yet
+    float warm = 0.0f;
     auto load = [&](uint32_t at, uint32_t count, Eight& e) {
 #pragma unroll
         for (uint32_t h = 0; h < 2; ++h) {
@@ -174,15 +224,6 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
         // each wave tests its items in turn and keeps those that touch the group
         uint32_t kept = 0;
         if (threadIdx.x == 0) unfinished = 0;
-        uint32_t r[kDrawPer];
-        auto fetch = [&](uint32_t at) {
-#pragma unroll
-            for (uint32_t i = 0; i < kDrawPer; ++i) {
-                const uint32_t k = at + i * 64 + lane;
-                r[i] = k < end ? rw[k] : kDrawNone;
-            }
-        };
-        fetch(pos);
         while (pos < end && kept + kDrawPer * 64 <= kDrawSeg) {
             uint32_t c[kDrawPer];
 #pragma unroll
@@ -226,7 +267,15 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
             const uint2 it = e < k_end ? list[at] : make_uint2(kDrawNone, 0u);
             const bool hit = G == 1 && sh == 0 ? e < k_end : rect_touches(it.x, tlim);
             const uint64_t m = __ballot(hit);
-            if (hit) queue[waiting + (uint32_t)__popcll(m & lanemask_lt())] = (uint32_t)win_beg + it.y;
+            // One word of every item kept, in flight while the entries before it are drawn: the items come from
+            // the last cache level, at about a microsecond for every eight that a wave draws, and then from L2.
+            // (Single tiles' ranges are short.)
+            if constexpr (G > 1) asm volatile("" ::"v"(warm));
+            if (hit) {
+                const uint32_t at_item = (uint32_t)win_beg + it.y;
+                queue[waiting + (uint32_t)__popcll(m & lanemask_lt())] = at_item;
+                if constexpr (G > 1) warm = items[(uint64_t)at_item * 3].x;
+            }
             waiting += (uint32_t)__popcll(m);
             wave_fence();
             uint32_t q = 0;
@@ -256,6 +305,7 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
         }
         if (!more) break;
         __syncthreads();  // the list and the counts are read before they are filled again
+        fetch(pos);
     }
     if (ahead) draw(E0);
     if (waiting) {
@@ -270,6 +320,20 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
 #pragma unroll
         for (int q = 0; q < 4; ++q) sums[(wave * NR + ch * 4 + q) * 64 + lane] = tile.acc[ch][q];
     __syncthreads();
+    auto out = [&](uint32_t x, uint32_t y) {
+        if constexpr (NCH == 4)
+            return image + (((uint64_t)(win / P.win_cols) * P.size + y) * P.stride + (uint64_t)(win % P.win_cols) * P.size + x) * 4;
+        else
+            return image + (((uint64_t)win * P.size + y) * P.size + x) * NCH;
+    };
+    auto put = [&](float* o, const float (&v)[NCH]) {
+        if constexpr (NCH == 4) {
+            *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int ch = 0; ch < NCH; ++ch) o[ch] = v[ch];
+        }
+    };
     for (uint32_t t = threadIdx.x; t < TILES * 256; t += NW * 64) {
         const uint32_t tl = t / 256, row = t % 256 / 16, col = t % 16;
         const uint32_t x = (gx0 + tl % G) * 16 + col, y = (gy0 + tl / G) * 16 + row;
@@ -281,17 +345,48 @@ __global__ __launch_bounds__(NW * 64, 4) void k_draw_tiles(DrawPlan P, const flo
             for (uint32_t p = 0; p < WPT; ++p)
                 v[ch] += sums[((p * TILES + tl) * NR + ch * 4 + row % 4) * 64 + row / 4 * 16 + col];
         }
-        if (P.splits > 1) {
+        if (G == 1 && P.splits > 1) {
             const uint64_t pixel = ((uint64_t)win * P.size + y) * P.size + x, all = (uint64_t)P.windows * P.size * P.size;
 #pragma unroll
             for (int ch = 0; ch < NCH; ++ch) partials[((uint64_t)blockIdx.y * NCH + ch) * all + pixel] = v[ch];
-        } else if constexpr (NCH == 4) {
-            const uint64_t at = ((uint64_t)(win / P.win_cols) * P.size + y) * P.stride + (uint64_t)(win % P.win_cols) * P.size + x;
-            reinterpret_cast<float4*>(image)[at] = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            float* o = image + (((uint64_t)win * P.size + y) * P.size + x) * NCH;
+        } else if (G > 1 && share.range > 0) {
 #pragma unroll
-            for (int ch = 0; ch < NCH; ++ch) o[ch] = v[ch];
+            for (int ch = 0; ch < NCH; ++ch) partials[((uint64_t)(blockIdx.x - P.groups) * NCH + ch) * (TILES * 256) + t] = v[ch];
+        } else {
+            put(out(x, y), v);
+        }
+    }
+    if constexpr (G > 1) {
+        if (share.ranges == 1) return;
+        // the last of the group's blocks adds the ranges up: the first in the image, the others from their slots
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __syncthreads();
+        if (threadIdx.x == 0) last_ticket = __hip_atomic_fetch_add(&crowd[blk], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (last_ticket != share.ranges - 1) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (threadIdx.x == 0) crowd[blk] = 0;  // for the next drawing
+        for (uint32_t t = threadIdx.x; t < TILES * 256; t += NW * 64) {
+            const uint32_t tl = t / 256, row = t % 256 / 16, col = t % 16;
+            const uint32_t x = (gx0 + tl % G) * 16 + col, y = (gy0 + tl / G) * 16 + row;
+            if (x >= (uint32_t)P.size || y >= (uint32_t)P.size) continue;
+            float* o = out(x, y);
+            const float* slot = partials + (uint64_t)share.slot * NCH * (TILES * 256) + t;
+            float v[NCH];
+#pragma unroll
+            for (int ch = 0; ch < NCH; ++ch) v[ch] = o[ch];
+            for (uint32_t s = 1; s < share.ranges; s += 8) {  // eight ranges' loads at a time
+                float w[8][NCH];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u, slot += NCH * (TILES * 256))
+#pragma unroll
+                    for (int ch = 0; ch < NCH; ++ch) w[u][ch] = s + u < share.ranges ? slot[ch * (TILES * 256)] : 0.0f;
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u)
+#pragma unroll
+                    for (int ch = 0; ch < NCH; ++ch) v[ch] += w[u][ch];
+            }
+            put(o, v);
         }
     }
 }
@@ -339,6 +434,13 @@ bool make_draw_plan(int size, int radius, uint32_t windows, uint32_t per_window,
     // the largest groups that still give every CU a block
     p.group = blocks(4) >= cus ? 4 : blocks(2) >= cus ? 2 : 1;
     p.groups_x = ((uint32_t)p.tiles_x + p.group - 1) / p.group;
+    p.groups = (uint32_t)std::min<uint64_t>(blocks(p.group), UINT32_MAX);
+    // Groups: an object on a part of the window leaves most CUs without items, so the further ranges of crowded
+    // groups' items go to blocks of their own, at most one per CU (draw_crowd). Measured, one block per group
+    // against ranges: 100,000 particles on a tenth of a 512x512 view 2,232 -> 178 us, four such views 4,626 ->
+    // 608 us, on a fiftieth of a 1024x1024 view 5,793 -> 311 us, a splat of 300,000 on a tenth of 2048x2048 2,722 ->
+    // 433 us; even drawings keep their times (65,536 at 512x512 27 us).
+    p.extra = p.group > 1 && p.groups <= kDrawGroups && count >= 1024 ? std::min(count / 256, kCrowdMost) : 0;
     // Single tiles: ranges of at least 512 of a window's items go to blocks of their own, for four blocks per
     // CU and for about 128 items per block where the items spread over the window (four times that where
     // an object fills its middle), so that crowded tiles leave no CU waiting. Measured, one range against
@@ -352,29 +454,45 @@ bool make_draw_plan(int size, int radius, uint32_t windows, uint32_t per_window,
         const uint64_t crowd = (uint64_t)((double)n * side * side / 128.0);
         p.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({std::max(4 * cus / blocks(1), crowd), n / 512, 16}));
     }
-    p.partial_floats = p.splits > 1 ? (uint64_t)p.splits * channels * windows * size * size : 0;
+    p.partial_floats = p.splits > 1 ? (uint64_t)p.splits * channels * windows * size * size
+                                    : (uint64_t)p.extra * channels * p.group * p.group * 256;
     if (blocks(p.group) >= (1ull << 31)) return false;
     *plan = p;
     return true;
 }
 
-template <int NCH>
-static hipError_t launch_draw_n(const DrawPlan& p, const DrawItem* items, const uint32_t* rects, float* partials,
-                                float* image, hipStream_t stream) {
-    auto k = p.group == 4 ? k_draw_tiles<NCH, 4, 16> : p.group == 2 ? k_draw_tiles<NCH, 2, 16> : k_draw_tiles<NCH, 1, 4>;
-    hipLaunchKernelGGL(k, dim3(p.groups_x * p.groups_x * p.windows, p.splits), dim3(p.group == 1 ? 256 : 1024), 0, stream, p,
-                       reinterpret_cast<const float4*>(items), rects, partials, image);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.splits == 1) return e;
-    const uint64_t pixels = (uint64_t)p.windows * p.size * p.size;
-    hipLaunchKernelGGL(k_draw_reduce<NCH>, dim3((uint32_t)((pixels + 255) / 256)), dim3(256), 0, stream, p, partials, image);
+__global__ __launch_bounds__(256) void k_draw_clear(uint32_t* tickets) {
+    tickets[blockIdx.x * 256 + threadIdx.x] = 0;
+}
+
+hipError_t reserve_draw(const DrawPlan& p, SplatWorkspace& ws, hipStream_t stream) {
+    hipError_t e = ws.partials.reserve(p.partial_floats * 4);
+    if (e != hipSuccess || !p.extra || ws.crowd.ptr) return e;
+    if ((e = ws.crowd.reserve(kCrowdWords * 4)) != hipSuccess) return e;
+    // the tickets are zero between drawings: the block that takes a group's last one clears it
+    hipLaunchKernelGGL(k_draw_clear, dim3(kDrawGroups / 256), dim3(256), 0, stream, ws.crowd.as<uint32_t>());
     return hipGetLastError();
 }
 
-hipError_t launch_draw(const DrawPlan& p, const DrawItem* items, const uint32_t* rects, float* partials, float* image,
+template <int NCH>
+static hipError_t launch_draw_n(const DrawPlan& p, const DrawItem* items, const uint32_t* rects, SplatWorkspace& ws,
+                                float* image, hipStream_t stream) {
+    auto k = p.group == 4 ? k_draw_tiles<NCH, 4, 16> : p.group == 2 ? k_draw_tiles<NCH, 2, 16> : k_draw_tiles<NCH, 1, 4>;
+    hipLaunchKernelGGL(k, dim3(p.groups + p.extra, p.splits), dim3(p.group == 1 ? 256 : 1024), 0, stream, p,
+                       reinterpret_cast<const float4*>(items), rects, ws.partials.as<float>(), ws.crowd.as<uint32_t>(),
+                       image);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.splits == 1) return e;
+    const uint64_t pixels = (uint64_t)p.windows * p.size * p.size;
+    hipLaunchKernelGGL(k_draw_reduce<NCH>, dim3((uint32_t)((pixels + 255) / 256)), dim3(256), 0, stream, p,
+                       ws.partials.as<float>(), image);
+    return hipGetLastError();
+}
+
+hipError_t launch_draw(const DrawPlan& p, const DrawItem* items, const uint32_t* rects, SplatWorkspace& ws, float* image,
                        hipStream_t stream) {
-    return p.channels == 4 ? launch_draw_n<4>(p, items, rects, partials, image, stream)
-                           : launch_draw_n<5>(p, items, rects, partials, image, stream);
+    return p.channels == 4 ? launch_draw_n<4>(p, items, rects, ws, image, stream)
+                           : launch_draw_n<5>(p, items, rects, ws, image, stream);
 }
 
 }  // namespace npa

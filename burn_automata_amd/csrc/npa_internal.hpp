@@ -409,6 +409,7 @@ struct SplatWorkspace {
     DevBuf params, item_start, keys, vals, sorted, ranks, table, totals, offsets, count, flags, scan;
     DevBuf attrs;  // render attributes of a state's particles: colours [n][3], opacities [n], sigmas [n]
     DevBuf partials;  // the drawing's partial images, one per item range
+    DevBuf crowd;     // the drawing's crowded groups (npa_draw.hpp)
     DevBuf order;      // oriented raster: depth order
     DevBuf sort_temp;  // oriented raster: the radix sort's temporary storage
     DevBuf decoded;  // oriented raster of a state: its decoded Gaussians

@@ -116,3 +116,73 @@ def test_huge_finite_colours_stay_in_their_footprint(ctx):
     want = to_np(want).reshape(got.shape)
     assert np.isfinite(want).all() and np.isfinite(got).all()
     np.testing.assert_allclose(got.astype(np.float64), want.astype(np.float64), rtol=2e-4, atol=1e-4)
+
+
+def _splat64(pos, col, cfg):
+    """The splat of a cloud in 64 bits, on the box of pixels it reaches: sum_p col_p scale_p e_p(y) e_p(x) with the
+    32-bit pixel coordinates and sigma of the splat. Returns the box's first column and row and [y, x, 4]."""
+    size, span = f32(cfg.image_size), f32(cfg.hi) - f32(cfg.lo)
+    sigma = f32(cfg.sigma) * size * f32(cfg.pixel_size) / span
+    r, t = max(1, int(np.ceil(f32(5) * sigma))), float(size * f32(cfg.pixel_size) / span)
+    px = (pos[:, 0] - f32(cfg.lo)) / span * (size - f32(1))
+    py = (size - f32(1)) - (pos[:, 1] - f32(cfg.lo)) / span * (size - f32(1))
+    axes, at = [], []
+    for p in (px, py):
+        b = np.floor(p).astype(int)
+        x = np.arange(max(0, b.min() - r), min(cfg.image_size - 1, b.max() + r) + 1)
+        w = np.exp(-(x[None, :] - p[:, None].astype(np.float64)) ** 2 / (2 * float(sigma) ** 2))
+        axes.append(w * (np.abs(x[None, :] - b[:, None]) <= r))
+        at.append(x[0])
+    wx, wy = axes
+    scale = t * t / np.maximum(wx.sum(1) * wy.sum(1), 1e-8)
+    v = np.concatenate([col.astype(np.float64), np.ones((len(col), 1))], 1) * scale[:, None]
+    return at, np.stack([wy.T @ (wx * v[:, c:c + 1]) for c in range(4)], -1)
+
+
+@pytest.mark.parametrize("n,size,spread,share", [
+    (40000, 520, 0.02, 10000), (600000, 520, 0.01, 9400),  # groups of 2x2 tiles
+    (6000, 1040, 0.01, 512), (600000, 1040, 0.01, 9400),   # of 4x4: a few ranges, and the most, whose lists are filled twice
+    (9000, 2048, 0.04, 1200), (5000, 2033, 0.5, 5000)])
+def test_crowded_splats(ctx, n, size, spread, share):
+    """A cloud on a few tiles. Every 97th particle's colour is a thousand times the others', so a lost run of
+    particles shows; a wave's sums take one rounding for four items, `share` of them at most."""
+    pos, col, _, _ = _particles(n, size + n, spread)
+    pos[:, 0] += f32(0.31)
+    col[::97] *= 1000
+    cfg = Splat2dConfig(image_size=size, sigma=1.0, pixel_size=2.0 / size)
+    got = to_np(K.splat_particles_2d(pos, col, cfg, ctx=ctx)).reshape(size, size, 4)
+    (x0, y0), want = _splat64(pos, col, cfg)
+    box = got[y0:y0 + want.shape[0], x0:x0 + want.shape[1]].astype(np.float64)
+    assert np.count_nonzero(got) == np.count_nonzero(box)
+    for ch in range(4):
+        e = np.max(np.abs(box[..., ch] - want[..., ch])) / np.max(np.abs(want[..., ch]))
+        print(f"channel {ch}: {e:.2e}")
+        assert e <= TOL + share / 4 * 2.0 ** -24
+    for _ in range(2):  # the ranges' counters are left as they were found
+        np.testing.assert_array_equal(to_np(K.splat_particles_2d(pos, col, cfg, ctx=ctx)).reshape(got.shape), got)
+
+
+@pytest.mark.parametrize("n,size,views,spread", [(6000, 256, (0, 1, 2, 3), 0.03), (7000, 520, (0, 1, 2, 3), 0.05),
+                                                 (5000, 530, (1,), 0.02), (3000, 1024, (3,), 0.3)])
+def test_crowded_renders_match_the_oracle(ctx, n, size, views, spread):
+    pos, col, op, sg = _particles(n, n, spread)
+    pos[:, 0] -= f32(0.4)
+    cfg = RenderLossConfig(image_size=size)
+    got = to_np(K.render_views(pos, col, op, sg, cfg, views, ctx=ctx))
+    for k, v in enumerate(views):
+        want = O.splat_projected(O.project_positions(v, pos, cfg.world_scale), col, op, sg, cfg)
+        assert _err(got[k], want) <= TOL
+    np.testing.assert_array_equal(to_np(K.render_views(pos, col, op, sg, cfg, views, ctx=ctx)), got)
+
+
+def test_crowded_windows(ctx):
+    batch, n, size, cols = 4, 3000, 500, 2
+    pos, col, _, _ = _particles(batch * n, 9, 0.02)
+    pos[n:2 * n, :2] += f32(0.5)
+    pos[3 * n:, 1] -= f32(0.98)
+    cfg = Splat2dConfig(image_size=size, sigma=1.2, pixel_size=2.0 / size)
+    got = to_np(K.splat_particles_2d_tiled(pos, col, batch, n, cfg, cols, ctx=ctx))
+    for b in range(batch):
+        want = to_np(O.splat_particles_2d(pos[b * n:(b + 1) * n], col[b * n:(b + 1) * n], cfg)).reshape(size, size, 4)
+        win = got[b // cols * size:(b // cols + 1) * size, b % cols * size:(b % cols + 1) * size]
+        assert _err(win, want) <= TOL
