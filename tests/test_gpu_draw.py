@@ -186,3 +186,16 @@ def test_crowded_windows(ctx):
         want = to_np(O.splat_particles_2d(pos[b * n:(b + 1) * n], col[b * n:(b + 1) * n], cfg)).reshape(size, size, 4)
         win = got[b // cols * size:(b // cols + 1) * size, b % cols * size:(b % cols + 1) * size]
         assert _err(win, want) <= TOL
+
+
+@pytest.mark.parametrize("size", [2032, 2033, 4096])  # 127 tiles an axis, 128 (rectangles in pairs of tiles), 256
+@pytest.mark.parametrize("corner", [(-1, -1), (1, 1), (0.37, 1), (1, -0.2)])
+def test_rectangles_of_wide_images(ctx, size, corner):
+    pos, col, _, _ = _particles(300, size, 0.02)
+    pos[:, :2] += np.asarray(corner, f32)
+    cfg = Splat2dConfig(image_size=size, sigma=1.3, pixel_size=2.0 / size)
+    got = to_np(K.splat_particles_2d(pos, col, cfg, ctx=ctx)).reshape(size, size, 4)
+    (x0, y0), want = _splat64(pos, col, cfg)
+    box = got[y0:y0 + want.shape[0], x0:x0 + want.shape[1]]
+    assert np.count_nonzero(got) == np.count_nonzero(box)
+    assert _err(box, want) <= TOL

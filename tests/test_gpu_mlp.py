@@ -70,6 +70,21 @@ def test_two_kernel_step_bit_exact(ctx, d, S, H, n, periodic):
     np.testing.assert_array_equal(to_np(got.next_states), want.next_states)
 
 
+@pytest.mark.parametrize("d,S,H", [(2, 16, 128), (3, 24, 256), (2, 5, 65)])
+@pytest.mark.parametrize("scale,w2", [(1e-37, 0.3), (3e-39, 0.3), (3e-39, 1e-6), (1e-42, 0.3)])
+def test_subnormal_products_bit_exact(ctx, d, S, H, scale, w2):
+    """Without biases: features, products and hidden units below the smallest normal number keep their bits."""
+    m = NpaConfig(spatial_dims=d, state_dims=S, hidden_dims=H)
+    w = _weights(m, H)
+    w["b1"], w["b2"], w["w2"] = 0 * w["b1"], 0 * w["b2"], w["w2"] * f32(w2 / 0.3)
+    feats = (np.random.default_rng(S).normal(size=(40, m.perception_dims())) * scale).astype(f32)
+    want_dx, want_ds = O.forward_from_features_with_eps(m, w, feats, 0.1)
+    dx, ds = NpaModel(m, w).forward_from_features_with_eps(feats, 0.1, ctx=ctx)
+    assert np.count_nonzero(want_ds)
+    np.testing.assert_array_equal(to_np(dx), np.asarray(want_dx).reshape(40, 4))
+    np.testing.assert_array_equal(to_np(ds), np.asarray(want_ds).reshape(40, S))
+
+
 def test_more_rows_than_one_launch_takes(ctx):
     """Rows past 2^26 go to another launch: the same results as the same rows of a short call."""
     import torch
