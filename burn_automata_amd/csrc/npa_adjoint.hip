@@ -202,9 +202,9 @@ __device__ __forceinline__ void adj_walk(const StepParams& P, const AdjointArgs&
 // One wave per 16 particles over their lists of accepted neighbours: a walk over the 3^D cells'
 // candidates runs its body for all 16 particles whenever one of them accepts, about three times as
 // often. Lane q takes the pair quantities of every fourth entry, and all four lanes that entry's sums for
-// their channels. Bound: VALU issue and the rows' gathers at two to three waves per SIMD. Measured on
-// 8 x 4,096 2D particles, 41 neighbours each, S = 16: 176 -> 27 us; 2 x 8,192 3D particles, 65
-// neighbours, S = 24: 438 -> 39 us.
+// their channels. Bound: VALU issue and the rows' gathers, at two waves per SIMD (the 2D system below)
+// or one (the 3D system). Measured on 8 x 4,096 2D particles, 41 neighbours each, S = 16: 176 -> 27 us;
+// 2 x 8,192 3D particles, 65 neighbours, S = 24: 438 -> 39 us.
 template <int D, int SM>
 __global__ __launch_bounds__(64) void k_adj_prep(StepParams P, AdjointArgs A) {
     using Row = AdjRow<D, SM>;
@@ -610,111 +610,110 @@ __global__ __launch_bounds__(64) void k_adj_gather(StepParams P, AdjointArgs A) 
 template <int D>
 __global__ __launch_bounds__(256) void k_adj_density_kernel(StepParams P, AdjointArgs A) {
     constexpr uint32_t MAXC = max_chunks(D);
-    const uint32_t nrows = *A.row_count, l = threadIdx.x % 16;
-    for (uint32_t it = blockIdx.x; it * 16 < nrows; it += gridDim.x) {
-        const uint32_t row = it * 16 + threadIdx.x / 16;
-        if (row >= nrows) continue;  // whole 16-lane groups
-        const uint32_t s = A.act_rows[row];
-        const uint32_t b = s / P.N;
-        const float4 own = A.dpos[s];
-        const float pk[3] = {own.x, own.y, own.z};
-        float pa[3] = {0.0f, 0.0f, 0.0f};
-        auto add = [&](const float4& o, bool test) {
-            float d[3];
-            d[0] = delta_axis(pk[0], o.x, 0, P.g);
-            d[1] = delta_axis(pk[1], o.y, 1, P.g);
-            d[2] = 0.0f;
-            float r2 = d[0] * d[0];
-            r2 += d[1] * d[1];
-            if constexpr (D == 3) {
-                d[2] = delta_axis(pk[2], o.z, 2, P.g);
-                r2 += d[2] * d[2];
-            }
-            if (test && !(r2 < P.g.eps2)) return;
-            const float x = P.g.eps2 - r2;
-            const float w = 6.0f * P.g.k6 * (x * x) * (o.w + own.w);
+    const uint32_t row = (blockIdx.y * gridDim.x + blockIdx.x) * 16 + threadIdx.x / 16, l = threadIdx.x % 16;
+    if (row >= *A.row_count) return;  // whole 16-lane groups leave together
+    const uint32_t s = A.act_rows[row];
+    const uint32_t b = s / P.N;
+    const float4 own = A.dpos[s];
+    const float pk[3] = {own.x, own.y, own.z};
+    float pa[3] = {0.0f, 0.0f, 0.0f};
+    auto add = [&](const float4& o, bool test) {
+        float d[3];
+        d[0] = delta_axis(pk[0], o.x, 0, P.g);
+        d[1] = delta_axis(pk[1], o.y, 1, P.g);
+        d[2] = 0.0f;
+        float r2 = d[0] * d[0];
+        r2 += d[1] * d[1];
+        if constexpr (D == 3) {
+            d[2] = delta_axis(pk[2], o.z, 2, P.g);
+            r2 += d[2] * d[2];
+        }
+        if (test && !(r2 < P.g.eps2)) return;
+        const float x = P.g.eps2 - r2;
+        const float w = 6.0f * P.g.k6 * (x * x) * (o.w + own.w);
 #pragma unroll
-            for (int a = 0; a < D; ++a) pa[a] = fmaf(w, d[a], pa[a]);
+        for (int a = 0; a < D; ++a) pa[a] = fmaf(w, d[a], pa[a]);
+    };
+    const uint32_t nc = A.nb_count[row];
+    if (nc <= MAXC) {
+        // three chunks at a time, the next three's records and these chunks' first sixteen slots (all that
+        // most cells hold) in flight together
+        constexpr int U = 3;
+        uint64_t mask[U];
+        uint32_t base[U];
+        auto fetch = [&](uint32_t c0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t c = c0 + u;
+                mask[u] = c < nc ? A.nb_mask[(uint64_t)row * MAXC + c] : 0ull;
+                base[u] = c < nc ? A.nb_base[(uint64_t)row * MAXC + c] : 0u;
+            }
         };
-        const uint32_t nc = A.nb_count[row];
-        if (nc <= MAXC) {
-            // three chunks at a time, the next three's records and these chunks' first sixteen slots (all that
-            // most cells hold) in flight together
-            constexpr int U = 3;
-            uint64_t mask[U];
-            uint32_t base[U];
-            auto fetch = [&](uint32_t c0) {
+        fetch(0);
+        for (uint32_t c = 0; c < nc; c += U) {
+            uint64_t m[U];
+            uint32_t at[U];
+            float4 o[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t c = c0 + u;
-                    mask[u] = c < nc ? A.nb_mask[(uint64_t)row * MAXC + c] : 0ull;
-                    base[u] = c < nc ? A.nb_base[(uint64_t)row * MAXC + c] : 0u;
-                }
-            };
-            fetch(0);
-            for (uint32_t c = 0; c < nc; c += U) {
-                uint64_t m[U];
-                uint32_t at[U];
-                float4 o[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    m[u] = mask[u] >> l;
-                    at[u] = base[u] + l;
-                    o[u] = m[u] & 1ull ? A.dpos[at[u]] : own;  // the particle itself adds nothing (d = 0)
-                }
-                fetch(c + U);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    add(o[u], false);
-#pragma unroll
-                    for (uint32_t i = 1; i < 4; ++i)
-                        if ((m[u] >> (16 * i)) & 1ull) add(A.dpos[at[u] + 16 * i], false);
-                }
+            for (int u = 0; u < U; ++u) {
+                m[u] = mask[u] >> l;
+                at[u] = base[u] + l;
+                o[u] = m[u] & 1ull ? A.dpos[at[u]] : own;  // the particle itself adds nothing (d = 0)
             }
-        } else {  // more chunks than were recorded: test the candidates of the 3^D cells
-            float pi[3];
-            int ci[3];
-            load_rec<D>(A.srec, A.scoord, s, pi, ci);
-            for (int k = 0; k < (D == 3 ? 27 : 9); ++k) {
-                const int64_t n0 = (int64_t)ci[0] + k % 3 - 1, n1 = (int64_t)ci[1] + (k / 3) % 3 - 1;
-                const int64_t n2 = D == 3 ? (int64_t)ci[2] + k / 9 - 1 : 0;
-                uint32_t beg = 0, end = 0;
-                bool filter = false;
-                if (!cell_range(P, A.bo, b, n0, n1, n2, beg, end, filter)) continue;
-                for (uint32_t j = beg + l; j < end; j += 16) {
-                    if (filter) {
-                        float pj[3];
-                        int cj[3];
-                        load_rec<D>(A.srec, A.scoord, j, pj, cj);
-                        if ((int64_t)cj[0] != n0 || (int64_t)cj[1] != n1 || (D == 3 && (int64_t)cj[2] != n2)) continue;
-                    }
-                    add(A.dpos[j], true);
-                }
+            fetch(c + U);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                add(o[u], false);
+#pragma unroll
+                for (uint32_t i = 1; i < 4; ++i)
+                    if ((m[u] >> (16 * i)) & 1ull) add(A.dpos[at[u] + 16 * i], false);
             }
         }
+    } else {  // more chunks than were recorded: test the candidates of the 3^D cells
+        float pi[3];
+        int ci[3];
+        load_rec<D>(A.srec, A.scoord, s, pi, ci);
+        for (int k = 0; k < (D == 3 ? 27 : 9); ++k) {
+            const int64_t n0 = (int64_t)ci[0] + k % 3 - 1, n1 = (int64_t)ci[1] + (k / 3) % 3 - 1;
+            const int64_t n2 = D == 3 ? (int64_t)ci[2] + k / 9 - 1 : 0;
+            uint32_t beg = 0, end = 0;
+            bool filter = false;
+            if (!cell_range(P, A.bo, b, n0, n1, n2, beg, end, filter)) continue;
+            for (uint32_t j = beg + l; j < end; j += 16) {
+                if (filter) {
+                    float pj[3];
+                    int cj[3];
+                    load_rec<D>(A.srec, A.scoord, j, pj, cj);
+                    if ((int64_t)cj[0] != n0 || (int64_t)cj[1] != n1 || (D == 3 && (int64_t)cj[2] != n2)) continue;
+                }
+                add(A.dpos[j], true);
+            }
+        }
+    }
 #pragma unroll
-        for (int a = 0; a < D; ++a) {
-            pa[a] = quad_sum(pa[a]);
-            pa[a] += __shfl_xor(pa[a], 4, 16);
-            pa[a] += __shfl_xor(pa[a], 8, 16);
-        }
-        if (l == 0) {
-            const float4 p0 = A.ppos[s];
-            A.pos_adj[(uint64_t)b * P.N + A.perm[s]] = make_float4(p0.x + pa[0], p0.y + pa[1], D == 3 ? p0.z + pa[2] : 0.0f, 0.0f);
-        }
+    for (int a = 0; a < D; ++a) {
+        pa[a] = quad_sum(pa[a]);
+        pa[a] += __shfl_xor(pa[a], 4, 16);
+        pa[a] += __shfl_xor(pa[a], 8, 16);
+    }
+    if (l == 0) {
+        const float4 p0 = A.ppos[s];
+        A.pos_adj[(uint64_t)b * P.N + A.perm[s]] = make_float4(p0.x + pa[0], p0.y + pa[1], D == 3 ? p0.z + pa[2] : 0.0f, 0.0f);
     }
 }
 
 template <int D, int SM>
 static hipError_t launch_adjoint_t(const StepParams& p, const AdjointArgs& a, hipStream_t stream) {
-    // a launch holds fewer than 2^32 threads, so past 2^24 particles a block takes several sixteens
-    const dim3 waves(std::min((p.T + 15) / 16, 1u << 20));
+    // a launch's row of blocks holds fewer than 2^32 threads: past 2^24 particles a block of the pair kernels takes
+    // several sixteens, and the density kernel's blocks have more rows
+    const uint32_t sixteens = (p.T + 15) / 16;
+    const dim3 waves(std::min(sixteens, 1u << 20)), blocks(waves.x, (sixteens + waves.x - 1) / waves.x);
     hipLaunchKernelGGL((k_adj_prep<D, SM>), waves, dim3(64), 0, stream, p, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_adj_gather<D, SM>), waves, dim3(64), 0, stream, p, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_adj_density_kernel<D>, waves, dim3(256), 0, stream, p, a);
+    hipLaunchKernelGGL(k_adj_density_kernel<D>, blocks, dim3(256), 0, stream, p, a);
     return hipGetLastError();
 }
 

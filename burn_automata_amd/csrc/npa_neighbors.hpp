@@ -277,7 +277,8 @@ __device__ __forceinline__ void append_accepted(const StepParams& P, const float
                 // batches of 4 candidates per lane: loads first (index clamped to
                 // the chunk, so every load is in bounds), then branch-free tests. The boundary and the
                 // bin's filter are chosen per chunk: tested by candidate the compiler turns both into
-                // selects for every one of them (a dense 2D cloud's second pass 1,122 -> 1,220 us).
+                // selects for every one of them (a step of 60,000 particles, 730 neighbours each, S = 8: 1,108 us,
+                // now 987).
                 uint64_t acc = 0;
                 auto tests = [&](auto periodic, auto filtered) {
 #pragma unroll 1
