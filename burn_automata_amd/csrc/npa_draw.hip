@@ -471,7 +471,8 @@ hipError_t reserve_draw(const DrawPlan& p, SplatWorkspace& ws, hipStream_t strea
     if ((e = ws.crowd.reserve(kCrowdWords * 4)) != hipSuccess) return e;
     // the tickets are zero between drawings: the block that takes a group's last one clears it
     hipLaunchKernelGGL(k_draw_clear, dim3(kDrawGroups / 256), dim3(256), 0, stream, ws.crowd.as<uint32_t>());
-    return hipGetLastError();
+    if ((e = hipGetLastError()) != hipSuccess) ws.crowd.release();  // cleared by the next drawing, then
+    return e;
 }
 
 template <int NCH>

@@ -301,7 +301,7 @@ struct StepParams {
     uint32_t N, B, S, H, F;
     uint32_t SS;    // sorted state row stride (state_stride_for(S))
     uint32_t FP;    // padded feature row width (padded_features)
-    uint32_t T;     // total particles B*N (feature-major row count)
+    uint32_t T;     // total particles B*N
     uint32_t state_grad, density_grad, log_norm_grad, log_norm_dgrad, hybrid, position_features;
     float state_scale;  // normalize_state_gradient factor
     float dgrad_scale;  // normalize_density_gradient factor

@@ -448,7 +448,10 @@ npa_status npa_state_step_into_gaussians(npa_state* state, uint32_t steps, uint3
  *     would take transmittance T below 1e-4; rgb += colour alpha T, T *= 1 - alpha. The power is
  *     evaluated as qa dx^2 + qc dy^2 + qb dx dy with the conic pre-scaled by -log2(e)/2, -log2(e),
  *     -log2(e)/2 in fused multiply-adds, and e^power as 2^(that).
- * image[height][width][4] = premultiplied r, g, b and 1 - T; it is overwritten. */
+ * image[height][width][4] = premultiplied r, g, b and 1 - T; it is overwritten.
+ * Workspace kept by the context (or, below, the state): up to 65,536 Gaussians 4 B per Gaussian and group
+ * of tiles (at most 512 groups, 128 MiB), beyond that about 20 B per (tile, Gaussian) pair, whose number is
+ * read back first. */
 enum { NPA_RASTER_COLOR_SH = 0, NPA_RASTER_COLOR_RGB = 1 };
 typedef struct npa_raster_camera {
     float view[16];           /* row-major world -> camera */

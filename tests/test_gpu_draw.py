@@ -199,3 +199,30 @@ def test_rectangles_of_wide_images(ctx, size, corner):
     box = got[y0:y0 + want.shape[0], x0:x0 + want.shape[1]]
     assert np.count_nonzero(got) == np.count_nonzero(box)
     assert _err(box, want) <= TOL
+
+
+def test_crowded_splat_replays_in_a_graph(ctx):
+    """A captured drawing of crowded groups, replayed with eager drawings in between, equals the eager one."""
+    import torch
+    pos, col, _, _ = _particles(20000, 3, 0.02)
+    pos, col = torch.from_numpy(pos).cuda(), torch.from_numpy(col).cuda()
+    other = [torch.from_numpy(a).cuda() for a in _particles(9000, 5, 0.05)[:2]]
+    cfg = Splat2dConfig(image_size=600, sigma=1.0, pixel_size=2.0 / 600)
+    want = K.splat_particles_2d(pos, col, cfg, ctx=ctx).clone()
+    want_other = K.splat_particles_2d(*other, cfg, ctx=ctx).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    home = torch.cuda.current_stream().cuda_stream
+    try:
+        with torch.cuda.graph(graph):
+            ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+            got = K.splat_particles_2d(pos, col, cfg, ctx=ctx)
+    finally:
+        ctx.set_stream(home)
+    for _ in range(3):
+        got.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(K.splat_particles_2d(*other, cfg, ctx=ctx), want_other)
